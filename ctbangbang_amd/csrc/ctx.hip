@@ -7,7 +7,6 @@
 
 #include <algorithm>
 #include <cmath>
-#include <complex>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -110,6 +109,7 @@ struct ctbb_ctx {
     // filter on `stream`.
     hipStream_t stream_head = nullptr;
     hipEvent_t ev_prep_done = nullptr, ev_head = nullptr;
+    hipEvent_t ev_default = nullptr;     // work queued on the default stream (ctbb_filter_rows_dev)
     // the head's own workspaces (adaptive-filter output and work, rebinned
     // rows, zero-padded pull), so it touches nothing the previous call or
     // other entry points use
@@ -232,79 +232,22 @@ int check_geometry(const recon_metadata *mr) {
     return CTBB_OK;
 }
 
-// Filter taps of the prm's ReconKernel, cached per (install dir, channels, kernel).
-// In-place radix-2 DFT (forward sign) of a power-of-two length, FP64.
-void dft_pow2(std::vector<std::complex<double>> &x) {
-    const size_t n = x.size();
-    for (size_t i = 1, j = 0; i < n; i++) {
-        size_t bit = n >> 1;
-        for (; j & bit; bit >>= 1) j ^= bit;
-        j ^= bit;
-        if (i < j) std::swap(x[i], x[j]);
-    }
-    for (size_t len = 2; len <= n; len <<= 1) {
-        const double ang = -2.0 * M_PI / static_cast<double>(len);
-        for (size_t i = 0; i < n; i += len)
-            for (size_t k = 0; k < len / 2; k++) {
-                const std::complex<double> w(std::cos(ang * k), std::sin(ang * k));
-                const std::complex<double> u = x[i + k], v = x[i + k + len / 2] * w;
-                x[i + k] = u + v;
-                x[i + k + len / 2] = u - v;
-            }
-    }
-}
-
-// DFT of length L (forward sign) of the first `count` values of x zero-padded,
-// FP64, directly from a table of the L roots of unity.
-std::vector<std::complex<double>> dft_direct(const float *x, size_t count, size_t L) {
-    std::vector<std::complex<double>> w(L), X(L);
-    for (size_t t = 0; t < L; t++) {
-        const double a = -2.0 * M_PI * static_cast<double>(t) / static_cast<double>(L);
-        w[t] = std::complex<double>(std::cos(a), std::sin(a));
-    }
-    for (size_t k = 0; k < L; k++) {
-        std::complex<double> acc = 0.0;
-        size_t t = 0;                                   // m k mod L
-        for (size_t m = 0; m < count; m++) {
-            acc += static_cast<double>(x[m]) * w[t];
-            t += k;
-            if (t >= L) t -= L;
-        }
-        X[k] = acc;
-    }
-    return X;
-}
-
-// FFT32 form of the filter: H = DFT_L(taps zero-padded) / L and the
-// twiddles e^(-2 pi i t / L), evaluated in FP64 and rounded once, into
-// ctx->spec, with L = 3072 for 2n <= 3072 and 4096 for 2n <= 4096 (wider
-// filters use the FP32 product).
-int make_spec(ctbb_ctx *ctx, const float *taps, size_t count) {
+// FFT32 form of the filter: the spectrum and twiddles of `count` taps on the
+// device (d_taps) into ctx->spec, queued on ctx->stream, with L = 3072 for
+// 2n <= 3072 and 4096 for 2n <= 4096 (wider filters use the FP32 product).
+int make_spec(ctbb_ctx *ctx, const float *d_taps, size_t count) {
     if (count > 4096) return CTBB_OK;
-    const size_t L = count <= 3072 ? 3072 : 4096;
-    std::vector<std::complex<double>> h;
-    if (L == 4096) {
-        h.assign(L, 0.0);
-        for (size_t m = 0; m < count; m++) h[m] = taps[m];
-        dft_pow2(h);
-    } else {
-        h = dft_direct(taps, count, L);
-    }
-    std::vector<float> sp(4 * L);
-    for (size_t k = 0; k < L; k++) {
-        sp[2 * k] = static_cast<float>(h[k].real() / L);
-        sp[2 * k + 1] = static_cast<float>(h[k].imag() / L);
-        const double a = -2.0 * M_PI * static_cast<double>(k) / L;
-        sp[2 * L + 2 * k] = static_cast<float>(std::cos(a));
-        sp[2 * L + 2 * k + 1] = static_cast<float>(std::sin(a));
-    }
+    const int L = count <= 3072 ? 3072 : 4096;
     ctx->spec_len = 0;
-    const int st = upload(ctx, ctx->spec, sp.data(), sp.size() * sizeof(float));
+    int st = ctx->spec.ensure(2 * static_cast<size_t>(L) * sizeof(float2));
     if (st) return st;
-    ctx->spec_len = static_cast<int>(L);
+    st = launch_filter_spectrum(d_taps, static_cast<int>(count), L, ctx->spec.as<float2>(), ctx->stream);
+    if (st) return st;
+    ctx->spec_len = L;
     return CTBB_OK;
 }
 
+// Filter taps of the prm's ReconKernel, cached per (install dir, channels, kernel).
 int ensure_taps(ctbb_ctx *ctx, const recon_metadata *mr) {
     std::string key = std::string(mr->install_dir) + "|" + std::to_string(mr->cg.n_channels) + "|" +
                       std::to_string(mr->rp.recon_kernel);
@@ -314,7 +257,7 @@ int ensure_taps(ctbb_ctx *ctx, const recon_metadata *mr) {
     if (st) return st;
     st = upload(ctx, ctx->taps, t.data(), t.size() * sizeof(float));
     if (st) return st;
-    st = make_spec(ctx, t.data(), t.size());
+    st = make_spec(ctx, ctx->taps.as<float>(), t.size());
     if (st) return st;
     ctx->taps_key = key;
     return CTBB_OK;
@@ -828,7 +771,7 @@ void ctbb_ctx_destroy(ctbb_ctx *c) {
     }
     if (c->ev_sync) (void)hipEventDestroy(c->ev_sync);
     if (c->stream_bp) (void)hipStreamDestroy(c->stream_bp);
-    for (hipEvent_t e : {c->ev_prep_done, c->ev_head})
+    for (hipEvent_t e : {c->ev_prep_done, c->ev_head, c->ev_default})
         if (e) (void)hipEventDestroy(e);
     if (c->stream_head) (void)hipStreamDestroy(c->stream_head);
     for (hipGraphExec_t g : c->live_graphs) (void)hipGraphExecDestroy(g);
@@ -923,14 +866,17 @@ int ctbb_filter_rows_dev(ctbb_ctx *c, const float *d_taps, int n, size_t n_rows_
     if (hipSetDevice(c->device) != hipSuccess) return CTBB_ERR_HIP;
     c->reset_events();
     if (c->opt.filter_mode == CTBB_FILTER_FFT32) {
-        // the spectrum of these taps (the cached one belongs to a prm's filter)
-        std::vector<float> t(2 * static_cast<size_t>(n));
-        if (hipStreamSynchronize(c->stream) != hipSuccess ||
-            hipMemcpy(t.data(), d_taps, t.size() * sizeof(float), hipMemcpyDeviceToHost) != hipSuccess)
+        // The spectrum of these taps, computed on the device every call (the
+        // cached one belongs to a prm's filter).  The default stream is
+        // waited for on the device, so taps and rows written there are seen.
+        if (!c->ev_default && hipEventCreateWithFlags(&c->ev_default, hipEventDisableTiming) != hipSuccess)
             return CTBB_ERR_HIP;
-        int st = make_spec(c, t.data(), t.size());
-        if (st) return st;
+        if (hipEventRecord(c->ev_default, nullptr) != hipSuccess ||
+            hipStreamWaitEvent(c->stream, c->ev_default, 0) != hipSuccess)
+            return CTBB_ERR_HIP;
         c->taps_key.clear();
+        const int st = make_spec(c, d_taps, 2 * static_cast<size_t>(n));
+        if (st) return st;
     }
     return do_filter(c, d_taps, n, n_rows_total, d_in, d_out, c->opt.proj_dtype == CTBB_PROJ_BF16);
 }

@@ -315,8 +315,8 @@ __global__ __launch_bounds__(256) void conv_valu_kernel(FilterArgs a) {
 // y[n + l] = sum_k x[k] taps[n + l - k] for l in [0, n) without wrap-around
 // (n + l - k lies in [1, 2n - 1]).  Two rows a, b travel as one complex
 // signal a + i b: h is real, so y = (a (*) h) + i (b (*) h).
-// The host supplies H = DFT_L(h) / L and the twiddles e^(-2 pi i t / L),
-// both evaluated in FP64 and rounded once.  L = 3072 where 2n <= 3072 (the
+// H = DFT_L(h) / L and the twiddles e^(-2 pi i t / L) come from
+// filter_spectrum_kernel, evaluated in FP64 and rounded once.  L = 3072 where 2n <= 3072 (the
 // shipped scanners: 1472 and 1344 oversampled channels), else 4096.
 // Transforms (Stockham, the passes in between through LDS with one pad
 // entry per 16 to spread the banks; the inverse is conj(DFT(conj(Y)))):
@@ -639,7 +639,71 @@ __global__ __launch_bounds__(256) void fft_filter_kernel(FilterArgs a) {
     }
 }
 
+// Spectrum of the taps and twiddles of the FFT form: spec[k] = DFT_L(taps)[k]
+// / L (taps zero-padded from `count` to L) and spec[L + t] = e^(-2 pi i t / L),
+// evaluated in FP64 and rounded once.  The taps are real, so one wave takes
+// bin k <= L / 2 and also writes bin L - k as its conjugate.  Each lane sums
+// its taps m = lane, lane + 64, ... by Horner's rule in w^64 (w = e^(-2 pi i
+// k / L), at most 64 steps: error far below FP32), times w^lane; 3072 x 2944
+// products took 7.4 ms on a host core, with a copy of the taps back and an
+// upload around them, and take 6.1 us here (8.2 us for 4096; bound by latency:
+// 1537 waves of 46 dependent FP64 steps and three sine/cosine pairs; loading
+// the taps one step at a time took 12 and 26 us).
+constexpr int SPEC_WAVES = 4;
+
+__global__ __launch_bounds__(64 * SPEC_WAVES) void filter_spectrum_kernel(const float *__restrict__ taps, int count,
+                                                                          int L, float2 *__restrict__ spec) {
+    const int lane = threadIdx.x & 63;
+    const int k = blockIdx.x * SPEC_WAVES + (threadIdx.x >> 6);
+    const int t = blockIdx.x * (64 * SPEC_WAVES) + threadIdx.x;
+    double sn, cs;
+    if (t < L) {
+        sincospi(-2.0 * t / L, &sn, &cs);
+        spec[L + t] = make_float2(static_cast<float>(cs), static_cast<float>(sn));
+    }
+    if (k > L / 2) return;
+    // (products of indices reduced mod L: exact angles)
+    sincospi(-2.0 * ((64 * k) % L) / L, &sn, &cs);
+    // (the last group may be short; the others are loaded eight at a time,
+    // ahead of the dependent products)
+    const int last = (count - 1) >> 6;
+    double re = 64 * last + lane < count ? static_cast<double>(taps[64 * last + lane]) : 0.0, im = 0.0;
+    auto step = [&](float x) {
+        const double nr = fma(re, cs, fma(-im, sn, static_cast<double>(x)));
+        im = fma(re, sn, im * cs);
+        re = nr;
+    };
+    int q = last - 1;
+    for (; q >= 7; q -= 8) {
+        float x[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++) x[e] = taps[64 * (q - e) + lane];
+#pragma unroll
+        for (int e = 0; e < 8; e++) step(x[e]);
+    }
+    for (; q >= 0; q--) step(taps[64 * q + lane]);
+    sincospi(-2.0 * ((k * lane) % L) / L, &sn, &cs);
+    double hr = fma(re, cs, -im * sn), hi = fma(re, sn, im * cs);
+    for (int s = 32; s > 0; s >>= 1) {
+        hr += __shfl_xor(hr, s, 64);
+        hi += __shfl_xor(hi, s, 64);
+    }
+    if (lane == 0) {
+        const float fr = static_cast<float>(hr / L), fi = static_cast<float>(hi / L);
+        spec[k] = make_float2(fr, fi);
+        if (k > 0 && 2 * k < L) spec[L - k] = make_float2(fr, -fi);
+    }
+}
+
 }  // namespace
+
+int launch_filter_spectrum(const float *d_taps, int count, int L, float2 *d_spec, hipStream_t stream) {
+    if (!d_taps || !d_spec || count <= 0 || count > L || (L != FFT_L && L != FFT_L3)) return CTBB_ERR_ARG;
+    const unsigned grid = static_cast<unsigned>((L / 2 + 1 + SPEC_WAVES - 1) / SPEC_WAVES);
+    // (grid * 256 threads >= L: the twiddles are covered)
+    hipLaunchKernelGGL(filter_spectrum_kernel, dim3(grid), dim3(64 * SPEC_WAVES), 0, stream, d_taps, count, L, d_spec);
+    return hipGetLastError() == hipSuccess ? CTBB_OK : CTBB_ERR_HIP;
+}
 
 int launch_filter(const FilterArgs &a, hipStream_t stream) {
     if (!a.in || !a.out || !a.taps || a.n <= 0) return CTBB_ERR_ARG;
