@@ -148,89 +148,153 @@ __global__ __launch_bounds__(64) void af_thresh(const float *sm, float *thr, int
     if (threadIdx.x == 0) thr[p] = T;
 }
 
-// reference preprocessing.cuh:208-285 (3D branch, __FILTER_3D__ defined)
-// Output sample (i, j, p): copied when x <= T, else the 5x5x5 weighted
-// smoothing of its neighbourhood.
-__device__ __forceinline__ float af_value(const float *__restrict__ raw, float x, float T, int i, int j, int p,
-                                          int n_proj, int n_rows_raw, int nch, size_t ps) {
-    if (!(x > T)) return x;
-    float norm = 0.0f, val = 0.0f;
-    // (outer loops rolled: few registers, so the kernels fit beside a
-    // backprojection; the order of the sums is unchanged)
+// Apply step, reference preprocessing.cuh:208-285 (3D branch, __FILTER_3D__
+// defined): a sample x <= T is kept, one above it becomes the 5x5x5 weighted
+// mean of its neighbourhood, weights triangle_3d(5, ii, jj, kk) with
+// ceil(5/2) = 3 (peak at offset +1), summed over channel, row, view in this
+// order, each sum one chain of fused multiply-adds.
+//
+// One wave takes 64 channels x kRows rows of one view, a lane one channel.
+// A wave with no sample above T copies its rows.  Otherwise the lane walks
+// the channels ii (rolled) and rows of its neighbourhood, loads the row's 5
+// views once and feeds them to every output row they belong to: 60 loads per
+// channel for 8 output rows, 37.5 per output instead of 125, with 125 fused
+// multiply-adds.  Neighbours outside the pull contribute nothing: they read
+// as zeros through the buffer descriptors (one per view, of the frame's size
+// and of size 0 for a view outside the pull; a row or channel outside the
+// frame gives an offset past its end), and a zero leaves the sum as it is.
+// The sums keep the order and so the bits of the one-sample form.
+// Bound by the VALU where samples are smoothed and by HBM elsewhere; views
+// are dealt to the XCDs in contiguous bands so that the 5 frames around a
+// view are read from one L2.  4096 views of 32 x 672 samples with a fixed
+// threshold of 1.204: 4.52 ms with one thread per four samples and 125
+// guarded loads each, 0.36 ms here (with no sample above T, 8448 views of
+// 32 x 736: 0.26 ms, 6.1 TB/s).
+constexpr int kRows = 8;
+
+__device__ __forceinline__ constexpr int af_tri(int i) { return 3 - (i < 3 ? 3 - i : i - 3); }
+
+__device__ __forceinline__ void af_smooth_rows(const float *raw, float (&acc)[kRows], int i, int j0, int p, int n_proj,
+                                               int n_rows_raw, int nch, size_t ps) {
+    __amdgpu_buffer_rsrc_t rs[5];
+#pragma unroll
+    for (int kk = 0; kk < 5; kk++) {
+        const int fp = p + kk - 2;
+        const bool in = fp >= 0 && fp < n_proj;
+        rs[kk] = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(raw + ps * (in ? fp : p)), static_cast<short>(0),
+                                                   in ? static_cast<int>(ps * sizeof(float)) : 0, 0x00020000);
+    }
+#pragma unroll
+    for (int r = 0; r < kRows; r++) acc[r] = 0.0f;
+    const int row_b = nch * 4;
 #pragma unroll 1
     for (int ii = 0; ii < 5; ii++) {
-        const int fc = i + ii - 2;
-#pragma unroll 1
-        for (int jj = 0; jj < 5; jj++) {
-            const int fr = j + jj - 2;
-            for (int kk = 0; kk < 5; kk++) {
-                const int fp = p + kk - 2;
-                if (fr < 0 || fc < 0 || fp < 0 || fr >= n_rows_raw || fc >= nch || fp >= n_proj) continue;
-                // triangle_3d(5, ii, jj, kk), ceil(5/2) = 3: peak at offset +1
-                const float t = static_cast<float>((3 - abs(ii - 3)) + (3 - abs(jj - 3)) + (3 - abs(kk - 3)) + 1);
-                norm += t;
-                val = fmaf(raw[ps * fp + static_cast<size_t>(nch) * fr + fc], t, val);
+        const int c = i + ii - 2;
+        const float ta = static_cast<float>(3 - abs(ii - 3));
+        // byte offset of (row j0 - 2, channel c); a channel outside the frame
+        // stays past the end of every frame (< 2 GiB) for all kRows + 4 rows
+        int off = c >= 0 && c < nch ? (j0 - 2) * row_b + c * 4 : static_cast<int>(0x80000000u);
+        const bool c_in = off != static_cast<int>(0x80000000u);
+#pragma unroll
+        for (int q = 0; q < kRows + 4; q++) {           // row j0 - 2 + q
+            float v[5];
+#pragma unroll
+            for (int kk = 0; kk < 5; kk++)
+                v[kk] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs[kk], off, 0, 0));
+            off = c_in ? off + row_b : off;
+#pragma unroll
+            for (int r = 0; r < kRows; r++) {
+                const int jj = q - r;                   // output row j0 + r sees it as row offset jj - 2
+                if (jj < 0 || jj > 4) continue;
+#pragma unroll
+                for (int kk = 0; kk < 5; kk++)
+                    acc[r] = fmaf(v[kk], ta + static_cast<float>(af_tri(jj) + af_tri(kk) + 1), acc[r]);
             }
         }
     }
-    return (1.0f / norm) * val;
 }
 
-// One thread per sample (low register use: runs beside a backprojection).
-__global__ __launch_bounds__(256) void af_apply(const float *raw, const float *thr, float *out, int n_proj,
-                                                int n_rows_raw, int nch) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;   // channel
-    const int j = blockIdx.y;                                // row
-    const int p = blockIdx.z;                                // view
-    if (i >= nch) return;
-    const size_t ps = static_cast<size_t>(nch) * n_rows_raw;
-    const size_t idx = ps * p + static_cast<size_t>(j) * nch + i;
-    out[idx] = af_value(raw, raw[idx], thr[p], i, j, p, n_proj, n_rows_raw, nch, ps);
-}
-
-// Four consecutive samples of a view's frame per thread, 16-byte loads and
-// stores (for a GPU that runs nothing else: the first block of a pipeline
-// and the stage entry point).
-__global__ __launch_bounds__(256) void af_apply4(const float *raw, const float *thr, float *out, int n_proj,
-                                                 int n_rows_raw, int nch) {
-    const int p = blockIdx.y;
-    const size_t ps = static_cast<size_t>(nch) * n_rows_raw;
-    const int e = (blockIdx.x * blockDim.x + threadIdx.x) * 4;   // sample in the frame
-    if (static_cast<size_t>(e) >= ps) return;
-    const size_t base = ps * p + e;
-    const float T = thr[p];
-    const float4 x = *reinterpret_cast<const float4 *>(raw + base);
-    float4 y = x;
-    if (x.x > T || x.y > T || x.z > T || x.w > T) {
-        float *yv = reinterpret_cast<float *>(&y);
-        const float xv[4] = {x.x, x.y, x.z, x.w};
+// Sum of the weights of the neighbours inside the pull (whole numbers below
+// 2^24: exact in any order).
+__device__ __forceinline__ float af_norm(int i, int j, int p, int n_proj, int n_rows_raw, int nch) {
+    auto axis = [](int at, int n, int &count, int &sum) {
+        count = sum = 0;
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const int j = (e + q) / nch, i = e + q - j * nch;
-            yv[q] = af_value(raw, xv[q], T, i, j, p, n_proj, n_rows_raw, nch, ps);
-        }
-    }
-    *reinterpret_cast<float4 *>(out + base) = y;
+        for (int o = 0; o < 5; o++)
+            if (at + o - 2 >= 0 && at + o - 2 < n) {
+                count += 1;
+                sum += af_tri(o);
+            }
+    };
+    int ni, nj, nk, si, sj, sk;
+    axis(i, nch, ni, si);
+    axis(j, n_rows_raw, nj, sj);
+    axis(p, n_proj, nk, sk);
+    return static_cast<float>(si * nj * nk + sj * ni * nk + sk * ni * nj + ni * nj * nk);
 }
 
-// Only the views the filter changes: view p is unchanged where its maximum
-// (af_sup, from 0) is at or below its threshold, since af_value keeps every
-// sample x <= T.  One workgroup per view flags it (hot[p]) and, if changed,
-// writes its filtered frame; a reader takes the other views from the raw
-// pull.  (C1: about 6% of the views.)
-__global__ __launch_bounds__(256) void af_apply_hot(const float *raw, const float *sup, const float *thr, float *out,
-                                                    unsigned char *hot, int n_proj, int n_rows_raw, int nch) {
-    const int p = blockIdx.x;
+// Rows j0 .. j0 + kRows - 1 of channels i (one per lane) of view p.
+__device__ __forceinline__ void af_apply_rows(const float *raw, float T, float *out, int i, int j0, int p, int n_proj,
+                                              int n_rows_raw, int nch, size_t ps) {
+    const size_t base = ps * p + static_cast<size_t>(j0) * nch + i;
+    float x[kRows];
+    bool hot = false;
+#pragma unroll
+    for (int r = 0; r < kRows; r++) {
+        x[r] = i < nch && j0 + r < n_rows_raw ? raw[base + static_cast<size_t>(r) * nch] : 0.0f;
+        hot |= i < nch && j0 + r < n_rows_raw && x[r] > T;
+    }
+    if (__builtin_amdgcn_ballot_w64(hot)) {
+        float acc[kRows];
+        af_smooth_rows(raw, acc, i, j0, p, n_proj, n_rows_raw, nch, ps);
+#pragma unroll
+        for (int r = 0; r < kRows; r++)
+            if (x[r] > T) x[r] = (1.0f / af_norm(i, j0 + r, p, n_proj, n_rows_raw, nch)) * acc[r];
+    }
+#pragma unroll
+    for (int r = 0; r < kRows; r++)
+        if (i < nch && j0 + r < n_rows_raw) out[base + static_cast<size_t>(r) * nch] = x[r];
+}
+
+// Waves (64 channels x kRows rows) of a view.
+__host__ __device__ __forceinline__ int af_view_waves(int n_rows_raw, int nch) {
+    return ((nch + 63) / 64) * ((n_rows_raw + kRows - 1) / kRows);
+}
+
+// bpv workgroups of 4 waves per view, XCD x the x-th eighth of the views.
+// kHot: only the views the filter changes (view p is unchanged where its
+// maximum, af_sup from 0, is at or below its threshold); hot[p] flags them,
+// and a reader takes the other views from the raw pull (C1: about 6% of the
+// views are hot).  37 VGPRs: a wave of it fits beside a backprojection's four.
+template <bool kHot>
+__device__ __forceinline__ void af_apply_block(const float *raw, const float *sup, const float *thr, float *out,
+                                               unsigned char *hot, int n_proj, int n_rows_raw, int nch, int bpv) {
+    const int xcd = blockIdx.x & 7, idx = blockIdx.x >> 3, band = (n_proj + 7) / 8;
+    const int pv = idx / bpv, p = xcd * band + pv, part = idx - pv * bpv;
+    if (pv >= band || p >= n_proj) return;
     const float T = thr[p];
-    const bool h = sup[p] > T;
-    if (threadIdx.x == 0) hot[p] = h ? 1 : 0;
-    if (!h) return;
-    const size_t ps = static_cast<size_t>(nch) * n_rows_raw;
-    for (int j = 0; j < n_rows_raw; j++)
-        for (int i = threadIdx.x; i < nch; i += 256) {
-            const size_t idx = ps * p + static_cast<size_t>(j) * nch + i;
-            out[idx] = af_value(raw, raw[idx], T, i, j, p, n_proj, n_rows_raw, nch, ps);
-        }
+    if (kHot) {
+        const bool h = sup[p] > T;
+        if (part == 0 && threadIdx.x == 0) hot[p] = h ? 1 : 0;
+        if (!h) return;
+    }
+    const int tiles = (nch + 63) / 64;
+    const int w = part * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (w >= af_view_waves(n_rows_raw, nch)) return;
+    const int g = w / tiles;
+    af_apply_rows(raw, T, out, (w - g * tiles) * 64 + (threadIdx.x & 63), g * kRows, p, n_proj, n_rows_raw, nch,
+                  static_cast<size_t>(nch) * n_rows_raw);
+}
+
+__global__ __launch_bounds__(256) void af_apply(const float *raw, const float *thr, float *out, int n_proj,
+                                                int n_rows_raw, int nch, int bpv) {
+    af_apply_block<false>(raw, nullptr, thr, out, nullptr, n_proj, n_rows_raw, nch, bpv);
+}
+
+__global__ __launch_bounds__(256) void af_apply_hot(
+    const float *raw, const float *sup, const float *thr, float *out, unsigned char *hot, int n_proj, int n_rows_raw,
+    int nch, int bpv) {
+    af_apply_block<true>(raw, sup, thr, out, hot, n_proj, n_rows_raw, nch, bpv);
 }
 
 // Fixed-threshold mode: every view's threshold is the same constant.
@@ -277,18 +341,15 @@ int launch_adaptive(const AdaptiveArgs &a, hipStream_t stream) {
             hipLaunchKernelGGL(af_thresh<false>, dim3(a.n_proj), dim3(64), 0, stream, sm, thr, a.n_proj, n_range,
                                a.n_proj_ffs, a.strength);
     }
-    if (a.hot_only) {
-        hipLaunchKernelGGL(af_apply_hot, dim3(a.n_proj), dim3(256), 0, stream, a.raw, sup, thr, a.out,
-                           adaptive_hot_flags(a.work, a.n_proj), a.n_proj, a.n_rows_raw, a.nch);
-        return hipGetLastError() == hipSuccess ? CTBB_OK : CTBB_ERR_HIP;
-    }
-    const bool aligned = (reinterpret_cast<uintptr_t>(a.raw) & 15u) == 0 && (reinterpret_cast<uintptr_t>(a.out) & 15u) == 0;
-    if (a.vec4 && aligned)
-        hipLaunchKernelGGL(af_apply4, dim3(static_cast<unsigned>((frame / 4 + 255) / 256), a.n_proj), dim3(256), 0,
-                           stream, a.raw, thr, a.out, a.n_proj, a.n_rows_raw, a.nch);
+    const int bpv = (af_view_waves(a.n_rows_raw, a.nch) + 3) / 4;
+    const unsigned long long grid = 8ull * static_cast<unsigned long long>((a.n_proj + 7) / 8) * bpv;
+    if (grid > 0x7fffffffull) return CTBB_ERR_SHAPE;
+    if (a.hot_only)
+        hipLaunchKernelGGL(af_apply_hot, dim3(static_cast<unsigned>(grid)), dim3(256), 0, stream, a.raw, sup, thr, a.out,
+                           adaptive_hot_flags(a.work, a.n_proj), a.n_proj, a.n_rows_raw, a.nch, bpv);
     else
-        hipLaunchKernelGGL(af_apply, dim3((a.nch + 255) / 256, a.n_rows_raw, a.n_proj), dim3(256), 0, stream, a.raw,
-                           thr, a.out, a.n_proj, a.n_rows_raw, a.nch);
+        hipLaunchKernelGGL(af_apply, dim3(static_cast<unsigned>(grid)), dim3(256), 0, stream, a.raw, thr, a.out,
+                           a.n_proj, a.n_rows_raw, a.nch, bpv);
     return hipGetLastError() == hipSuccess ? CTBB_OK : CTBB_ERR_HIP;
 }
 

@@ -491,11 +491,9 @@ int do_finalize(ctbb_ctx *ctx, const recon_metadata *mr, const float *d_image, f
     return launch_finalize_blob(ctx, mr, d_image, d_final, ctx->fin_tab.as<char>(), mt, nf, ctx->stream);
 }
 
-// vec4: the 16-byte apply kernel (for a GPU that runs nothing else; the
-// one-sample kernel needs few registers and runs beside a backprojection).
 // hot: write d_out only for the views the filter changes and return their
 // flags in *hot (inside the work buffer, valid until its next use).
-int do_adaptive(ctbb_ctx *ctx, const recon_metadata *mr, const float *d_raw, float *d_out, bool vec4 = true,
+int do_adaptive(ctbb_ctx *ctx, const recon_metadata *mr, const float *d_raw, float *d_out,
                 hipStream_t on = nullptr, DevBuf *work = nullptr, const unsigned char **hot = nullptr,
                 int max_groups = 0) {
     const ct_geom &cg = mr->cg;
@@ -507,7 +505,6 @@ int do_adaptive(ctbb_ctx *ctx, const recon_metadata *mr, const float *d_raw, flo
     a.nch = static_cast<int>(cg.n_channels);
     a.n_proj_ffs = static_cast<int>(cg.n_proj_ffs);
     a.strength = mr->rp.adaptive_filtration_s;
-    a.vec4 = vec4 ? 1 : 0;
     a.fixed_threshold = ctx->opt.adaptive_threshold;
     a.hot_only = hot ? 1 : 0;
     a.max_groups = max_groups;
@@ -583,7 +580,7 @@ int prep_block(ctbb_ctx *c, recon_metadata *mr, const float *win, void *d_out, h
     if (c->opt.adaptive_filter) {
         st = af.ensure(n * frame * sizeof(float));
         if (st) return st;
-        st = do_adaptive(c, mr, win, af.as<float>(), false, head, head ? &c->head_work : nullptr, &hot,
+        st = do_adaptive(c, mr, win, af.as<float>(), head, head ? &c->head_work : nullptr, &hot,
                          c->prep_groups);
         if (st) return st;
     }
@@ -1564,7 +1561,7 @@ int batch_persistent(ctbb_ctx *c, int n_scans, recon_metadata *const *mrs, const
                     st = block_window(c, m, d_raws[jobs[j].s], n_raw[jobs[j].s], &win);
                     const unsigned char *hot = nullptr;
                     if (!st && c->opt.adaptive_filter)
-                        st = do_adaptive(c, m, win, c->raw_af.as<float>(), false, nullptr, nullptr, &hot,
+                        st = do_adaptive(c, m, win, c->raw_af.as<float>(), nullptr, nullptr, &hot,
                                          c->prep_groups);
                     if (!st)
                         st = do_rebin(c, m, win, reinterpret_cast<float *>(slot_ptr(jobs[j])),

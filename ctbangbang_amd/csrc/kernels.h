@@ -109,7 +109,6 @@ struct AdaptiveArgs {
     int n_proj, n_rows_raw, nch;
     int n_proj_ffs;
     float strength;
-    int vec4;                  // 1: 16-byte apply kernel where aligned (GPU otherwise idle)
     float fixed_threshold;     // > 0: this threshold for every view instead of the KK bisection
     // 1: write out only for the views the filter changes (those whose maximum
     // exceeds their threshold), flagged in adaptive_hot_flags(work, n_proj);

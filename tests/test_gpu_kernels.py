@@ -37,3 +37,39 @@ def test_fft_filter_spectrum_sizes(ctx, n, rows):
     got = host(out).reshape(rows, n)
     ctx.set_options(filter_mode=cb.FILTER_F32)
     assert np.abs(got - want).max() <= 2e-6 * np.abs(want).max()
+
+
+def _mini(tmp_path, channels, nrows, ffs="none"):
+    """Planned small scan on a scanner of `channels` channels."""
+    from ctbangbang_amd import scans
+    d = str(tmp_path)
+    scans.mini_install(d, dict(scans.MINI_SCANNER, NChannels=channels, CentralChannel=channels / 2 - 0.25))
+    prm = str(tmp_path / "m.prm")
+    cb.write_prm(prm, scans.mini_tokens(ffs, nrows=nrows, rotations=max(12, 96 // nrows)))
+    mr = cb.metadata_from_prm(prm, install_dir=d)
+    cb.plan_block(mr, 0)
+    return mr
+
+
+@pytest.mark.parametrize("channels,nrows", [(4, 1), (60, 6), (64, 8), (68, 9), (132, 17)])
+def test_adaptive_smoothing_edges(ctx, tmp_path, channels, nrows):
+    """5x5x5 smoothing bit for bit at the edges of the 64-channel x 8-row wave
+    tile, in the first and last views, and around infinite and NaN samples."""
+    import oracle
+    mr = _mini(tmp_path, channels, nrows)
+    n = int(mr.ri.n_proj_pull)
+    rng = np.random.default_rng(channels + nrows)
+    raw = rng.random((n, nrows, channels)).astype(np.float32)
+    raw[n // 2, nrows // 2, channels // 2] = np.inf
+    raw[n // 2 + 9, 0, channels - 1] = np.nan
+    T = np.float32(0.6)
+    raw_d = dev(raw.ravel())
+    out = torch.empty_like(raw_d)
+    ctx.set_options(adaptive_threshold=float(T))
+    ctx.adaptive_filter_dev(mr, raw_d, out)
+    ctx.synchronize()
+    ctx.set_options(adaptive_threshold=0.0)
+    want = oracle.adaptive_apply(mr, raw.reshape(n, -1), np.full(n, T, dtype=np.float32))
+    assert np.count_nonzero(want != raw.reshape(n, -1)) > 0.2 * raw.size
+    assert np.array_equal(host(out).reshape(n, -1), want, equal_nan=True)
+    cb.free_metadata(mr)
