@@ -15,8 +15,14 @@
 // using FP64-derived per-channel coordinate maps (geometry.cpp).
 //
 // Output element (v, r, c) = rebinned projection v + add_projections, row r,
-// oversampled channel c.  Threads run along c (coalesced writes, raw reads at
-// channel ~c/2 of a handful of readings that stay in L1/L2).
+// oversampled channel c.  Threads run along c (coalesced writes).  In every
+// mode it interpolates linearly between two channel taps, each linear between
+// the readings p and p + 1 of its focal spot, p + f = (v + add) - aoff, and
+// aoff does not depend on the view: from one view to the next p moves by
+// exactly one reading, the upper one becoming the lower, and f stays but for
+// the rounding of the index.  A thread that walks kViews views therefore
+// loads one new sample per tap and view at an address that only advances by
+// a uniform step.
 //
 // Every raw sample the reconstruction uses reaches some rebinned sample
 // (non-finite values propagate through the interpolation), so the kernels
@@ -31,7 +37,15 @@ namespace ctbb {
 
 namespace {
 
-constexpr int kViewsPerThread = 8;
+// Views per thread (one more reading is loaded than views are written), and
+// views whose loads are in flight together.  1934 views of 64 rows x 1472
+// channels, four focal spots: 550 us (822 us with four loads per output and
+// the index arithmetic per view and tap); 16 to 128 views, batches of 4 or 8
+// and any occupancy from 4 waves per SIMD up stay within 545-575 us: the
+// kernel is bound by the cache lines a gather touches (a wave's 64 channels
+// lie on about 14 readings' rows), 90-110 cycles per CU and wave of output.
+constexpr int kViews = 16;
+constexpr int kBatch = 4;
 
 // Clamp a fractional index into [0, n-1] and split it into the two taps and
 // the weight of the upper tap (texture clamp addressing).
@@ -51,103 +65,166 @@ __device__ __forceinline__ void report_nonfinite(unsigned *flag, bool bad) {
         *reinterpret_cast<volatile unsigned *>(flag) = 1u;
 }
 
-// Base of frame f of the pull: with kHot the adaptive filter's output where
-// it changed the frame, the raw pull otherwise.
-template <bool kHot>
-__device__ __forceinline__ const float *frame_src(const RebinArgs &a, size_t f) {
-    if (!kHot) return a.raw;
-    return a.hot[f] ? a.raw_af : a.raw;
+// Smallest value over a wave (all lanes active), in a scalar register.
+__device__ __forceinline__ int wave_min(int v) {
+    for (int s = 32; s > 0; s >>= 1) v = min(v, __shfl_xor(v, s, 64));
+    return __builtin_amdgcn_readfirstlane(v);
 }
 
 // The (x, y, z) workgroups of the rebin's grid (x: 256 output channels, y:
-// row, z: kViewsPerThread views), in dispatch order, taken in a stride of
-// gridDim.x by the launched one-dimensional grid (fewer workgroups than the
-// grid has: the rebin then leaves room on every CU for a kernel launched
-// beside it).
+// row, z: kViews views), in dispatch order, taken in a stride of gridDim.x by
+// the launched one-dimensional grid (fewer workgroups than the grid has: the
+// rebin then leaves room on every CU for a kernel launched beside it).
 template <class F>
 __device__ __forceinline__ void for_each_block(const RebinArgs &a, F f) {
     const unsigned gx = static_cast<unsigned>(a.nos + 255) / 256u, gxy = gx * static_cast<unsigned>(a.n_rows);
-    const unsigned total = gxy * static_cast<unsigned>((a.n_proj_out + kViewsPerThread - 1) / kViewsPerThread);
+    const unsigned total = gxy * static_cast<unsigned>((a.n_proj_out + kViews - 1) / kViews);
     for (unsigned vb = blockIdx.x; vb < total; vb += gridDim.x) {
         const unsigned bz = vb / gxy, rem = vb - bz * gxy, br = rem / gx;
         f(rem - br * gx, br, bz);
     }
 }
 
+// kHot: frames whose flag a.hot is set come from a.raw_af (the adaptive
+// filter's output where it changed the frame), the others from the pull.
 template <bool kHot>
 __device__ __forceinline__ void rebin_block(const RebinArgs &a, unsigned bx, unsigned br, unsigned bz, bool &bad) {
-    const int c = static_cast<int>(bx) * 256 + static_cast<int>(threadIdx.x);
+    const int cl = static_cast<int>(bx) * 256 + static_cast<int>(threadIdx.x);
+    const int c = min(cl, a.nos - 1);                   // (lanes past the row repeat its last channel, unstored)
+    const bool store = cl < a.nos;
     const int r = static_cast<int>(br);
-    if (c >= a.nos) return;
-    const size_t frame = static_cast<size_t>(a.n_rows_raw) * a.nch;
-    const float *__restrict__ aoff = a.aoff;
-    float *__restrict__ outp = a.out;
-
-    int set, j;
-    if (a.kind == 0 || a.kind == 2) {
-        set = 0;
-        j = r;
-    } else {
-        // interleaved rows: set 0 (-dr focal spot(s)) -> row 2j, set 1 -> 2j+1,
-        // swapped with ReverseRowInterleave
-        set = (r & 1) ^ (a.reverse_rows ? 1 : 0);
-        j = r >> 1;
-    }
+    // set of the row (kinds 1 and 3 interleave rows: set 0, the -dr focal
+    // spot(s), -> row 2j, set 1 -> 2j + 1, swapped with ReverseRowInterleave)
+    const bool inter = (a.kind & 1) != 0;
+    const int set = inter ? (r & 1) ^ (a.reverse_rows ? 1 : 0) : 0;
+    const int j = inter ? r >> 1 : r;
+    // the two channel taps: raw channel, focal spot and azimuthal offset of
+    // each (kinds 0 and 1: neighbouring raw channels of one spot; 2 and 3:
+    // neighbouring oversampled channels, alternately of the set's two spots)
     const float by = a.bidx[set * a.nos + c];
-
-    // per-thread constants of the output channel (independent of the view)
-    int c0 = 0, c1 = 0, m0 = 0, m1 = 0;
-    float fc = 0.0f, fm = 0.0f, ao0, ao1 = 0.0f;
+    int t0, t1, ch0, ch1, fs0, fs1;
+    float fc, ao0, ao1;
     if (a.kind <= 1) {
-        taps(by, a.nch, c0, c1, fc);
-        ao0 = aoff[set * a.nos + c];
+        taps(by, a.nch, t0, t1, fc);
+        ch0 = t0;
+        ch1 = t1;
+        fs0 = fs1 = a.kind == 1 ? set : 0;
+        ao0 = ao1 = a.aoff[set * a.nos + c];
     } else {
-        taps(by, a.nos, m0, m1, fm);
-        ao0 = aoff[set * a.nos + m0];
-        ao1 = aoff[set * a.nos + m1];
+        taps(by, a.nos, t0, t1, fc);
+        ch0 = t0 >> 1;
+        ch1 = t1 >> 1;
+        fs0 = 2 * set + (t0 & 1);
+        fs1 = 2 * set + (t1 & 1);
+        ao0 = a.aoff[set * a.nos + t0];
+        ao1 = a.aoff[set * a.nos + t1];
     }
-
-    for (int vv = 0; vv < kViewsPerThread; vv++) {
-        const int v = static_cast<int>(bz) * kViewsPerThread + vv;
-        if (v >= a.n_proj_out) break;
-        const float proj = static_cast<float>(v + a.add);
-        float out;
-        if (a.kind <= 1) {
-            // single 2D bilinear fetch in (channel, sheet projection)
-            const int fs = a.kind == 1 ? set : 0;
-            int p0, p1;
-            float fa;
-            taps(proj - ao0, a.n_proj, p0, p1, fa);
-            const size_t f0 = static_cast<size_t>(p0) * a.n_ffs + fs, f1 = static_cast<size_t>(p1) * a.n_ffs + fs;
-            const float *s0 = frame_src<kHot>(a, f0) + static_cast<size_t>(j) * a.nch + f0 * frame;
-            const float *s1 = frame_src<kHot>(a, f1) + static_cast<size_t>(j) * a.nch + f1 * frame;
-            const float t0 = fmaf(fc, s0[c1] - s0[c0], s0[c0]);
-            const float t1 = fmaf(fc, s1[c1] - s1[c0], s1[c0]);
-            out = fmaf(fa, t1 - t0, t0);
-        } else {
-            // two-pass modes: radial tap pair over the interleaved azimuthal
-            // rebin of the focal-spot pair `set`
-            float t[2];
+    const int v0 = static_cast<int>(bz) * kViews;
+    const int n_v = min(kViews, a.n_proj_out - v0);
+    // reading of the lower azimuthal tap at view v0
+    const float fl0 = floorf(-ao0), fl1 = floorf(-ao1);
+    const int p0 = v0 + a.add + static_cast<int>(fl0), p1 = v0 + a.add + static_cast<int>(fl1);
+    const size_t frame = static_cast<size_t>(a.n_rows_raw) * a.nch;
+    float *out = a.out + (static_cast<size_t>(v0) * a.n_rows + r) * a.nos;
+    const size_t ostep = static_cast<size_t>(a.n_rows) * a.nos;
+    const size_t step = static_cast<size_t>(a.n_ffs) * frame;       // samples from one reading of a spot to the next
+    const int p_lo = wave_min(min(p0, p1)), p_hi = -wave_min(-max(p0, p1)) + n_v;
+    // every reading inside the pull, and all of them (and the output rows)
+    // within 32-bit byte offsets
+    bool plain = p_lo >= 0 && p_hi < a.n_proj &&
+                 static_cast<unsigned long long>(p_hi - p_lo + 1) * step < (1ull << 29) && kViews * ostep < (1ull << 29);
+    if (kHot && plain) {
+        // a wave whose readings the filter left alone reads the pull
+        bool h = false;
+        for (int f = p_lo * a.n_ffs + static_cast<int>(threadIdx.x & 63); f < (p_hi + 1) * a.n_ffs; f += 64)
+            h |= a.hot[f] != 0;
+        plain = __builtin_amdgcn_ballot_w64(h) == 0;
+    }
+    if (plain) {
+        // Buffer accesses: descriptors over the readings p_lo .. p_hi and the
+        // n_v output rows, constant 32-bit lane offsets, the view's step in
+        // the scalar offset.  A lane past the row has an output offset past
+        // the end and stores nothing.
+        const unsigned step_b = static_cast<unsigned>(step) * 4u, ostep_b = static_cast<unsigned>(ostep) * 4u;
+        const __amdgpu_buffer_rsrc_t src = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<float *>(a.raw + static_cast<size_t>(p_lo) * step), static_cast<short>(0),
+            static_cast<int>(static_cast<unsigned>(p_hi - p_lo + 1) * step_b), 0x00020000);
+        const __amdgpu_buffer_rsrc_t dst = __builtin_amdgcn_make_buffer_rsrc(
+            out, static_cast<short>(0), static_cast<int>(static_cast<unsigned>(n_v - 1) * ostep_b + a.nos * 4u),
+            0x00020000);
+        const unsigned fb = static_cast<unsigned>(frame) * 4u, jb = static_cast<unsigned>(j * a.nch) * 4u;
+        const int o0 = static_cast<int>(static_cast<unsigned>((p0 - p_lo) * a.n_ffs + fs0) * fb + jb + static_cast<unsigned>(ch0) * 4u);
+        const int o1 = static_cast<int>(static_cast<unsigned>((p1 - p_lo) * a.n_ffs + fs1) * fb + jb + static_cast<unsigned>(ch1) * 4u);
+        const int oc = store ? c * 4 : static_cast<int>(0x80000000u);
+        auto load = [&](int o, unsigned so) {
+            return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(src, o, static_cast<int>(so), 0));
+        };
+        float u0 = load(o0, 0), u1 = load(o1, 0);
+        unsigned so = 0, oo = 0;
+        float chk = 0.0f;           // NaN once an output is not finite
+        float proj = static_cast<float>(v0 + a.add);
+        auto view = [&](float w0, float w1) {
+            // weight of the upper reading: the FP32 index proj - aoff less the
+            // lower reading's number proj + floor(-aoff) (both steps exact but
+            // for the index's own rounding)
+            const float fa0 = (proj - ao0) - (proj + fl0), fa1 = (proj - ao1) - (proj + fl1);
+            proj += 1.0f;
+            const float x0 = fmaf(fa0, w0 - u0, u0), x1 = fmaf(fa1, w1 - u1, u1);
+            float y = fmaf(fc, x1 - x0, x0);
+            asm volatile("" : "+v"(y));     // one view after the other: no packing of several into wider registers
+            u0 = w0;
+            u1 = w1;
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(y), dst, oc, static_cast<int>(oo), 0);
+            chk = fmaf(y, 0.0f, chk);
+            oo += ostep_b;
+        };
+        int vv = 0;
+#pragma unroll 1
+        for (; vv + kBatch <= n_v; vv += kBatch) {
+            float w0[kBatch], w1[kBatch];
 #pragma unroll
-            for (int h = 0; h < 2; h++) {
-                const int m = h ? m1 : m0;
-                const int fs = 2 * set + (m & 1);
-                const int ch = m >> 1;
-                int p0, p1;
-                float fa;
-                taps(proj - (h ? ao1 : ao0), a.n_proj, p0, p1, fa);
-                const size_t f0 = static_cast<size_t>(p0) * a.n_ffs + fs, f1 = static_cast<size_t>(p1) * a.n_ffs + fs;
-                const float u0 = frame_src<kHot>(a, f0)[static_cast<size_t>(j) * a.nch + ch + f0 * frame];
-                const float u1 = frame_src<kHot>(a, f1)[static_cast<size_t>(j) * a.nch + ch + f1 * frame];
-                t[h] = fmaf(fa, u1 - u0, u0);
+            for (int e = 0; e < kBatch; e++) {
+                so += step_b;
+                w0[e] = load(o0, so);
+                w1[e] = load(o1, so);
             }
-            out = fmaf(fm, t[1] - t[0], t[0]);
+            __builtin_amdgcn_sched_barrier(0);      // all of the batch's loads in flight
+#pragma unroll
+            for (int e = 0; e < kBatch; e++) view(w0[e], w1[e]);
         }
-        outp[(static_cast<size_t>(v) * a.n_rows + r) * a.nos + c] = out;
-        bad |= !__builtin_isfinite(out);
+#pragma unroll 1
+        for (; vv < n_v; vv++) {
+            so += step_b;
+            view(load(o0, so), load(o1, so));
+        }
+        bad |= chk != 0.0f;         // (true for NaN)
+        return;
+    }
+    // readings clamped into the pull, each from its own source
+    auto sample = [&](int p, int fs, int ch) {
+        const size_t f = static_cast<size_t>(min(max(p, 0), a.n_proj - 1)) * a.n_ffs + fs;
+        const float *s = kHot && a.hot[f] ? a.raw_af : a.raw;
+        return s[f * frame + static_cast<size_t>(j) * a.nch + ch];
+    };
+    out += c;
+    float u0 = sample(p0, fs0, ch0), u1 = sample(p1, fs1, ch1);
+#pragma unroll 1
+    for (int vv = 0; vv < n_v; vv++) {
+        const float proj = static_cast<float>(v0 + a.add + vv);
+        const float fa0 = (proj - ao0) - (proj + fl0), fa1 = (proj - ao1) - (proj + fl1);
+        const float w0 = sample(p0 + vv + 1, fs0, ch0), w1 = sample(p1 + vv + 1, fs1, ch1);
+        const float x0 = fmaf(fa0, w0 - u0, u0), x1 = fmaf(fa1, w1 - u1, u1);
+        const float y = fmaf(fc, x1 - x0, x0);
+        u0 = w0;
+        u1 = w1;
+        if (store) *out = y;
+        bad |= !__builtin_isfinite(y);
+        out += ostep;
     }
 }
 
+// One workgroup per (x, y, z) block of the grid.  Few registers: waves of it
+// fit in the 64 per lane a running backprojection leaves.
 template <bool kHot>
 __global__ __launch_bounds__(256) void rebin_kernel(RebinArgs a) {
     bool bad = false;
@@ -155,112 +232,12 @@ __global__ __launch_bounds__(256) void rebin_kernel(RebinArgs a) {
     report_nonfinite(a.nonfinite, bad);
 }
 
-// The same arithmetic with 32-bit byte offsets from the (uniform) raw and
-// output bases, one template per channel-tap form (kinds 0/1: bilinear in
-// raw channel and azimuth; 2/3: two oversampled-channel taps, each bilinear
-// in azimuth), for pulls and outputs below 4 GiB.  Few registers (<= 32
-// VGPRs), so its waves fit beside a running backprojection (4 waves per SIMD
-// of 112 VGPRs leave 64 per lane) and the rebin of the next block overlaps
-// it.
-__device__ __forceinline__ float ld(const float *base, unsigned boff) {
-    return *reinterpret_cast<const float *>(reinterpret_cast<const char *>(base) + boff);
-}
-
-// Sample at byte offset boff of frame f (kHot: from the adaptive filter's
-// output where it changed frame f).
-template <bool kHot>
-__device__ __forceinline__ float ld_frame(const RebinArgs &a, unsigned f, unsigned boff) {
-    if (!kHot) return ld(a.raw, boff);
-    return ld(a.hot[f] ? a.raw_af : a.raw, boff);
-}
-
-template <bool kSplit, bool kHot>
-__device__ __forceinline__ void rebin32_block(const RebinArgs &a, unsigned bx, unsigned br, unsigned bz, bool &bad) {
-    const int c = bx * blockDim.x + threadIdx.x;
-    const int r = br;
-    if (c >= a.nos) return;
-    const unsigned frame_b = static_cast<unsigned>(a.n_rows_raw * a.nch) * 4u;
-    int set, j;
-    if (a.kind == 0 || a.kind == 2) {
-        set = 0;
-        j = r;
-    } else {
-        set = (r & 1) ^ (a.reverse_rows ? 1 : 0);
-        j = r >> 1;
-    }
-    const float by = a.bidx[set * a.nos + c];
-    int c0, c1;
-    float fc, ao0, ao1 = 0.0f;
-    if (!kSplit) {
-        taps(by, a.nch, c0, c1, fc);
-        ao0 = a.aoff[set * a.nos + c];
-    } else {
-        taps(by, a.nos, c0, c1, fc);
-        ao0 = a.aoff[set * a.nos + c0];
-        ao1 = a.aoff[set * a.nos + c1];
-    }
-    const unsigned row_b = static_cast<unsigned>(j * a.nch) * 4u;
-    const int v0 = bz * kViewsPerThread;
-    unsigned ob = (static_cast<unsigned>(v0 * a.n_rows + r) * static_cast<unsigned>(a.nos) + c) * 4u;
-    const unsigned ostep = static_cast<unsigned>(a.n_rows * a.nos) * 4u;
-    for (int vv = 0; vv < kViewsPerThread; vv++) {
-        const int v = v0 + vv;
-        if (v >= a.n_proj_out) break;
-        const float proj = static_cast<float>(v + a.add);
-        float out;
-        if (!kSplit) {
-            const unsigned fs = a.kind == 1 ? static_cast<unsigned>(set) : 0u;
-            int p0, p1;
-            float fa;
-            taps(proj - ao0, a.n_proj, p0, p1, fa);
-            const unsigned f0 = static_cast<unsigned>(p0 * a.n_ffs) + fs, f1 = static_cast<unsigned>(p1 * a.n_ffs) + fs;
-            const unsigned b0 = f0 * frame_b + row_b, b1 = f1 * frame_b + row_b;
-            const float s00 = ld_frame<kHot>(a, f0, b0 + 4u * c0), s01 = ld_frame<kHot>(a, f0, b0 + 4u * c1);
-            const float s10 = ld_frame<kHot>(a, f1, b1 + 4u * c0), s11 = ld_frame<kHot>(a, f1, b1 + 4u * c1);
-            const float t0 = fmaf(fc, s01 - s00, s00);
-            const float t1 = fmaf(fc, s11 - s10, s10);
-            out = fmaf(fa, t1 - t0, t0);
-        } else {
-            float t[2];
-#pragma unroll
-            for (int h = 0; h < 2; h++) {
-                const int m = h ? c1 : c0;
-                const unsigned fs = static_cast<unsigned>(2 * set + (m & 1));
-                const unsigned ch_b = row_b + 4u * static_cast<unsigned>(m >> 1);
-                int p0, p1;
-                float fa;
-                taps(proj - (h ? ao1 : ao0), a.n_proj, p0, p1, fa);
-                const unsigned f0 = static_cast<unsigned>(p0 * a.n_ffs) + fs, f1 = static_cast<unsigned>(p1 * a.n_ffs) + fs;
-                const float u0 = ld_frame<kHot>(a, f0, f0 * frame_b + ch_b);
-                const float u1 = ld_frame<kHot>(a, f1, f1 * frame_b + ch_b);
-                t[h] = fmaf(fa, u1 - u0, u0);
-            }
-            out = fmaf(fc, t[1] - t[0], t[0]);
-        }
-        *reinterpret_cast<float *>(reinterpret_cast<char *>(a.out) + ob) = out;
-        bad |= !__builtin_isfinite(out);
-        ob += ostep;
-    }
-}
-
-// One workgroup per (x, y, z) block of the grid.  At most 32 VGPRs (the
-// attribute counts pairs here): two waves per SIMD fit in the 64 per lane a
-// running backprojection leaves.
-template <bool kSplit, bool kHot>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8), amdgpu_num_vgpr(16))) void rebin32_kernel(
-    RebinArgs a) {
-    bool bad = false;
-    rebin32_block<kSplit, kHot>(a, blockIdx.x, blockIdx.y, blockIdx.z, bad);
-    report_nonfinite(a.nonfinite, bad);
-}
-
 // A one-dimensional grid of RebinArgs::max_groups workgroups looping over the
-// blocks, at most 32 VGPRs as above.
-template <bool kSplit, bool kHot>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8), amdgpu_num_vgpr(16))) void rebin32_loop_kernel(
-    RebinArgs a) {
+// blocks.
+template <bool kHot>
+__global__ __launch_bounds__(256) void rebin_loop_kernel(RebinArgs a) {
     bool bad = false;
-    for_each_block(a, [&](unsigned bx, unsigned br, unsigned bz) { rebin32_block<kSplit, kHot>(a, bx, br, bz, bad); });
+    for_each_block(a, [&](unsigned bx, unsigned br, unsigned bz) { rebin_block<kHot>(a, bx, br, bz, bad); });
     report_nonfinite(a.nonfinite, bad);
 }
 
@@ -273,39 +250,18 @@ int launch_rebin(const RebinArgs &a, hipStream_t stream) {
     if (a.add < 0 || a.add + a.n_proj_out > a.n_proj) return CTBB_ERR_SHAPE;
     const int rows_needed = (a.kind == 1 || a.kind == 3) ? 2 * a.n_rows_raw : a.n_rows_raw;
     if (a.n_rows != rows_needed) return CTBB_ERR_SHAPE;
-    const dim3 grid((a.nos + 255) / 256, a.n_rows, (a.n_proj_out + kViewsPerThread - 1) / kViewsPerThread);
+    const dim3 grid((a.nos + 255) / 256, a.n_rows, (a.n_proj_out + kViews - 1) / kViews);
     if (grid.z > 65535u || grid.y > 65535u || a.max_groups < 0) return CTBB_ERR_SHAPE;
     const unsigned long long blocks = static_cast<unsigned long long>(grid.x) * grid.y * grid.z;
-    const unsigned long long raw_bytes = static_cast<unsigned long long>(a.n_proj) * a.n_ffs * a.n_rows_raw * a.nch * 4ull;
-    const unsigned long long out_bytes = static_cast<unsigned long long>(a.n_proj_out) * a.n_rows * a.nos * 4ull;
     const bool hot = a.hot != nullptr;
-    if (raw_bytes < (1ull << 32) && out_bytes < (1ull << 32)) {
-        if (a.max_groups > 0 && static_cast<unsigned long long>(a.max_groups) < blocks) {
-            const dim3 g1(static_cast<unsigned>(a.max_groups));
-            if (a.kind <= 1 && !hot)
-                hipLaunchKernelGGL((rebin32_loop_kernel<false, false>), g1, dim3(256), 0, stream, a);
-            else if (a.kind <= 1)
-                hipLaunchKernelGGL((rebin32_loop_kernel<false, true>), g1, dim3(256), 0, stream, a);
-            else if (!hot)
-                hipLaunchKernelGGL((rebin32_loop_kernel<true, false>), g1, dim3(256), 0, stream, a);
-            else
-                hipLaunchKernelGGL((rebin32_loop_kernel<true, true>), g1, dim3(256), 0, stream, a);
-        } else if (a.kind <= 1 && !hot) {
-            hipLaunchKernelGGL((rebin32_kernel<false, false>), grid, dim3(256), 0, stream, a);
-        } else if (a.kind <= 1) {
-            hipLaunchKernelGGL((rebin32_kernel<false, true>), grid, dim3(256), 0, stream, a);
-        } else if (!hot) {
-            hipLaunchKernelGGL((rebin32_kernel<true, false>), grid, dim3(256), 0, stream, a);
-        } else {
-            hipLaunchKernelGGL((rebin32_kernel<true, true>), grid, dim3(256), 0, stream, a);
-        }
+    if (a.max_groups > 0 && static_cast<unsigned long long>(a.max_groups) < blocks) {
+        const dim3 g1(static_cast<unsigned>(a.max_groups));
+        if (hot) hipLaunchKernelGGL(rebin_loop_kernel<true>, g1, dim3(256), 0, stream, a);
+        else hipLaunchKernelGGL(rebin_loop_kernel<false>, g1, dim3(256), 0, stream, a);
+    } else if (hot) {
+        hipLaunchKernelGGL(rebin_kernel<true>, grid, dim3(256), 0, stream, a);
     } else {
-        // (more than 32 VGPRs: long-lived workgroups of it would keep a
-        // backprojection workgroup off their CU, so its grid stays whole)
-        if (hot)
-            hipLaunchKernelGGL(rebin_kernel<true>, grid, dim3(256), 0, stream, a);
-        else
-            hipLaunchKernelGGL(rebin_kernel<false>, grid, dim3(256), 0, stream, a);
+        hipLaunchKernelGGL(rebin_kernel<false>, grid, dim3(256), 0, stream, a);
     }
     return hipGetLastError() == hipSuccess ? CTBB_OK : CTBB_ERR_HIP;
 }

@@ -39,13 +39,17 @@ def test_fft_filter_spectrum_sizes(ctx, n, rows):
     assert np.abs(got - want).max() <= 2e-6 * np.abs(want).max()
 
 
-def _mini(tmp_path, channels, nrows, ffs="none"):
-    """Planned small scan on a scanner of `channels` channels."""
+def _mini(tmp_path, channels, nrows, ffs="none", turn=192, centre=None, **scanner):
+    """Planned small scan on a scanner of `channels` channels and `turn`
+    projections per turn."""
     from ctbangbang_amd import scans
     d = str(tmp_path)
-    scans.mini_install(d, dict(scans.MINI_SCANNER, NChannels=channels, CentralChannel=channels / 2 - 0.25))
+    scans.mini_install(d, dict(scans.MINI_SCANNER, NChannels=channels, NProjTurn=turn,
+                               CentralChannel=channels / 2 - 0.25 if centre is None else centre, **scanner))
     prm = str(tmp_path / "m.prm")
-    cb.write_prm(prm, scans.mini_tokens(ffs, nrows=nrows, rotations=max(12, 96 // nrows)))
+    tok = scans.mini_tokens(ffs, nrows=nrows, rotations=max(12, 96 // nrows))
+    tok["Readings"] = tok["Readings"] // 192 * turn
+    cb.write_prm(prm, tok)
     mr = cb.metadata_from_prm(prm, install_dir=d)
     cb.plan_block(mr, 0)
     return mr
@@ -72,4 +76,30 @@ def test_adaptive_smoothing_edges(ctx, tmp_path, channels, nrows):
     want = oracle.adaptive_apply(mr, raw.reshape(n, -1), np.full(n, T, dtype=np.float32))
     assert np.count_nonzero(want != raw.reshape(n, -1)) > 0.2 * raw.size
     assert np.array_equal(host(out).reshape(n, -1), want, equal_nan=True)
+    cb.free_metadata(mr)
+
+
+@pytest.mark.parametrize("ffs,channels,nrows,centre,reverse", [
+    ("none", 28, 1, None, 0), ("none", 33, 3, 20.0, 0), ("phi", 66, 2, None, 0), ("z", 97, 4, 30.0, 1),
+    ("both", 129, 4, None, 1), ("both", 130, 6, 100.0, 0)])
+def test_rebin_edges(ctx, tmp_path, ffs, channels, nrows, centre, reverse):
+    """Rebinning where a row ends inside a wave or a workgroup, with a number
+    of views that is no multiple of a thread's, swapped row interleave, and a
+    detector so far off centre that readings before and after the pull are
+    clamped.  Tolerance: the stage's 2e-5 of the largest raw sample, and the
+    azimuthal index's FP32 rounding (half a unit in the last place of the
+    number of readings, for each of the two taps) times the largest step
+    between two readings (1)."""
+    import oracle
+    mr = _mini(tmp_path, channels, nrows, ffs, turn=190, centre=centre, ReverseRowInterleave=reverse)
+    s = cb.block_sizes(mr)
+    rng = np.random.default_rng(channels)
+    raw = rng.random(s.raw_pull).astype(np.float32)
+    out = torch.empty(s.rebin, dtype=torch.float32, device="cuda")
+    raw_d = dev(raw)
+    ctx.rebin_dev(mr, raw_d, out)
+    ctx.synchronize()
+    want = oracle.rebin(mr, raw, double=True)
+    got = host(out).reshape(want.shape)
+    assert np.abs(got - want).max() <= 2e-5 + np.spacing(np.float32(mr.ri.n_proj_pull // mr.ri.n_ffs))
     cb.free_metadata(mr)
