@@ -7,14 +7,15 @@
 // arithmetic in the same order (including the fused multiply-adds nvcc forms
 // for "acc += a*b"), so results are bit-identical to a sequential FP32
 // restatement:
-//   1. view maximum         one workgroup per view, tree max (order-free)
+//   1. view maximum         one workgroup per view, tree max (order-free); the
+//      stage copies the pull on the way
 //   2. 18-degree smoothing  one thread per view, sequential fmaf sum
 //   3. 180-degree min/max + eccentricity, and
 //   4. threshold bisection  one wavefront per view: the view's window is
-//      copied once to LDS (min and max taken on the way, order-free), then
+//      held in registers (min and max taken on the way, order-free), then
 //      exact integer counts over it
-//   5. 5x5x5 triangle smoothing of samples above threshold: one thread per
-//      sample (coalesced along channels)
+//   5. 5x5x5 triangle smoothing of samples above threshold: a wave takes 64
+//      channels x 8 rows of a view
 // A fixed-threshold mode (no counterpart in the reference) skips steps 1-4
 // and smooths the samples above one given line-integral threshold, e.g.
 // ln(I0 / N) for a noise threshold of N photons at I0 incident photons.
@@ -42,15 +43,22 @@ __device__ __forceinline__ float wave_min(float v) {
 
 // View maximum, one workgroup per view (max is order-free, so any reduction
 // order gives the reference's value), gridDim.x workgroups looping over the
-// n_proj views.  frame % 4 == 0 is checked on the host.
-__global__ __launch_bounds__(256) void af_sup(const float *raw, float *sup, size_t frame, int n_proj) {
+// n_proj views.  frame % 4 == 0 is checked on the host.  kCopy: the frame is
+// also copied to out (16-byte stores), so that the apply step only rewrites
+// the views the filter changes instead of reading the whole pull again:
+// bound by HBM, 8448 views of 32 x 736 in 304 us (5.2 TB/s) against 163 us for the
+// maximum and 261 us for an apply step over every view.
+template <bool kCopy>
+__global__ __launch_bounds__(256) void af_sup(const float *raw, float *sup, float *out, size_t frame, int n_proj) {
     __shared__ float red[4];
     for (int p = blockIdx.x; p < n_proj; p += gridDim.x) {
         const float4 *f = reinterpret_cast<const float4 *>(raw + static_cast<size_t>(p) * frame);
+        float4 *o = reinterpret_cast<float4 *>(out + static_cast<size_t>(p) * frame);
         float m = 0.0f;   // reference starts from 0.0f (preprocessing.cuh:75)
         for (size_t i = threadIdx.x; i < frame / 4; i += 256) {
             const float4 v = f[i];
             m = fmaxf(fmaxf(m, fmaxf(v.x, v.y)), fmaxf(v.z, v.w));
+            if (kCopy) o[i] = v;
         }
         m = wave_max(m);
         if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
@@ -60,20 +68,26 @@ __global__ __launch_bounds__(256) void af_sup(const float *raw, float *sup, size
     }
 }
 
-// reference preprocessing.cuh:87-113
-__global__ void af_smooth(const float *sup, float *sm, int n_proj, int n_avg) {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= n_proj) return;
-    const int off = n_avg / 2;
-    const int max_idx = n_proj - 1;
+// reference preprocessing.cuh:87-113.  64 views per workgroup, their window
+// of maxima (edge indices clamped) in LDS: the n_avg dependent fused
+// multiply-adds then wait for LDS instead of memory (8448 views, n_avg 231:
+// 5.3 against 23 us).
+constexpr int kSmoothViews = 64;
+
+__global__ __launch_bounds__(kSmoothViews) void af_smooth(const float *sup, float *sm, int n_proj, int n_avg) {
+    extern __shared__ float w[];                // [kSmoothViews + n_avg]
+    const int p0 = blockIdx.x * kSmoothViews, off = n_avg / 2, max_idx = n_proj - 1;
+    for (int i = threadIdx.x; i < kSmoothViews + n_avg; i += kSmoothViews) {
+        int idx = p0 - off + i;
+        idx = idx < 0 ? 0 : (idx > max_idx ? max_idx : idx);
+        w[i] = sup[idx];
+    }
+    __syncthreads();
     const float inv = 1.0f / static_cast<float>(n_avg);
     float acc = 0.0f;
-    for (int i = 0; i < n_avg; i++) {
-        int idx = p - off + i;
-        idx = idx < 0 ? 0 : (idx > max_idx ? max_idx : idx);
-        acc = fmaf(inv, sup[idx], acc);
-    }
-    sm[p] = acc;
+#pragma unroll 8
+    for (int i = 0; i < n_avg; i++) acc = fmaf(inv, w[threadIdx.x + i], acc);
+    if (p0 + static_cast<int>(threadIdx.x) < n_proj) sm[p0 + threadIdx.x] = acc;
 }
 
 // The counting window of reference preprocessing.cuh:32-62 (clipped to the
@@ -87,45 +101,44 @@ __device__ __forceinline__ void af_window(int &start_idx, int &numel_range, int 
     if (diff > max_idx) numel_range -= (diff - max_idx);
 }
 
-// rhs of reference preprocessing.cuh:32-62 for a window of numel values:
-// the exact count of values above T, then the reference's float products.
-__device__ __forceinline__ float af_rhs_wave(const float *win, int numel, float T, float inv_pi_npf_a,
-                                             float inv_npf) {
-    int cnt = 0;
-    for (int i = threadIdx.x & 63; i < numel; i += 64) cnt += win[i] > T ? 1 : 0;
-    for (int s = 32; s > 0; s >>= 1) cnt += __shfl_xor(cnt, s, 64);
-    return inv_pi_npf_a * static_cast<float>(cnt) * inv_npf;
-}
-
 // reference preprocessing.cuh:115-206; one wavefront per view.  The view's
-// window is copied to LDS once (kLds, when it fits in the dynamic LDS the
-// host gives the launch), its minimum and maximum taken on the way (the
-// reference's 180-degree range, preprocessing.cuh:115-163: the same views as
-// the counting window, its clamped edge indices repeat values inside it),
-// and every bisection step counts from there; otherwise each step reads the
-// window from memory.
-template <bool kLds>
+// window stays in registers (kVals per lane, lane l the values l, l + 64,
+// ...; kVals = 0: windows over 64 * 44 values are read from memory at every
+// step), its minimum and maximum taken on the way (the reference's 180-degree
+// range, preprocessing.cuh:115-163: the same views as the counting window,
+// its clamped edge indices repeat values inside it).  A bisection step counts
+// the values above T exactly with one compare per register and scalar
+// population counts; once the counts at both ends of the interval agree no
+// value lies between them, every later count is the same and only T moves.
+// Bound by instruction issue: 8448 views with 2305 values 51 us against
+// 111 us with the window in LDS, shuffles and a count at every step (four
+// waves per view, which repeat the scalar steps: 61 us).
+template <int kVals>
 __global__ __launch_bounds__(64) void af_thresh(const float *sm, float *thr, int n_proj, int n_range, int n_proj_ffs,
                                                 float strength) {
-    extern __shared__ float win_lds[];
-    const int p = blockIdx.x;
+    const int p = blockIdx.x, lane = threadIdx.x;
     const int max_idx = n_proj - 1;
     int start = p - n_range / 2, numel = n_range;
     af_window(start, numel, max_idx);
     const float *win = sm + start;
+    float v[kVals > 0 ? kVals : 1];
     float hi = 0.0f, lo = 10000.0f;     // the reference's starting values
-    for (int i = threadIdx.x; i < numel; i += 64) {
-        const float v = win[i];
-        hi = fmaxf(hi, v);
-        lo = fminf(lo, v);
-        if (kLds) win_lds[i] = v;
+    if (kVals > 0) {
+#pragma unroll
+        for (int q = 0; q < kVals; q++) {
+            const float x = win[min(64 * q + lane, numel - 1)];     // (unconditional: all loads in flight)
+            hi = fmaxf(hi, x);
+            lo = fminf(lo, x);
+            v[q] = 64 * q + lane < numel ? x : -1.0f;               // (never above T >= 0)
+        }
+    } else {
+        for (int i = lane; i < numel; i += 64) {
+            hi = fmaxf(hi, win[i]);
+            lo = fminf(lo, win[i]);
+        }
     }
     hi = wave_max(hi);
     lo = wave_min(lo);
-    if (kLds) {
-        __syncthreads();
-        win = win_lds;
-    }
     float e = 1 - lo / hi;
     e = (e - 0.3f) / (0.5f - 0.3f);
     const float ecc = e > 1 ? 1.0f : (e < 0 ? 0.0f : e);
@@ -134,18 +147,48 @@ __global__ __launch_bounds__(64) void af_thresh(const float *sm, float *thr, int
     float lower = lo, upper = hi;
     float T = (hi + lo) / 2.0f;
     const float lhs = 0.03f * strength * ecc;
-    float rhs = af_rhs_wave(win, numel, T, inv_pi, inv_npf);
+    auto count = [&](float t) {
+        int cnt = 0;
+        if (kVals > 0) {
+#pragma unroll
+            for (int q = 0; q < kVals; q++) cnt += __builtin_popcountll(__builtin_amdgcn_ballot_w64(v[q] > t));
+        } else {
+            for (int i0 = 0; i0 < numel; i0 += 64)
+                cnt += __builtin_popcountll(__builtin_amdgcn_ballot_w64(i0 + lane < numel && win[i0 + lane] > t));
+        }
+        return cnt;
+    };
+    // rhs of reference preprocessing.cuh:32-62: the exact count of values
+    // above T, then the reference's float products
+    int cnt = count(T), cnt_lower = -1, cnt_upper = 0;  // (above the maximum: none)
+    float rhs = inv_pi * static_cast<float>(cnt) * inv_npf;
     int iter = 0;
     while (static_cast<double>(fabsf(lhs - rhs) / lhs) > 0.01) {
         if (iter >= 20) break;
         iter += 1;
-        if (rhs > lhs) lower = T;
-        else if (rhs < lhs) upper = T;
-        else break;
+        if (rhs > lhs) {
+            lower = T;
+            cnt_lower = cnt;
+        } else if (rhs < lhs) {
+            upper = T;
+            cnt_upper = cnt;
+        } else {
+            break;
+        }
         T = (lower + upper) / 2.0f;
-        rhs = af_rhs_wave(win, numel, T, inv_pi, inv_npf);
+        if (cnt_lower == cnt_upper) {
+            // rhs, and with it the test and the side taken, stays
+            for (; iter < 20; iter++) {
+                if (rhs > lhs) lower = T;
+                else upper = T;
+                T = (lower + upper) / 2.0f;
+            }
+            break;
+        }
+        cnt = count(T);
+        rhs = inv_pi * static_cast<float>(cnt) * inv_npf;
     }
-    if (threadIdx.x == 0) thr[p] = T;
+    if (lane == 0) thr[p] = T;
 }
 
 // Apply step, reference preprocessing.cuh:208-285 (3D branch, __FILTER_3D__
@@ -174,6 +217,11 @@ constexpr int kRows = 8;
 
 __device__ __forceinline__ constexpr int af_tri(int i) { return 3 - (i < 3 ? 3 - i : i - 3); }
 
+// kGroup rows are loaded at a time: with smoothed samples everywhere the other
+// waves cover the loads and one row at a time needs the fewest registers (0.36
+// against 0.39 ms for two); where few waves smooth, each waits for memory at
+// every group.
+template <int kGroup>
 __device__ __forceinline__ void af_smooth_rows(const float *raw, float (&acc)[kRows], int i, int j0, int p, int n_proj,
                                                int n_rows_raw, int nch, size_t ps) {
     __amdgpu_buffer_rsrc_t rs[5];
@@ -195,21 +243,28 @@ __device__ __forceinline__ void af_smooth_rows(const float *raw, float (&acc)[kR
         // stays past the end of every frame (< 2 GiB) for all kRows + 4 rows
         int off = c >= 0 && c < nch ? (j0 - 2) * row_b + c * 4 : static_cast<int>(0x80000000u);
         const bool c_in = off != static_cast<int>(0x80000000u);
+        static_assert((kRows + 4) % kGroup == 0, "whole groups of rows");
 #pragma unroll
-        for (int q = 0; q < kRows + 4; q++) {           // row j0 - 2 + q
-            float v[5];
+        for (int q0 = 0; q0 < kRows + 4; q0 += kGroup) {
+            float v[kGroup][5];
 #pragma unroll
-            for (int kk = 0; kk < 5; kk++)
-                v[kk] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs[kk], off, 0, 0));
-            off = c_in ? off + row_b : off;
-#pragma unroll
-            for (int r = 0; r < kRows; r++) {
-                const int jj = q - r;                   // output row j0 + r sees it as row offset jj - 2
-                if (jj < 0 || jj > 4) continue;
+            for (int g = 0; g < kGroup; g++) {          // row j0 - 2 + q0 + g
 #pragma unroll
                 for (int kk = 0; kk < 5; kk++)
-                    acc[r] = fmaf(v[kk], ta + static_cast<float>(af_tri(jj) + af_tri(kk) + 1), acc[r]);
+                    v[g][kk] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs[kk], off, 0, 0));
+                off = c_in ? off + row_b : off;
             }
+            if (kGroup > 1) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int g = 0; g < kGroup; g++)
+#pragma unroll
+                for (int r = 0; r < kRows; r++) {
+                    const int jj = q0 + g - r;          // output row j0 + r sees it as row offset jj - 2
+                    if (jj < 0 || jj > 4) continue;
+#pragma unroll
+                    for (int kk = 0; kk < 5; kk++)
+                        acc[r] = fmaf(v[g][kk], ta + static_cast<float>(af_tri(jj) + af_tri(kk) + 1), acc[r]);
+                }
         }
     }
 }
@@ -233,7 +288,9 @@ __device__ __forceinline__ float af_norm(int i, int j, int p, int n_proj, int n_
     return static_cast<float>(si * nj * nk + sj * ni * nk + sk * ni * nj + ni * nj * nk);
 }
 
-// Rows j0 .. j0 + kRows - 1 of channels i (one per lane) of view p.
+// Rows j0 .. j0 + kRows - 1 of channels i (one per lane) of view p; kCopied:
+// out already holds the raw samples, only waves that smooth some are written.
+template <bool kCopied, int kGroup>
 __device__ __forceinline__ void af_apply_rows(const float *raw, float T, float *out, int i, int j0, int p, int n_proj,
                                               int n_rows_raw, int nch, size_t ps) {
     const size_t base = ps * p + static_cast<size_t>(j0) * nch + i;
@@ -246,10 +303,12 @@ __device__ __forceinline__ void af_apply_rows(const float *raw, float T, float *
     }
     if (__builtin_amdgcn_ballot_w64(hot)) {
         float acc[kRows];
-        af_smooth_rows(raw, acc, i, j0, p, n_proj, n_rows_raw, nch, ps);
+        af_smooth_rows<kGroup>(raw, acc, i, j0, p, n_proj, n_rows_raw, nch, ps);
 #pragma unroll
         for (int r = 0; r < kRows; r++)
             if (x[r] > T) x[r] = (1.0f / af_norm(i, j0 + r, p, n_proj, n_rows_raw, nch)) * acc[r];
+    } else if (kCopied) {
+        return;
     }
 #pragma unroll
     for (int r = 0; r < kRows; r++)
@@ -262,39 +321,35 @@ __host__ __device__ __forceinline__ int af_view_waves(int n_rows_raw, int nch) {
 }
 
 // bpv workgroups of 4 waves per view, XCD x the x-th eighth of the views.
-// kHot: only the views the filter changes (view p is unchanged where its
-// maximum, af_sup from 0, is at or below its threshold); hot[p] flags them,
-// and a reader takes the other views from the raw pull (C1: about 6% of the
-// views are hot).  37 VGPRs: a wave of it fits beside a backprojection's four.
-template <bool kHot>
-__device__ __forceinline__ void af_apply_block(const float *raw, const float *sup, const float *thr, float *out,
-                                               unsigned char *hot, int n_proj, int n_rows_raw, int nch, int bpv) {
+enum ApplyMode {
+    kAllViews,      // every view
+    kHotFlagged,    // only the views the filter changes (view p is unchanged where its maximum, af_sup from 0, is at or
+                    // below its threshold); hot[p] flags them, a reader takes the others from the raw pull
+    kHotCopied      // only those views, and of them only the samples it changes: out holds a copy of the pull
+};
+
+// (kHotFlagged takes 56 VGPRs: beside a backprojection's four waves of 112 one
+// of it fits.)
+template <int kMode>
+__global__ __launch_bounds__(256) void af_apply(const float *raw, const float *sup, const float *thr, float *out,
+                                                unsigned char *hot, int n_proj, int n_rows_raw, int nch, int bpv) {
     const int xcd = blockIdx.x & 7, idx = blockIdx.x >> 3, band = (n_proj + 7) / 8;
     const int pv = idx / bpv, p = xcd * band + pv, part = idx - pv * bpv;
     if (pv >= band || p >= n_proj) return;
     const float T = thr[p];
-    if (kHot) {
+    if (kMode != kAllViews) {
         const bool h = sup[p] > T;
-        if (part == 0 && threadIdx.x == 0) hot[p] = h ? 1 : 0;
+        if (kMode == kHotFlagged && part == 0 && threadIdx.x == 0) hot[p] = h ? 1 : 0;
         if (!h) return;
     }
-    const int tiles = (nch + 63) / 64;
-    const int w = part * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    if (w >= af_view_waves(n_rows_raw, nch)) return;
-    const int g = w / tiles;
-    af_apply_rows(raw, T, out, (w - g * tiles) * 64 + (threadIdx.x & 63), g * kRows, p, n_proj, n_rows_raw, nch,
-                  static_cast<size_t>(nch) * n_rows_raw);
-}
-
-__global__ __launch_bounds__(256) void af_apply(const float *raw, const float *thr, float *out, int n_proj,
-                                                int n_rows_raw, int nch, int bpv) {
-    af_apply_block<false>(raw, nullptr, thr, out, nullptr, n_proj, n_rows_raw, nch, bpv);
-}
-
-__global__ __launch_bounds__(256) void af_apply_hot(
-    const float *raw, const float *sup, const float *thr, float *out, unsigned char *hot, int n_proj, int n_rows_raw,
-    int nch, int bpv) {
-    af_apply_block<true>(raw, sup, thr, out, hot, n_proj, n_rows_raw, nch, bpv);
+    const int tiles = (nch + 63) / 64, waves = af_view_waves(n_rows_raw, nch);
+#pragma unroll 1
+    for (int w = part * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); w < waves; w += 4 * bpv) {
+        const int g = w / tiles;
+        af_apply_rows<kMode == kHotCopied, kMode == kAllViews ? 1 : 2>(
+            raw, T, out, (w - g * tiles) * 64 + (threadIdx.x & 63), g * kRows, p, n_proj, n_rows_raw, nch,
+            static_cast<size_t>(nch) * n_rows_raw);
+    }
 }
 
 // Fixed-threshold mode: every view's threshold is the same constant.
@@ -324,32 +379,54 @@ int launch_adaptive(const AdaptiveArgs &a, hipStream_t stream) {
     const unsigned g1 = static_cast<unsigned>((a.n_proj + 255) / 256);
     if (a.max_groups < 0) return CTBB_ERR_SHAPE;
     const unsigned gsup = static_cast<unsigned>(a.max_groups > 0 && a.max_groups < a.n_proj ? a.max_groups : a.n_proj);
-    if (a.fixed_threshold > 0.0f) {
+    // A per-view threshold leaves most views unchanged (it is placed so that
+    // few of the view maxima exceed it), so out of place the pull is copied
+    // while its maxima are taken and only the changed views are visited again;
+    // a fixed threshold has no maxima to take and reads the pull once.
+    const bool aligned = (reinterpret_cast<uintptr_t>(a.raw) & 15u) == 0 && (reinterpret_cast<uintptr_t>(a.out) & 15u) == 0;
+    const bool fixed = a.fixed_threshold > 0.0f;
+    const bool copied = !a.hot_only && !fixed && aligned;
+    if (fixed) {
         if (!(a.fixed_threshold < 3.0e38f)) return CTBB_ERR_ARG;
         hipLaunchKernelGGL(af_const, dim3(g1), dim3(256), 0, stream, thr, a.n_proj, a.fixed_threshold);
-        // (the view maxima decide which views hot_only writes)
-        if (a.hot_only) hipLaunchKernelGGL(af_sup, dim3(gsup), dim3(256), 0, stream, a.raw, sup, frame, a.n_proj);
-    } else {
-        hipLaunchKernelGGL(af_sup, dim3(gsup), dim3(256), 0, stream, a.raw, sup, frame, a.n_proj);
-        hipLaunchKernelGGL(af_smooth, dim3(g1), dim3(256), 0, stream, sup, sm, a.n_proj, n_avg);
-        // the counting window (at most n_range values) in LDS when it takes <= 16 KB
-        const size_t win_bytes = static_cast<size_t>(n_range) * sizeof(float);
-        if (win_bytes <= 16384)
-            hipLaunchKernelGGL(af_thresh<true>, dim3(a.n_proj), dim3(64), win_bytes, stream, sm, thr, a.n_proj,
-                               n_range, a.n_proj_ffs, a.strength);
+    }
+    // (with a fixed threshold the view maxima decide which views hot_only writes)
+    if (copied)
+        hipLaunchKernelGGL(af_sup<true>, dim3(gsup), dim3(256), 0, stream, a.raw, sup, a.out, frame, a.n_proj);
+    else if (!fixed || a.hot_only)
+        hipLaunchKernelGGL(af_sup<false>, dim3(gsup), dim3(256), 0, stream, a.raw, sup, a.out, frame, a.n_proj);
+    if (!fixed) {
+        const size_t win = (kSmoothViews + static_cast<size_t>(n_avg)) * sizeof(float);
+        if (win > 65536) return CTBB_ERR_SHAPE;
+        hipLaunchKernelGGL(af_smooth, dim3(static_cast<unsigned>((a.n_proj + kSmoothViews - 1) / kSmoothViews)),
+                           dim3(kSmoothViews), win, stream, sup, sm, a.n_proj, n_avg);
+        if (n_range <= 64 * 16)
+            hipLaunchKernelGGL(af_thresh<16>, dim3(a.n_proj), dim3(64), 0, stream, sm, thr, a.n_proj, n_range,
+                               a.n_proj_ffs, a.strength);
+        else if (n_range <= 64 * 44)
+            hipLaunchKernelGGL(af_thresh<44>, dim3(a.n_proj), dim3(64), 0, stream, sm, thr, a.n_proj, n_range,
+                               a.n_proj_ffs, a.strength);
         else
-            hipLaunchKernelGGL(af_thresh<false>, dim3(a.n_proj), dim3(64), 0, stream, sm, thr, a.n_proj, n_range,
+            hipLaunchKernelGGL(af_thresh<0>, dim3(a.n_proj), dim3(64), 0, stream, sm, thr, a.n_proj, n_range,
                                a.n_proj_ffs, a.strength);
     }
-    const int bpv = (af_view_waves(a.n_rows_raw, a.nch) + 3) / 4;
+    // (a form that visits few views gives a workgroup up to 16 of a view's
+    // waves: most of its workgroups only find their view unchanged)
+    const bool few = a.hot_only || copied;
+    const int bpv = (af_view_waves(a.n_rows_raw, a.nch) + (few ? 15 : 3)) / (few ? 16 : 4);
     const unsigned long long grid = 8ull * static_cast<unsigned long long>((a.n_proj + 7) / 8) * bpv;
     if (grid > 0x7fffffffull) return CTBB_ERR_SHAPE;
+    unsigned char *hot = adaptive_hot_flags(a.work, a.n_proj);
+    const dim3 g(static_cast<unsigned>(grid));
     if (a.hot_only)
-        hipLaunchKernelGGL(af_apply_hot, dim3(static_cast<unsigned>(grid)), dim3(256), 0, stream, a.raw, sup, thr, a.out,
-                           adaptive_hot_flags(a.work, a.n_proj), a.n_proj, a.n_rows_raw, a.nch, bpv);
+        hipLaunchKernelGGL(af_apply<kHotFlagged>, g, dim3(256), 0, stream, a.raw, sup, thr, a.out, hot, a.n_proj,
+                           a.n_rows_raw, a.nch, bpv);
+    else if (copied)
+        hipLaunchKernelGGL(af_apply<kHotCopied>, g, dim3(256), 0, stream, a.raw, sup, thr, a.out, hot, a.n_proj,
+                           a.n_rows_raw, a.nch, bpv);
     else
-        hipLaunchKernelGGL(af_apply, dim3(static_cast<unsigned>(grid)), dim3(256), 0, stream, a.raw, thr, a.out,
-                           a.n_proj, a.n_rows_raw, a.nch, bpv);
+        hipLaunchKernelGGL(af_apply<kAllViews>, g, dim3(256), 0, stream, a.raw, sup, thr, a.out, hot, a.n_proj,
+                           a.n_rows_raw, a.nch, bpv);
     return hipGetLastError() == hipSuccess ? CTBB_OK : CTBB_ERR_HIP;
 }
 

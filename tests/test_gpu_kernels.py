@@ -103,3 +103,27 @@ def test_rebin_edges(ctx, tmp_path, ffs, channels, nrows, centre, reverse):
     got = host(out).reshape(want.shape)
     assert np.abs(got - want).max() <= 2e-5 + np.spacing(np.float32(mr.ri.n_proj_pull // mr.ri.n_ffs))
     cb.free_metadata(mr)
+
+
+@pytest.mark.parametrize("turn", [126, 2040, 2052, 5626, 5636])
+def test_adaptive_threshold_windows(ctx, tmp_path, turn):
+    """Per-view threshold bit for bit around the window sizes that change the
+    bisection's form (1024 and 2816 values) and for a window that does not
+    fill one wave, with view maxima that vary over the turn; out of place on
+    16-byte aligned buffers and on buffers one sample off."""
+    import oracle
+    mr = _mini(tmp_path, 4, 16, turn=turn)
+    n = int(mr.ri.n_proj_pull)
+    rng = np.random.default_rng(turn)
+    size = 1.0 + 0.8 * np.sin(np.arange(n) * (4 * np.pi / turn))
+    raw = (rng.random((n, 64)) * size[:, None]).astype(np.float32)
+    want, thr = oracle.adaptive_filter(mr, raw)
+    assert 0 < np.count_nonzero(want != raw) and np.unique(thr).size > 16
+    for off in (0, 1):
+        buf = dev(np.concatenate([np.zeros(off, np.float32), raw.ravel()]))
+        out = torch.zeros(raw.size + off, dtype=torch.float32, device="cuda")
+        torch.cuda.synchronize()
+        ctx.adaptive_filter_dev(mr, buf[off:], out[off:])
+        ctx.synchronize()
+        assert np.array_equal(host(out)[off:].reshape(n, 64), want.reshape(n, 64)), off
+    cb.free_metadata(mr)
