@@ -25,9 +25,13 @@
 // W(q) = 0 for |q| >= 1 contributes exactly nothing; since q varies by less
 // than 1% across a wavefront, chunks of 4 slices that no lane sees are
 // skipped on a wave-uniform vote (about 40% of the (slice, view) pairs are
-// seen at the C1 geometry), chunks with |q| < 0.6 in every lane take a path
-// with W = 1, and the cos^2 taper is evaluated only for slices where some
-// lane is in 0.6 <= |q| < 1.  View-table entries reach the
+// seen at the C1 geometry), and chunks with |q| < 0.6 in every lane take a
+// path with W = 1; elsewhere the weight is evaluated for every slice without
+// branches.  What binds is instruction issue (VALU 80% busy at 64 rows x
+// 512^2, 90% at 1024^2, 4 waves per SIMD); a block of 512^2 x 1728 views takes
+// 5.55 ms (5.76 with a vote and a branch around the weight of each slice and
+// two instructions per LDS address), 1024^2 26.4 (27.9).  View-table entries
+// reach the
 // workgroup through a small LDS ring refilled every 64 views.
 //
 // Workgroups are remapped so the tiles running on one XCD are spatially
@@ -43,23 +47,23 @@ namespace ctbb {
 
 namespace {
 
-// Taper part of the Stierstorfer weight W(q), Q = 0.6 (reference
-// include/backproject.cuh:33-46), for 0.6 <= |q| < 1:
-//   cos^2(pi'/2 t) = sin^2(pi'/2 (1 - t) + (pi - pi')/2),  t = (|q| - 0.6) / 0.4,
-// pi' = 3.1415368979f.  The sine is an odd degree-7 polynomial v + v^3 P(v^2)
-// fitted for relative error (1.2e-6 on [0, pi/2]), so the weight stays
+// Stierstorfer weight W(q), Q = 0.6 (reference include/backproject.cuh:33-46),
+// for |q| < 1: W = cos^2(pi'/2 t), t = (|q| - 0.6) / 0.4 clamped to [0, 1],
+// pi' = 3.1415368979f.  The cosine is an even degree-8 polynomial of t (error
+// 5e-8): exactly 1 for |q| <= 0.6 and 2.8e-5 at t = 1, so the weight stays
 // strictly positive up to |q| -> 1 (7.8e-10 there, as the reference's): a
 // view that is the only one to see a voxel at an angle still gets
-// s_t / h_t = its sample.  Error of W < 2.5e-6 of W.
-__device__ __forceinline__ float stier_taper(float aq) {
-    const float u = __builtin_amdgcn_fmed3f(fmaf(aq, -2.5f, 2.5f), 0.0f, 1.0f);   // 1 - t
-    const float v = fmaf(u, 1.5707684f, 2.7877844e-05f);
-    const float v2 = v * v;
-    float p = -0.0001854245929280296f;
-    p = fmaf(p, v2, 0.008314281702041626f);
-    p = fmaf(p, v2, -0.16665853559970856f);
-    const float sn = fmaf(v * v2, p, v);
-    return sn * sn;
+// s_t / h_t = its sample.  Error of W < 2.1e-7.  (Evaluated for every slice
+// of a chunk that needs it, without a branch per slice.)
+__device__ __forceinline__ float stier_weight(float aq) {
+    const float t = __builtin_amdgcn_fmed3f(fmaf(aq, 2.5f, -1.5f), 0.0f, 1.0f);
+    const float t2 = t * t;
+    float p = 0.00085957017f;
+    p = fmaf(p, t2, -0.020811755f);
+    p = fmaf(p, t2, 0.25363523f);
+    p = fmaf(p, t2, -1.2336551f);
+    const float c = fmaf(p, t2, 1.0f);
+    return c * c;
 }
 
 __device__ __forceinline__ float bf16_to_f32(uint16_t h) {
@@ -130,6 +134,13 @@ template <int NZ, int CPT, int TPR, int ZS, bool kBf16, class Args>
 __device__ __forceinline__ void bp_tile(Args &a, int tile, int zblk, float2 *lds2) {
     constexpr int THREADS = 256 * ZS;
     const int tid = threadIdx.x;
+    // LDS byte address of the windows, and a pair at such an address
+    const unsigned lds_base = (unsigned)(uintptr_t)(__attribute__((address_space(3))) void *)lds2;
+    typedef float LdsPair __attribute__((ext_vector_type(2)));
+    auto lds_pair = [](unsigned at) {
+        const LdsPair v = *(const __attribute__((address_space(3))) LdsPair *)at;
+        return make_float2(v.x, v.y);
+    };
     const int tx = tile / a.tiles_y, ty = tile - tx * a.tiles_y;
     // Column of this thread in the 16x16 tile.  Each wave covers 4 x-rows of
     // 16; within it each group of 16 lanes (one LDS cycle of a 64-bit read)
@@ -364,8 +375,8 @@ __device__ __forceinline__ void bp_tile(Args &a, int tile, int zblk, float2 *lds
         // row coordinate (q + 1) hr = Ar z + Br, used directly where |q| < 0.6
         const float Ar = A * a.hr;
         const float Br = fmaf(B, a.hr, a.hr);
-        // LDS index of (row 0, channel c0) in this view's buffer
-        const unsigned colb = static_cast<unsigned>((t & 1) * n_stage) + ci;
+        // LDS byte address of (row 0, channel c0) in this view's buffer
+        const unsigned colb = lds_base + 8u * (static_cast<unsigned>((t & 1) * n_stage) + ci);
 
         // Slices in chunks of 4.  q is linear in z, so over a chunk it stays
         // within hw = 1.5 |A| of its value qm at the chunk centre: a chunk can
@@ -373,13 +384,13 @@ __device__ __forceinline__ void bp_tile(Args &a, int tile, int zblk, float2 *lds
         // |qm| < 0.6 - hw.  Both thresholds carry a margin of 1e-4, far above
         // the rounding of q, so a skipped chunk has |q| > 1 in every lane and
         // an interior chunk |q| < 0.6.  One wave vote skips chunks no lane
-        // sees; a second sends chunks interior for every lane (the common
-        // case) through a path with W = 1 and no clamping.  Elsewhere W is
-        // evaluated per slice, the taper only for slices where some lane has
-        // 0.6 <= |q| < 1 (a third, per-slice vote).  The 4 slices of a
-        // visible chunk then interpolate without branches (W = 0 for lanes
-        // that do not see a slice, row coordinate clamped into the window),
-        // so their LDS reads are in flight together.
+        // sees; a second sends chunks interior for every lane through a path
+        // with W = 1 and no clamping.  Elsewhere W is evaluated for every
+        // slice (a vote and a branch per slice to leave out the weight where
+        // no lane is in 0.6 <= |q| < 1 cost more than the weight).  The 4
+        // slices of a visible chunk then interpolate without branches (W = 0
+        // for lanes that do not see a slice, row coordinate clamped into the
+        // window), so their LDS reads are in flight together.
         const float hw = 1.5f * fabsf(A);
         const float t_vis = 1.0001f + hw;
         const float t_int = 0.5999f - hw;
@@ -399,29 +410,22 @@ __device__ __forceinline__ void bp_tile(Args &a, int tile, int zblk, float2 *lds
 #pragma unroll
                 for (int c = 0; c < 4; c++) {
                     const float q = fmaf(A, static_cast<float>(ZSTEP * zc + c), B);
-                    const float aq = fabsf(q);
-                    const bool vis = aq < 1.0f;
-                    const bool band = vis && aq >= 0.6f;
-                    float wc = vis ? 1.0f : 0.0f;
-                    if (__builtin_amdgcn_ballot_w64(band)) {
-                        const float tp = stier_taper(aq);
-                        wc = band ? tp : wc;
-                    }
-                    w[c] = wc;
+                    const float wq = stier_weight(fabsf(q));
+                    w[c] = fabsf(q) < 1.0f ? wq : 0.0f;
                     // row coordinate (q + 1) hr, in [0, n_rows - 1] where W != 0
                     rowf[c] = __builtin_amdgcn_fmed3f(fmaf(q, a.hr, a.hr), 0.0f, two_hr);
                 }
             }
             float2 e0[4], e1[4];
-            // the chunk's LDS reads (and, below, the next view's window
+            // the chunk's LDS reads (and, above, the next view's window
             // loads) are issued at raised wave priority, so waves start their
             // long-latency requests ahead of other waves' arithmetic
             __builtin_amdgcn_s_setprio(1);
 #pragma unroll
             for (int c = 0; c < 4; c++) {
-                const unsigned idx = colb + __umul24(static_cast<unsigned>(rowf[c]), static_cast<unsigned>(RS));
-                e0[c] = lds2[idx];
-                e1[c] = lds2[idx + RS];
+                const unsigned at = colb + __umul24(static_cast<unsigned>(rowf[c]), static_cast<unsigned>(8 * RS));
+                e0[c] = lds_pair(at);
+                e1[c] = lds_pair(at + 8 * RS);
             }
             // all 8 reads of the chunk are issued before the first is used
             __builtin_amdgcn_sched_barrier(0);
