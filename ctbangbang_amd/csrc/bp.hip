@@ -98,6 +98,18 @@ __device__ __forceinline__ float asin_small(float x) {
     return p * x;
 }
 
+// First angle of part `part` of `parts` (parts: the end).
+__device__ __forceinline__ int part_angle(int half, int parts, int part) { return half * part / parts; }
+
+// Whether a voxel column lies inside the acquisition field of view (explicit
+// rounding: every kernel that asks gets the same answer).
+template <class Args>
+__device__ __forceinline__ bool column_in_fov(Args &a, int xi, int yi) {
+    const float x = fmaf(a.xs, static_cast<float>(xi) - a.xc, a.x0);
+    const float y = fmaf(a.ys, static_cast<float>(yi) - a.yc, a.y0);
+    return sqrtf(fmaf(x, x, y * y)) < a.acq_half;
+}
+
 // NZ slices per thread; CPT staged channels per thread per view; TPR staging
 // threads per detector row (0: taken from the arguments at run time).  The
 // staged window covers rows_pad x W channels, rows_pad = 256 / TPR a power of
@@ -130,8 +142,12 @@ constexpr int ilog2(int v) { return v <= 1 ? 0 : 1 + ilog2(v >> 1); }
 // The workgroup leaves LDS free for reuse once every thread has returned.
 // Args: BpArgs, either a kernel argument or a job read through the scalar
 // cache (constant address space), so its fields stay in scalar registers.
+// part: the tile's views of one part of the block's angles (of a.parts), its
+// sums over them left in `out`: as they are, added to what `out` holds (add),
+// and in the last part of an image scaled and cut to the field of view (last).
 template <int NZ, int CPT, int TPR, int ZS, bool kBf16, class Args>
-__device__ __forceinline__ void bp_tile(Args &a, int tile, int zblk, float2 *lds2) {
+__device__ __forceinline__ void bp_tile(Args &a, int tile, int zblk, float2 *lds2, int part, float *out, bool add,
+                                        bool last) {
     constexpr int THREADS = 256 * ZS;
     const int tid = threadIdx.x;
     // LDS byte address of the windows, and a pair at such an address
@@ -267,8 +283,9 @@ __device__ __forceinline__ void bp_tile(Args &a, int tile, int zblk, float2 *lds
     // through an LDS ring of 128: chunk c (views 64c .. 64c + 63) is loaded
     // during view 64(c - 1), published by the next barrier and first read
     // 63 views later; its slot last held chunk c - 2.
-    const int n_views = a.half * a.n_ht;
-    const float4 *vtab = reinterpret_cast<const float4 *>(a.vtab);
+    const int i0 = part_angle(a.half, a.parts, part);
+    const int n_views = (part_angle(a.half, a.parts, part + 1) - i0) * a.n_ht;
+    const float4 *vtab = reinterpret_cast<const float4 *>(a.vtab) + i0 * a.n_ht;
     float4 *ring = reinterpret_cast<float4 *>(lds2 + 2 * n_stage);
     // Each entry's window base (the staged window's first channel for this
     // tile, the same in every lane) is computed once, by the thread that
@@ -451,7 +468,7 @@ __device__ __forceinline__ void bp_tile(Args &a, int tile, int zblk, float2 *lds
         }
     }
 
-    const bool in_fov = sqrtf(x * x + y * y) < a.acq_half;
+    const bool in_fov = column_in_fov(a, xi, yi);
     // slice bases in scalar registers (z0 is the same across a wave), the
     // column's 32-bit offset per lane
     const size_t nxy = static_cast<size_t>(a.nx) * a.ny;
@@ -459,8 +476,21 @@ __device__ __forceinline__ void bp_tile(Args &a, int tile, int zblk, float2 *lds
     const unsigned lane_off = static_cast<unsigned>(xi * a.ny + yi);
 #pragma unroll
     for (int z = 0; z < NZ; z++) {
-        float *os = a.out + static_cast<size_t>(zw + ZSTEP * (z & ~3) + (z & 3)) * nxy;
-        os[lane_off] = in_fov ? s[z] * a.out_scale : 0.0f;
+        float *os = out + static_cast<size_t>(zw + ZSTEP * (z & ~3) + (z & 3)) * nxy;
+        float v = add ? os[lane_off] + s[z] : s[z];
+        if (last) v = in_fov ? v * a.out_scale : 0.0f;
+        os[lane_off] = v;
+    }
+}
+
+// All parts of a tile, one after the other, into the image.
+template <int NZ, int CPT, int TPR, int ZS, bool kBf16, class Args>
+__device__ __forceinline__ void bp_tile_parts(Args &a, int tile, int zblk, float2 *lds2, int first, int end,
+                                              float *out) {
+    for (int part = first; part < end; part++) {
+        if (part != first) __syncthreads();                     // LDS reuse by the next part
+        bp_tile<NZ, CPT, TPR, ZS, kBf16>(a, tile, zblk, lds2, part, out, part != first,
+                                         first == 0 && end == a.parts && part == end - 1);
     }
 }
 
@@ -469,16 +499,55 @@ __device__ __forceinline__ void bp_tile(Args &a, int tile, int zblk, float2 *lds
 // tiles b, b + gridDim.x, ... — all of them placed at launch, so kernels
 // started beside the backprojection cannot take the registers a later
 // workgroup of it would need.  XCD-aware remap: hardware dispatches workgroup
-// b to XCD b % 8, and item i maps to tile (i % 8) per + i / 8, so each XCD
-// works through a contiguous band of tiles.
+// b to XCD b % 8, and item i maps to tile (i % 8) per + (i / 8) % per, so each
+// XCD works through a contiguous band of tiles (and through one part of the
+// angles after the other).
+// With a.partial an item is one part of a tile, its sums left in the part's
+// partial image; bp_sum_kernel then adds the parts in order, the sums of the
+// form without partial images.
 template <int NZ, int CPT, int TPR, int ZS, bool kBf16>
 __device__ __forceinline__ void bp_block_body(const BpArgs &a, float2 *lds2) {
     const int per = (a.n_tiles & 7) == 0 ? a.n_tiles >> 3 : 0;
-    for (int item = blockIdx.x; item < a.n_tiles; item += gridDim.x) {
-        const int tile = per ? (item & 7) * per + (item >> 3) : item;
+    const int items = a.partial ? a.n_tiles * a.parts : a.n_tiles;
+    for (int item = blockIdx.x; item < items; item += gridDim.x) {
+        int tile, part;
+        if (per) {
+            part = (item >> 3) / per;
+            tile = (item & 7) * per + ((item >> 3) - part * per);
+        } else {
+            part = item / a.n_tiles;
+            tile = item - part * a.n_tiles;
+        }
         if (item != static_cast<int>(blockIdx.x)) __syncthreads();   // LDS reuse by the next tile
-        bp_tile<NZ, CPT, TPR, ZS, kBf16>(a, tile, blockIdx.y, lds2);
+        const size_t img = 32 * static_cast<size_t>(a.nx) * a.ny;
+        const bool split = a.partial != nullptr;
+        bp_tile_parts<NZ, CPT, TPR, ZS, kBf16>(a, tile, blockIdx.y, lds2, part, split ? part + 1 : a.parts,
+                                               split ? a.partial + part * img : a.out);
     }
+}
+
+// Image of a block from its partial images: the parts added in order, scaled,
+// cut to the field of view.  4 voxels of a slice per thread (ny is a multiple
+// of 16), bound by HBM.
+__global__ __launch_bounds__(256) void bp_sum_kernel(BpArgs a) {
+    const size_t img = 32 * static_cast<size_t>(a.nx) * a.ny;
+    const size_t i = (static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x) * 4;
+    if (i >= img) return;
+    float4 v = *reinterpret_cast<const float4 *>(a.partial + i);
+    for (int p = 1; p < a.parts; p++) {
+        const float4 q = *reinterpret_cast<const float4 *>(a.partial + p * img + i);
+        v.x += q.x;
+        v.y += q.y;
+        v.z += q.z;
+        v.w += q.w;
+    }
+    const unsigned col = static_cast<unsigned>(i % (static_cast<size_t>(a.nx) * a.ny));
+    const int xi = static_cast<int>(col) / a.ny, yi = static_cast<int>(col) - xi * a.ny;
+    float *o = a.out + i;               // (any float alignment: the caller's image)
+    o[0] = column_in_fov(a, xi, yi) ? v.x * a.out_scale : 0.0f;
+    o[1] = column_in_fov(a, xi, yi + 1) ? v.y * a.out_scale : 0.0f;
+    o[2] = column_in_fov(a, xi, yi + 2) ? v.z * a.out_scale : 0.0f;
+    o[3] = column_in_fov(a, xi, yi + 3) ? v.w * a.out_scale : 0.0f;
 }
 
 // Two z-groups (512 threads, 4 waves per SIMD).  VGPR limits (the
@@ -547,7 +616,7 @@ __device__ __forceinline__ void bp_persistent_tile(const BpQueues &Q, const int 
     const __attribute__((address_space(4))) BpArgs &a =
         *(const __attribute__((address_space(4))) BpArgs *)(Q.jobs + lo);
     const int tile = (q * a.n_tiles) / 8 + (item - __builtin_amdgcn_readfirstlane(pre[lo]));
-    bp_tile<NZ, CPT, TPR, ZS, kBf16>(a, tile, 0, lds2);
+    bp_tile_parts<NZ, CPT, TPR, ZS, kBf16>(a, tile, 0, lds2, 0, a.parts, a.out);
 }
 
 template <int NZ, int CPT, int TPR, int ZS, bool kBf16>
@@ -650,7 +719,8 @@ int launch_c(const BpArgs &a, hipStream_t stream, bool beside) {
     // (C1 block: 5.82 against 5.87 ms for the resident grid, medians of 15
     // launches).
     const int ny = 32 / (NZ * ZS);
-    long gx = a.n_tiles;
+    const long items = a.partial ? static_cast<long>(a.n_tiles) * a.parts : a.n_tiles;
+    long gx = items;
     if (beside) {
         int dev = 0, n_cu = 0, per_cu = 0;
         if (hipGetDevice(&dev) != hipSuccess ||
@@ -659,12 +729,15 @@ int launch_c(const BpArgs &a, hipStream_t stream, bool beside) {
             return CTBB_ERR_HIP;
         gx = std::max(1, per_cu) * static_cast<long>(std::max(1, n_cu)) / ny;
         if ((a.n_tiles & 7) == 0) gx = std::max<long>(8, gx / 8 * 8);
-        gx = std::min<long>(gx, a.n_tiles);
+        gx = std::min<long>(gx, items);
     }
     dim3 grid(static_cast<unsigned>(gx), ny);
     void *args[] = {const_cast<BpArgs *>(&a)};
-    return hipLaunchKernel(kf, grid, dim3(256 * ZS), args, lds_bytes, stream) == hipSuccess ? CTBB_OK
-                                                                                           : CTBB_ERR_HIP;
+    if (hipLaunchKernel(kf, grid, dim3(256 * ZS), args, lds_bytes, stream) != hipSuccess) return CTBB_ERR_HIP;
+    if (!a.partial) return CTBB_OK;
+    const size_t img4 = 8 * static_cast<size_t>(a.nx) * a.ny;
+    hipLaunchKernelGGL(bp_sum_kernel, dim3(static_cast<unsigned>((img4 + 255) / 256)), dim3(256), 0, stream, a);
+    return hipGetLastError() == hipSuccess ? CTBB_OK : CTBB_ERR_HIP;
 }
 
 template <int NZ, int CPT, int TPR, int ZS>
@@ -781,9 +854,40 @@ int with_variant(int id, Op op) {
 
 }  // namespace
 
+// Parts the angles of a block are divided into.  With one part a block takes
+// as long as its rounds of tiles on the resident workgroups (two per CU): a
+// 256^2 image has 256 tiles, half a round, and a 400^2 image 625, a round and
+// a bit.  Parts multiply the workgroups and divide their work.  Modelled time
+// in rounds: a last round that puts at most one workgroup on a CU counts 0.65
+// (alone on its CU a workgroup runs faster, not twice as fast), each part
+// costs 1% (prologue, partial image and its sum).  More parts than one only
+// where they save 5%, with at least 32 angles each.  A function of the shape
+// and the device only: every way to backproject a block sums in this order.
+// One block of 64 rows x 1728 views, one part against the chosen number, ms:
+// 144^2 3.5 / 1.2, 208^2 4.4 / 3.0, 288^2 9.0 / 6.0, 400^2 5.5 / 3.8, 448^2
+// 5.7 / 4.3, 640^2 9.3 / 7.7 (512^2 keeps one); 16 rows x 3456 views, 256^2
+// 3.24 / 2.00.
+int backproject_parts(int n_tiles, int half, int n_cu) {
+    const long slots = 2l * std::max(n_cu, 1);
+    int best = 1;
+    double best_cost = 0.0;
+    for (int parts = 1; parts <= 16 && (parts == 1 || half >= 32 * parts); parts++) {
+        const long items = static_cast<long>(n_tiles) * parts, rest = items % slots;
+        const double rounds = static_cast<double>(items / slots) + (rest == 0 ? 0.0 : rest <= slots / 2 ? 0.65 : 1.0);
+        const double cost = rounds / parts * (1.0 + 0.01 * parts);
+        if (parts == 1) best_cost = cost * 0.95;
+        else if (cost < best_cost) {
+            best = parts;
+            best_cost = cost;
+        }
+    }
+    return best;
+}
+
 int backproject_variant(BpArgs &a) {
     if (a.nx % 16 || a.ny % 16 || a.nx <= 0 || a.ny <= 0) return -CTBB_ERR_SHAPE;
     if (a.n_rows < 2 || a.half <= 0 || a.n_ht <= 0) return -CTBB_ERR_SHAPE;
+    if (a.parts < 1 || a.parts > a.half || static_cast<long>(a.half) * (a.parts + 1) > 0x7fffffffL) return -CTBB_ERR_ARG;
     if (a.n_tiles != (a.nx / 16) * (a.ny / 16) || a.tiles_y != a.ny / 16) return -CTBB_ERR_ARG;
     if (a.nz != 16 && a.nz != 32) return -CTBB_ERR_ARG;
     const int zs = a.nz == 16 ? 2 : 1;

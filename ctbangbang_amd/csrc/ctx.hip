@@ -85,6 +85,7 @@ struct ctbb_ctx {
     ctbb::BpView *noalloc_vtab = nullptr;   // this device's `scratch` array
     DevBuf raw_in, raw_af, rebin_tmp, image_block, image_stack, af_work;
     DevBuf vtab, maps, taps, spec, fin_tab;
+    DevBuf bp_partial;         // partial images of a backprojection in parts
     int spec_len = 0;          // transform length of `spec` (3072 or 4096; 0: none)
     // 1 once a rebin met a non-finite output sample (read and cleared by
     // ctbb_ctx_synchronize)
@@ -341,7 +342,7 @@ int do_filter(ctbb_ctx *ctx, const float *d_taps, int n, size_t rows, const floa
     return st;
 }
 
-int fill_bp_args(const recon_metadata *mr, BpArgs &a) {
+int fill_bp_args(const ctbb_ctx *ctx, const recon_metadata *mr, BpArgs &a) {
     const ct_geom &cg = mr->cg;
     const recon_params &rp = mr->rp;
     if (rp.nx % 16 || rp.ny % 16 || rp.nx == 0 || rp.ny == 0) return CTBB_ERR_SHAPE;
@@ -381,20 +382,28 @@ int fill_bp_args(const recon_metadata *mr, BpArgs &a) {
     const double hy = 0.5 * rp.recon_fov + std::fabs(static_cast<double>(rp.y_origin));
     a.asin_small_only = std::sqrt(hx * hx + hy * hy) <= 0.449 * cg.r_f ? 1 : 0;
     a.out_scale = static_cast<float>(2.0 * static_cast<double>(kPiBp) / cg.n_proj_turn);
+    a.parts = backproject_parts(a.n_tiles, a.half, ctx->prep_groups / 2);
     return CTBB_OK;
 }
 
 int do_backproject(ctbb_ctx *ctx, const recon_metadata *mr, const void *d_rebin, const BpView *d_vtab,
-                   float *d_out, hipStream_t on = nullptr, bool timed = true, bool beside = false) {
+                   float *d_out, hipStream_t on = nullptr, bool timed = true, bool beside = false, bool alloc = true) {
     if (!on) on = ctx->stream;
     BpArgs a{};
-    int st = fill_bp_args(mr, a);
+    int st = fill_bp_args(ctx, mr, a);
     if (st) return st;
     a.nz = ctx->opt.bp_tile == 32 ? 32 : 16;
     if (ctx->opt.proj_dtype == CTBB_PROJ_BF16) a.rebin_bf16 = static_cast<const uint16_t *>(d_rebin);
     else a.rebin = static_cast<const float *>(d_rebin);
     a.vtab = d_vtab;
     a.out = d_out;
+    // partial images (one set: backprojections of a context follow each other,
+    // on its compute stream or on stream_bp, which wait for one another)
+    if (a.parts > 1 && alloc) {
+        st = ctx->bp_partial.ensure(32 * static_cast<size_t>(a.nx) * a.ny * a.parts * sizeof(float));
+        if (st) return st;
+        a.partial = ctx->bp_partial.as<float>();
+    }
     if (!timed) return launch_backproject(a, on, beside);
     EventPair e = ctx->begin("backproject", on);
     st = launch_backproject(a, on, beside);
@@ -651,7 +660,7 @@ int ensure_pipeline(ctbb_ctx *c, size_t rebin_bytes) {
 // call per scan: 1.19 against 1.30 s with the threshold at 4).
 bool bp_many_rounds(ctbb_ctx *c, const recon_metadata *mr) {
     BpArgs a{};
-    if (fill_bp_args(mr, a)) return false;
+    if (fill_bp_args(c, mr, a)) return false;
     a.nz = c->opt.bp_tile == 32 ? 32 : 16;
     if (c->opt.proj_dtype == CTBB_PROJ_BF16) a.rebin_bf16 = reinterpret_cast<const uint16_t *>(16);
     else a.rebin = reinterpret_cast<const float *>(16);      // placeholders for the variant choice
@@ -753,7 +762,7 @@ void ctbb_ctx_destroy(ctbb_ctx *c) {
     if (c->stream_bp) (void)hipStreamSynchronize(c->stream_bp);
     if (c->stream_head) (void)hipStreamSynchronize(c->stream_head);
     for (DevBuf *b : {&c->raw_in, &c->raw_af, &c->rebin_tmp, &c->image_block, &c->image_stack, &c->af_work,
-                      &c->vtab, &c->maps, &c->taps, &c->spec, &c->fin_tab, &c->pull[0], &c->pull[1],
+                      &c->vtab, &c->bp_partial, &c->maps, &c->taps, &c->spec, &c->fin_tab, &c->pull[0], &c->pull[1],
                       &c->image_stack2, &c->nonfinite, &c->head_af, &c->head_work, &c->head_rebin, &c->head_pad})
         b->release();
     for (DevBuf &b : c->filt) b.release();
@@ -906,7 +915,7 @@ int ctbb_backproject_dev_noalloc(ctbb_ctx *c, const struct recon_metadata *mr, c
     if (hipSetDevice(c->device) != hipSuccess) return CTBB_ERR_HIP;
     st = launch_view_table(c->noalloc_vtab, j.tube_start, j.half, j.n_ht, j.n_proj_turn, j.z_rot, c->stream);
     if (st) return st;
-    return do_backproject(c, mr, d_rebin, c->noalloc_vtab, d_image_block, c->stream, false);
+    return do_backproject(c, mr, d_rebin, c->noalloc_vtab, d_image_block, c->stream, false, false, /*alloc:*/ false);
 }
 
 // Backprojection autotuner: bp_tile 16 (two z-groups) or 32 (one group).
@@ -1346,7 +1355,7 @@ int batch_persistent(ctbb_ctx *c, int n_scans, recon_metadata *const *mrs, const
         }
         bs.slot_elems = (bs.slot_elems + 63) & ~static_cast<size_t>(63);      // 256-byte aligned slots
         bs.img_elems = static_cast<size_t>(m->ri.n_slices_recon) * m->rp.nx * m->rp.ny;
-        int st = fill_bp_args(m, bs.tmpl);
+        int st = fill_bp_args(c, m, bs.tmpl);
         if (st) return st;
         bs.tmpl.nz = c->opt.bp_tile == 32 ? 32 : 16;
         if (c->opt.proj_dtype == CTBB_PROJ_BF16) bs.tmpl.rebin_bf16 = reinterpret_cast<const uint16_t *>(16);

@@ -30,7 +30,12 @@ struct BpArgs {
     float inv_ds, two_cc, inv_rf, rf2, k_asin, coll, tanc, neg_td, hr;
     float half_w;              // footprint half width of a 16x16 tile, channels
     float acq_half, out_scale;
+    int parts;                 // the angles are summed in this many parts (backproject_parts)
+    float *partial;            // parts > 1: [parts][32][nx][ny], 16-byte aligned; each part in workgroups of its own
+                               // (null: one workgroup takes a tile's parts one after the other, same sums)
 };
+// Parts for a block of n_tiles tiles and `half` angles on n_cu compute units.
+int backproject_parts(int n_tiles, int half, int n_cu);
 // beside: the caller schedules other kernels to run beside this launch
 // (then the grid is only the resident workgroups, which stride over the
 // tiles; otherwise one workgroup per tile).
