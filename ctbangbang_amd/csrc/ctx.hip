@@ -426,22 +426,28 @@ int finalize_table(const recon_metadata *mr, std::vector<int> &src, std::vector<
     double tdd = mr->table_positions[1000] - mr->table_positions[0];
     int table_direction = tdd == 0.0 ? 1 : static_cast<int>(std::fabs(tdd) / tdd);
     const int nf = ctbb_n_slices_final(mr);
-    std::vector<float> raw_loc(n_raw), wt(n_raw);
-    for (int i = 0; i < n_raw; i++) raw_loc[i] = ri.recon_start_pos + recon_direction * i * rp.coll_slicewidth;
+    // Only raw slices within one thickness of a final slice have weight; the
+    // window has two slices of margin either side for the rounding of the
+    // positions (the others' zero weights change neither sums nor lists).
+    const int reach = static_cast<int>(std::fmin(std::ceil(rp.slice_thickness / rp.coll_slicewidth), 1.0e6f)) + 2;
     std::vector<std::vector<std::pair<int, float>>> lists(nf);
     int mt = 1;
     for (int k = 0; k < nf; k++) {
         const float loc = rp.start_pos + recon_direction * k * rp.slice_thickness;
+        const double at = static_cast<double>(loc - ri.recon_start_pos) * recon_direction / rp.coll_slicewidth;
+        const int mid = static_cast<int>(std::fmin(std::fmax(at, 0.0), n_raw - 1.0));
+        const int i0 = std::max(0, mid - reach), i1 = std::min(n_raw, mid + reach + 1);
         float sum = 0.0f;
-        for (int i = 0; i < n_raw; i++) {
-            wt[i] = std::fmax(0.0f, 1.0f - std::fabs(raw_loc[i] - loc) / rp.slice_thickness);
-            sum += wt[i];
+        for (int i = i0; i < i1; i++) {
+            const float raw_loc = ri.recon_start_pos + recon_direction * i * rp.coll_slicewidth;
+            const float wt = std::fmax(0.0f, 1.0f - std::fabs(raw_loc - loc) / rp.slice_thickness);
+            sum += wt;
+            if (wt != 0.0f) lists[k].push_back({i, wt});
         }
-        for (int i = 0; i < n_raw; i++) {
-            if (wt[i] == 0.0f) continue;
-            const int b = i / nb, z = i % nb;
-            const int s = recon_direction != table_direction ? b * nb + (nb - 1 - z) : i;
-            lists[k].push_back({s, wt[i] / sum});
+        for (auto &t : lists[k]) {
+            const int b = t.first / nb, z = t.first % nb;
+            if (recon_direction != table_direction) t.first = b * nb + (nb - 1 - z);
+            t.second /= sum;
         }
         if (static_cast<int>(lists[k].size()) > mt) mt = static_cast<int>(lists[k].size());
     }

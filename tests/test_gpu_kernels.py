@@ -166,3 +166,32 @@ def test_backproject_parts(ctx, tmp_path, nx, ny):
         err = np.abs(g[:, cx, cy] - want)
         assert np.count_nonzero(err > 2e-4 * np.abs(want).max()) <= 1e-3 * err.size
     cb.free_metadata(mr)
+
+
+@pytest.mark.parametrize("nx,ny,thickness,offset", [(32, 32, 2.4, 0), (16, 20, 0.7, 0), (15, 7, 9.6, 0), (32, 16, 8.4, 1),
+                                                    (48, 32, 19.2, 0)])
+def test_finalize_edges(ctx, tmp_path, nx, ny, thickness, offset):
+    """Thickening bit for bit with tap lists of one to more than two batches,
+    slice sizes that are no multiple of four and a stack one sample off
+    16-byte alignment, in both table directions."""
+    import oracle
+    from ctbangbang_amd import scans
+    scans.mini_install(str(tmp_path))
+    for table_dir in ("out", "in"):
+        tok = scans.mini_tokens("none", nrows=8, rotations=30, table_dir=table_dir)
+        tok.update(Nx=nx, Ny=ny, SliceThickness=thickness, NSlices=3, EndPos=tok["StartPos"] + 2 * thickness)
+        prm = str(tmp_path / "f.prm")
+        cb.write_prm(prm, tok)
+        mr = cb.metadata_from_prm(prm, install_dir=str(tmp_path))
+        s = cb.block_sizes(mr)
+        img = np.random.default_rng(nx + ny).random(s.image_stack).astype(np.float32) * 0.04
+        for mu in (0.0, 0.02):
+            ctx.set_options(mu_water=mu)
+            buf = dev(np.concatenate([np.zeros(offset, np.float32), img]))
+            out = torch.empty(s.final_stack + offset, dtype=torch.float32, device="cuda")
+            ctx.finalize_dev(mr, buf[offset:], out[offset:])
+            ctx.synchronize()
+            got = host(out)[offset:].reshape(-1, nx, ny)
+            assert np.array_equal(got, oracle.finalize(mr, img, mu, double=False))
+        cb.free_metadata(mr)
+    ctx.set_options(mu_water=0.0)
