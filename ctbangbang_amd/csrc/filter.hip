@@ -14,11 +14,12 @@
 //           operands: X*T ~= Xh*Th + Xh*Tl + Xl*Th, FP32 accumulation
 //   F16X3   the same with float16 splits; taps are pre-scaled by 2^10 (and
 //           the result by 2^-10) to keep the low parts out of the subnormals
-//   FFT32   FP32 4096-point FFT convolution (the form of the reference's CPU
-//           path), for n <= 2048; wider rows fall back to F32
-// Toeplitz tiles are 64 (F32) or 256 (split forms) rows x 64 columns; they
-// require n % 64 == 0 (1472 and 1344 for the 736- and 672-channel scanners);
-// other widths use a VALU kernel.
+//   FFT32   FP32 FFT convolution of 3072 or 4096 points (the form of the
+//           reference's CPU path), for n <= 2048; wider rows fall back to F32
+// Toeplitz tiles are 64 rows x 64 columns (F32) or 128 x 192 (split forms).  The
+// split forms require n % 64 == 0 (1472 and 1344 for the 736- and 672-channel
+// scanners); other widths take the F32 product, on the vector ALUs where
+// n % 4 != 0.
 #include <hip/hip_fp16.h>
 #include <hip/hip_runtime.h>
 
@@ -32,6 +33,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef short i16x4 __attribute__((ext_vector_type(4)));
 
 constexpr int BM = 64, BN = 64, BK = 32;
+constexpr int TAP_MARGIN = 64;     // >= BN - 4 columns, >= BK - 4 samples past the row
 constexpr int A_STRIDE = BK + 4;   // 36 floats: 16-byte aligned rows
 
 __device__ __forceinline__ uint16_t f32_to_bf16_rne(float f) {
@@ -40,12 +42,18 @@ __device__ __forceinline__ uint16_t f32_to_bf16_rne(float f) {
     return static_cast<uint16_t>(u >> 16);
 }
 
-// FP32 Toeplitz product on v_mfma_f32_16x16x4_f32.
+// FP32 Toeplitz product on v_mfma_f32_16x16x4_f32, n % 4 == 0 (samples past the
+// row are zeros, columns past it are not stored).  One chain of sums in the order
+// of the samples: a row's smooth part cancels from the far taps to the near ones,
+// where chains over parts of the row keep the parts' large sums and their
+// rounding (4x the largest error).  Matrix-core bound, 118 to
+// 125 of the 153 TFLOP/s that a large FP32 matrix product reaches.
+template <bool kEnd>
 __global__ __launch_bounds__(256) void toeplitz_f32_kernel(FilterArgs a) {
     extern __shared__ float smem[];
     const int n = a.n;
-    float *As = smem;                          // [BM][A_STRIDE]
-    float *Tf = smem + BM * A_STRIDE;          // [2n] taps
+    float *Tf = smem + 2 * BM * A_STRIDE;      // [2n] taps; kEnd: between margins of zeros
+    constexpr int kMargin = kEnd ? TAP_MARGIN : 0;
 
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = tid >> 6;
@@ -53,7 +61,8 @@ __global__ __launch_bounds__(256) void toeplitz_f32_kernel(FilterArgs a) {
     const size_t m0 = static_cast<size_t>(blockIdx.y) * BM;
     const int n0 = blockIdx.x * BN;
 
-    for (int j = tid; j < 2 * n; j += 256) Tf[j] = a.taps[j];
+    for (int j = tid; j < 2 * n + 2 * kMargin; j += 256)
+        Tf[j] = !kEnd || (j >= kMargin && j < 2 * n + kMargin) ? a.taps[j - kMargin] : 0.0f;
 
     f32x4 acc[2][2];
 #pragma unroll
@@ -66,25 +75,23 @@ __global__ __launch_bounds__(256) void toeplitz_f32_kernel(FilterArgs a) {
     const size_t gm = m0 + arow;
     const bool row_ok = gm < a.rows;
     const float *xrow = a.in + gm * n + aseg;
-    float4 x0 = make_float4(0.f, 0.f, 0.f, 0.f), x1 = x0;
-    if (row_ok) {
-        x0 = reinterpret_cast<const float4 *>(xrow)[0];
-        x1 = reinterpret_cast<const float4 *>(xrow)[1];
-    }
+    f32x4 x0 = f32x4{0.f, 0.f, 0.f, 0.f}, x1 = x0;
+    auto load = [&](int k0) {
+        if (kEnd) x0 = x1 = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (row_ok && (!kEnd || k0 + aseg < n)) x0 = *reinterpret_cast<const f32x4 *>(xrow + k0);
+        if (row_ok && (!kEnd || k0 + aseg + 4 < n)) x1 = *reinterpret_cast<const f32x4 *>(xrow + k0 + 4);
+    };
+    load(0);
 
     for (int k0 = 0; k0 < n; k0 += BK) {
-        __syncthreads();
-        {
-            float4 *dst = reinterpret_cast<float4 *>(As + arow * A_STRIDE + aseg);
-            dst[0] = x0;
-            dst[1] = x1;
-        }
+        // two chunks in LDS in turn: one barrier per chunk
+        float *As = smem + (k0 & BK) * (BM * A_STRIDE / BK);
+        f32x4 *dst = reinterpret_cast<f32x4 *>(As + arow * A_STRIDE + aseg);
+        dst[0] = x0;
+        dst[1] = x1;
         __syncthreads();
         // prefetch the next K chunk of this thread's row while the MFMAs run
-        if (k0 + BK < n && row_ok) {
-            x0 = reinterpret_cast<const float4 *>(xrow + k0 + BK)[0];
-            x1 = reinterpret_cast<const float4 *>(xrow + k0 + BK)[1];
-        }
+        if (k0 + BK < n) load(k0 + BK);
 #pragma unroll
         for (int kk = 0; kk < BK; kk += 4) {
             float af[2], bfv[2];
@@ -93,7 +100,7 @@ __global__ __launch_bounds__(256) void toeplitz_f32_kernel(FilterArgs a) {
 #pragma unroll
             for (int ct = 0; ct < 2; ct++) {
                 const int col = n0 + wc * 32 + ct * 16 + lr;
-                bfv[ct] = Tf[n + col - (k0 + kk + lk)];
+                bfv[ct] = Tf[kMargin + n + col - (k0 + kk + lk)];
             }
 #pragma unroll
             for (int rt = 0; rt < 2; rt++)
@@ -112,7 +119,7 @@ __global__ __launch_bounds__(256) void toeplitz_f32_kernel(FilterArgs a) {
             for (int e = 0; e < 4; e++) {
                 const size_t om = m0 + wr * 32 + rt * 16 + 4 * lk + e;
                 const int col = n0 + wc * 32 + ct * 16 + lr;
-                if (om < a.rows) {
+                if (om < a.rows && (!kEnd || col < n)) {
                     const float y = acc[rt][ct][e];
                     if (a.out_bf16)
                         reinterpret_cast<uint16_t *>(a.out)[om * n + col] = f32_to_bf16_rne(y);
@@ -126,30 +133,42 @@ __global__ __launch_bounds__(256) void toeplitz_f32_kernel(FilterArgs a) {
 // (MODE BF16X3) or float16 (MODE F16X3, taps scaled by 2^10 to keep the low
 // parts out of the subnormals), accumulated in FP32 as Xl*Th + Xh*Tl + Xh*Th
 // on gfx950's v_mfma_f32_32x32x16_{bf16,f16} (measured on MI355X at about
-// 1.7x the rate of the 16x16x32 forms).  Workgroup = 256 rows x 64 columns;
-// each wave owns 64 rows x 64 columns as 2 x 2 tiles of 32 x 32.
+// 1.7x the rate of the 16x16x32 forms).  Workgroup = 128 rows x 32 CT columns;
+// each wave owns 32 rows as CT = 6 tiles of 32 x 32, the three products of a
+// k-step one after the other over the tiles, so that a tile's dependent MFMAs
+// are six apart.
 // The A operand goes straight from global memory into MFMA fragments: K is
 // reduced in chunks of 32, and within a chunk lane l (half h = l / 32) holds
 // k = 16 h + 8 s + e, e = 0..7, for k-step s, so its two A fragments are the
 // 16 consecutive samples of its row (four float4 loads), split into hi/lo
-// in registers and used for both column tiles; the next chunk's loads are
+// in registers once for all column tiles; the next chunk's loads are
 // issued before the current chunk's MFMAs.  Only the reversed taps live in
 // LDS (four copies shifted by 0..3 so that every B fragment, 8 consecutive
 // reversed taps, is two 8-byte reads), written once, so the K loop has no
-// barriers.  D layout (32 x 32): lane l, register r -> row 8 (r / 4) + 4 h +
-// r % 4, column l % 32.  Workgroups are ordered so that the n / 64 column
-// tiles of one 256-row band run on the same XCD and share its L2 copy of the
-// band.
-template <int MODE>
-__global__ __launch_bounds__(256) void toeplitz_split_kernel(FilterArgs a, int n_rt, int n_ct) {
-    constexpr int TM = 256, TN = 64, TK = 32;
+// barriers.  Columns past the row are not stored.  D layout (32 x 32): lane l,
+// register r -> row 8 (r / 4) + 4 h + r % 4, column l % 32.  Workgroups are
+// ordered so that the column tiles of a 128-row band run on the same XCD and
+// share its L2 copy of the band.
+// Bound by power: with random rows the clock falls to 1.5-1.9 GHz at 50% busy
+// matrix cores, so what counts is the other work per MFMA.  Per wave tile, rows
+// x columns, 119168 rows of 1344 in F16X3 / 30011 of 1472 in BF16X3: 64 x 64
+// (each split operand used for 2 column tiles) 1.93 / 0.65 ms, 64 x 128 1.68 /
+// 0.49, 32 x 192 1.49 / 0.47, 32 x 224 1.48 / 0.53, 32 x 256 1.73 / 0.55 (spills).
+constexpr int SPLIT_TM = 128;                                   // rows of a workgroup
+// taps of one shifted copy for 32 CT columns
+__host__ __device__ constexpr int split_taps(int n, int CT) { return n + 32 * CT + 8; }
+
+// CT column tiles per wave: 6, or fewer (launch_split).
+template <int MODE, int CT>
+__global__ __launch_bounds__(256, 2) void toeplitz_split_kernel(FilterArgs a, int n_rt, int n_ct) {
+    constexpr int TM = SPLIT_TM, TN = 32 * CT, TK = 32;
     typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
     typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
     typedef short i16x8 __attribute__((ext_vector_type(8)));
     typedef float f32x16 __attribute__((ext_vector_type(16)));
     extern __shared__ uint16_t sh[];
     const int n = a.n;
-    const int tw = n + TN + 8;                 // window length per copy
+    const int tw = split_taps(n, CT);             // taps per copy
     uint16_t *Gh = sh;                         // [4][tw]
     uint16_t *Gl = Gh + 4 * tw;                // [4][tw]
 
@@ -159,13 +178,11 @@ __global__ __launch_bounds__(256) void toeplitz_split_kernel(FilterArgs a, int n
     const int rt_i = tile / n_ct, ct_i = tile - rt_i * n_ct;
     const size_t m0 = static_cast<size_t>(rt_i) * TM;
     const int n0 = ct_i * TN;
-
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = tid >> 6;
     const int l32 = lane & 31, h = lane >> 5;
     const int jb = n - 1 - (n0 + TN - 1);      // first reversed-tap index this tile needs
     const float tscale = MODE == CTBB_FILTER_F16X3 ? 1024.0f : 1.0f;
-
     auto split = [&](float v, uint16_t &hi, uint16_t &lo) {
         if (MODE == CTBB_FILTER_BF16X3) {
             const __bf16 hb = static_cast<__bf16>(v);
@@ -177,56 +194,47 @@ __global__ __launch_bounds__(256) void toeplitz_split_kernel(FilterArgs a, int n
             lo = __builtin_bit_cast(uint16_t, static_cast<_Float16>(v - static_cast<float>(hf)));
         }
     };
-
-    for (int e = tid; e < 4 * tw; e += 256) {
-        const int sft = e / tw, m = e - sft * tw;
-        const int j = jb + m + sft;           // reversed-tap index
-        const float t = (j >= 0 && j < 2 * n) ? a.taps[2 * n - 1 - j] * tscale : 0.0f;
-        split(t, Gh[e], Gl[e]);
+    for (int m = tid; m < tw + 3; m += 256) {
+        const int j = jb + m;                 // reversed-tap index
+        uint16_t hi, lo;
+        split(j >= 0 && j < 2 * n ? a.taps[2 * n - 1 - j] * tscale : 0.0f, hi, lo);
+#pragma unroll
+        for (int s = 0; s < 4; s++)           // copy s holds it at m - s
+            if (m >= s && m - s < tw) {
+                Gh[s * tw + m - s] = hi;
+                Gl[s * tw + m - s] = lo;
+            }
     }
     __syncthreads();
-
-    f32x16 acc[2][2];
+    f32x16 acc[CT];
 #pragma unroll
-    for (int i = 0; i < 2; i++)
+    for (int j = 0; j < CT; j++)
 #pragma unroll
-        for (int j = 0; j < 2; j++)
-#pragma unroll
-            for (int r = 0; r < 16; r++) acc[i][j][r] = 0.0f;
-
-    // fragment rows of this lane; rows past the end read the last row (their
+        for (int r = 0; r < 16; r++) acc[j][r] = 0.0f;
+    // fragment row of this lane; rows past the end read the last row (their
     // results are not stored)
-    const float *xrow[2];
+    const size_t gm = m0 + wave * 32 + l32;
+    const float *xrow = a.in + (gm < a.rows ? gm : a.rows - 1) * n + 16 * h;
+    auto load = [&](float4 (&x)[4], int k0) {
 #pragma unroll
-    for (int rt = 0; rt < 2; rt++) {
-        size_t gm = m0 + wave * 64 + rt * 32 + l32;
-        if (gm >= a.rows) gm = a.rows - 1;
-        xrow[rt] = a.in + gm * n + 16 * h;
-    }
-    auto load = [&](float4 (&x)[2][4], int k0) {
-#pragma unroll
-        for (int rt = 0; rt < 2; rt++)
-#pragma unroll
-            for (int q = 0; q < 4; q++) x[rt][q] = *reinterpret_cast<const float4 *>(xrow[rt] + k0 + 4 * q);
+        for (int q = 0; q < 4; q++) x[q] = *reinterpret_cast<const float4 *>(xrow + k0 + 4 * q);
     };
-    auto mma = [&](const float4 (&x)[2][4], int k0) {
+    auto mma = [&](const float4 (&x)[4], int k0) {
 #pragma unroll
         for (int s = 0; s < 2; s++) {
-            i16x8 ah[2], al[2];
+            const float4 u = x[2 * s], w = x[2 * s + 1];
+            const float v[8] = {u.x, u.y, u.z, u.w, w.x, w.y, w.z, w.w};
+            i16x8 ah, al;
 #pragma unroll
-            for (int rt = 0; rt < 2; rt++) {
-                const float4 u = x[rt][2 * s], w = x[rt][2 * s + 1];
-                const float v[8] = {u.x, u.y, u.z, u.w, w.x, w.y, w.z, w.w};
-#pragma unroll
-                for (int e = 0; e < 8; e++) {
-                    uint16_t hi, lo;
-                    split(v[e], hi, lo);
-                    ah[rt][e] = static_cast<short>(hi);
-                    al[rt][e] = static_cast<short>(lo);
-                }
+            for (int e = 0; e < 8; e++) {
+                uint16_t hi, lo;
+                split(v[e], hi, lo);
+                ah[e] = static_cast<short>(hi);
+                al[e] = static_cast<short>(lo);
             }
+            i16x8 bh[CT], bl[CT];
 #pragma unroll
-            for (int ct = 0; ct < 2; ct++) {
+            for (int ct = 0; ct < CT; ct++) {
                 const int col = n0 + ct * 32 + l32;
                 const int mm = (n - 1 - col + k0 + 16 * h + 8 * s) - jb;
                 const int sft = mm & 3;
@@ -234,32 +242,25 @@ __global__ __launch_bounds__(256) void toeplitz_split_kernel(FilterArgs a, int n
                 const uint16_t *pl = Gl + sft * tw + (mm - sft);
                 const i16x4 h0 = *reinterpret_cast<const i16x4 *>(ph), h1 = *reinterpret_cast<const i16x4 *>(ph + 4);
                 const i16x4 l0 = *reinterpret_cast<const i16x4 *>(pl), l1 = *reinterpret_cast<const i16x4 *>(pl + 4);
-                const i16x8 bh = __builtin_shufflevector(h0, h1, 0, 1, 2, 3, 4, 5, 6, 7);
-                const i16x8 bl = __builtin_shufflevector(l0, l1, 0, 1, 2, 3, 4, 5, 6, 7);
-#pragma unroll
-                for (int rt = 0; rt < 2; rt++) {
-                    if (MODE == CTBB_FILTER_BF16X3) {
-                        acc[rt][ct] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                            __builtin_bit_cast(bf16x8, al[rt]), __builtin_bit_cast(bf16x8, bh), acc[rt][ct], 0, 0, 0);
-                        acc[rt][ct] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                            __builtin_bit_cast(bf16x8, ah[rt]), __builtin_bit_cast(bf16x8, bl), acc[rt][ct], 0, 0, 0);
-                        acc[rt][ct] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
-                            __builtin_bit_cast(bf16x8, ah[rt]), __builtin_bit_cast(bf16x8, bh), acc[rt][ct], 0, 0, 0);
-                    } else {
-                        acc[rt][ct] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
-                            __builtin_bit_cast(f16x8, al[rt]), __builtin_bit_cast(f16x8, bh), acc[rt][ct], 0, 0, 0);
-                        acc[rt][ct] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
-                            __builtin_bit_cast(f16x8, ah[rt]), __builtin_bit_cast(f16x8, bl), acc[rt][ct], 0, 0, 0);
-                        acc[rt][ct] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
-                            __builtin_bit_cast(f16x8, ah[rt]), __builtin_bit_cast(f16x8, bh), acc[rt][ct], 0, 0, 0);
-                    }
-                }
+                bh[ct] = __builtin_shufflevector(h0, h1, 0, 1, 2, 3, 4, 5, 6, 7);
+                bl[ct] = __builtin_shufflevector(l0, l1, 0, 1, 2, 3, 4, 5, 6, 7);
             }
+#pragma unroll
+            for (int p = 0; p < 3; p++)         // lo x hi, hi x lo, hi x hi
+#pragma unroll
+                for (int ct = 0; ct < CT; ct++) {
+                    const i16x8 A = p == 0 ? al : ah, B = p == 1 ? bl[ct] : bh[ct];
+                    if (MODE == CTBB_FILTER_BF16X3)
+                        acc[ct] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                            __builtin_bit_cast(bf16x8, A), __builtin_bit_cast(bf16x8, B), acc[ct], 0, 0, 0);
+                    else
+                        acc[ct] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+                            __builtin_bit_cast(f16x8, A), __builtin_bit_cast(f16x8, B), acc[ct], 0, 0, 0);
+                }
         }
     };
-
     // n % 64 == 0, so the chunks come in pairs
-    float4 xa[2][4], xb[2][4];
+    float4 xa[4], xb[4];
     load(xa, 0);
     for (int k0 = 0; k0 < n; k0 += 2 * TK) {
         load(xb, k0 + TK);
@@ -270,25 +271,23 @@ __global__ __launch_bounds__(256) void toeplitz_split_kernel(FilterArgs a, int n
 
     const float oscale = 1.0f / tscale;
 #pragma unroll
-    for (int rt = 0; rt < 2; rt++)
+    for (int ct = 0; ct < CT; ct++)
 #pragma unroll
-        for (int ct = 0; ct < 2; ct++)
-#pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const size_t om = m0 + wave * 64 + rt * 32 + 8 * (r / 4) + 4 * h + (r % 4);
-                const int col = n0 + ct * 32 + l32;
-                if (om < a.rows) {
-                    const float y = acc[rt][ct][r] * oscale;
-                    if (a.out_bf16)
-                        reinterpret_cast<uint16_t *>(a.out)[om * n + col] = f32_to_bf16_rne(y);
-                    else
-                        reinterpret_cast<float *>(a.out)[om * n + col] = y;
-                }
+        for (int r = 0; r < 16; r++) {
+            const size_t om = m0 + wave * 32 + 8 * (r / 4) + 4 * h + (r % 4);
+            const int col = n0 + ct * 32 + l32;
+            if (om < a.rows && col < n) {
+                const float y = acc[ct][r] * oscale;
+                if (a.out_bf16)
+                    reinterpret_cast<uint16_t *>(a.out)[om * n + col] = f32_to_bf16_rne(y);
+                else
+                    reinterpret_cast<float *>(a.out)[om * n + col] = y;
             }
+        }
 }
 
 // Direct FP32 convolution on the vector ALUs for widths that are not a
-// multiple of 64: one workgroup per row, taps and row staged in LDS.
+// multiple of 4: one workgroup per row, taps and row staged in LDS.
 __global__ __launch_bounds__(256) void conv_valu_kernel(FilterArgs a) {
     extern __shared__ float smem[];
     const int n = a.n;
@@ -695,6 +694,44 @@ __global__ __launch_bounds__(64 * SPEC_WAVES) void filter_spectrum_kernel(const 
     }
 }
 
+// widest rows that are no multiple of 64 channels (a row and its taps in 64 KB
+// of LDS)
+constexpr int CONV_MAX_N = 64 * 1024 / (3 * static_cast<int>(sizeof(float)));
+
+template <int MODE, int CT>
+int launch_split_ct(const FilterArgs &a, size_t lds, hipStream_t stream) {
+    const size_t n_rt = (a.rows + SPLIT_TM - 1) / SPLIT_TM, n_ct = (static_cast<size_t>(a.n) + 32 * CT - 1) / (32 * CT);
+    if (n_rt * n_ct > 0x7fffffffu) return CTBB_ERR_SHAPE;
+    const void *kf = reinterpret_cast<const void *>(&toeplitz_split_kernel<MODE, CT>);
+    if (lds > 65536 &&
+        hipFuncSetAttribute(kf, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)) != hipSuccess)
+        return CTBB_ERR_SHAPE;
+    hipLaunchKernelGGL((toeplitz_split_kernel<MODE, CT>), dim3(static_cast<unsigned>(n_rt * n_ct)), dim3(256), lds,
+                       stream, a, static_cast<int>(n_rt), static_cast<int>(n_ct));
+    return hipGetLastError() == hipSuccess ? CTBB_OK : CTBB_ERR_HIP;
+}
+
+template <int MODE>
+int launch_split(const FilterArgs &a, hipStream_t stream) {
+    int dev = 0, n_cu = 0, max_lds = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+        hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess)
+        return CTBB_ERR_HIP;
+    auto lds_of = [&](int ct) { return 8 * static_cast<size_t>(split_taps(a.n, ct)) * sizeof(uint16_t); };
+    auto tiles = [&](size_t ct) { return (a.rows + SPLIT_TM - 1) / SPLIT_TM * ((a.n + 32 * ct - 1) / (32 * ct)); };
+    // A workgroup's time hardly depends on the other CUs, so few rows take the
+    // narrowest tile that one per CU still covers (rows of 1472, F16X3, us with
+    // CT = 2 / 4 / 6: 128 rows 30 / 39 / 48, 1500 rows 48 / 43 / 52, 2600 rows
+    // 57 / 53 / 59, 4000 rows 85 / 72 / 66, 20000 rows 384 / 303 / 277), as do rows
+    // so wide (n > 10000) that the taps of six leave no room in LDS.
+    const size_t room = static_cast<size_t>(max_lds), cus = static_cast<size_t>(n_cu);
+    if (lds_of(2) > room) return CTBB_ERR_SHAPE;
+    if (tiles(2) <= cus || lds_of(6) > room) return launch_split_ct<MODE, 2>(a, lds_of(2), stream);
+    if (tiles(4) <= cus) return launch_split_ct<MODE, 4>(a, lds_of(4), stream);
+    return launch_split_ct<MODE, 6>(a, lds_of(6), stream);
+}
+
 }  // namespace
 
 int launch_filter_spectrum(const float *d_taps, int count, int L, float2 *d_spec, hipStream_t stream) {
@@ -744,45 +781,29 @@ int launch_filter(const FilterArgs &a, hipStream_t stream) {
         return CTBB_OK;
     }
     // FFT32 with 2n > 4096 uses the FP32 Toeplitz product below
-    if (a.n % 64 != 0) {
-        if (a.rows > 0x7fffffffu) return CTBB_ERR_SHAPE;
-        size_t lds = 3 * static_cast<size_t>(a.n) * sizeof(float);
-        if (lds > 64 * 1024) return CTBB_ERR_SHAPE;
+    // Split products on the double-K MFMAs.  Widths that are no multiple of 64
+    // get FP32 products in every mode, on the matrix cores if the rows can be
+    // read 16 bytes at a time (30000 rows of 1840: 1.75 ms, 10.7 ms on the
+    // vector ALUs; 30000 of 36: 23 us, 30 us).
+    if (a.mode == CTBB_FILTER_BF16X3 && a.n % 64 == 0) return launch_split<CTBB_FILTER_BF16X3>(a, stream);
+    if (a.mode == CTBB_FILTER_F16X3 && a.n % 64 == 0) return launch_split<CTBB_FILTER_F16X3>(a, stream);
+    if (a.n % 64 == 0 && a.mode != CTBB_FILTER_F32 && a.mode != CTBB_FILTER_FFT32) return CTBB_ERR_ARG;
+    if (a.n % 64 != 0 && (a.n > CONV_MAX_N || a.rows > 0x7fffffffu)) return CTBB_ERR_SHAPE;
+    if (a.n % 64 != 0 && (a.n % 4 != 0 || reinterpret_cast<uintptr_t>(a.in) % 16 != 0)) {
+        const size_t lds = 3 * static_cast<size_t>(a.n) * sizeof(float);
         hipLaunchKernelGGL(conv_valu_kernel, dim3(static_cast<unsigned>(a.rows)), dim3(256), lds, stream, a);
-        return hipGetLastError() == hipSuccess ? CTBB_OK : CTBB_ERR_HIP;
-    }
-    if (a.mode == CTBB_FILTER_BF16X3 || a.mode == CTBB_FILTER_F16X3) {
-        // 256 x 64 tiles on the double-K MFMAs; > 64 KB of LDS per workgroup
-        constexpr int TM = 256;
-        const size_t n_rt = (a.rows + TM - 1) / TM, n_ct = static_cast<size_t>(a.n) / 64;
-        if (n_rt * n_ct > 0x7fffffffu) return CTBB_ERR_SHAPE;
-        const size_t lds2 = 8 * (static_cast<size_t>(a.n) + 72) * sizeof(uint16_t);
-        const void *kf = a.mode == CTBB_FILTER_BF16X3
-                             ? reinterpret_cast<const void *>(&toeplitz_split_kernel<CTBB_FILTER_BF16X3>)
-                             : reinterpret_cast<const void *>(&toeplitz_split_kernel<CTBB_FILTER_F16X3>);
-        if (lds2 > 65536) {
-            int dev = 0, max_lds = 0;
-            if (hipGetDevice(&dev) != hipSuccess ||
-                hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess)
-                return CTBB_ERR_HIP;
-            if (lds2 > static_cast<size_t>(max_lds)) return CTBB_ERR_SHAPE;
-            if (hipFuncSetAttribute(kf, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds2)) !=
-                hipSuccess)
-                return CTBB_ERR_SHAPE;
-        }
-        const dim3 grid(static_cast<unsigned>(n_rt * n_ct));
-        if (a.mode == CTBB_FILTER_BF16X3)
-            hipLaunchKernelGGL((toeplitz_split_kernel<CTBB_FILTER_BF16X3>), grid, dim3(256), lds2, stream, a,
-                               static_cast<int>(n_rt), static_cast<int>(n_ct));
-        else
-            hipLaunchKernelGGL((toeplitz_split_kernel<CTBB_FILTER_F16X3>), grid, dim3(256), lds2, stream, a,
-                               static_cast<int>(n_rt), static_cast<int>(n_ct));
         return hipGetLastError() == hipSuccess ? CTBB_OK : CTBB_ERR_HIP;
     }
     const size_t gy = (a.rows + BM - 1) / BM;
     // FP32 Toeplitz product (CTBB_FILTER_F32, and FFT32 rows wider than 2048)
-    const size_t lds = BM * A_STRIDE * sizeof(float) + 2 * a.n * sizeof(float);
-    if (lds > 64 * 1024) return CTBB_ERR_SHAPE;
+    if ((BM * A_STRIDE + 2 * static_cast<size_t>(a.n)) * sizeof(float) > 64 * 1024) return CTBB_ERR_SHAPE;
+    const bool end = a.n % 64 != 0;
+    const size_t lds = (2 * BM * A_STRIDE + 2 * static_cast<size_t>(a.n) + (end ? 2 * TAP_MARGIN : 0)) * sizeof(float);
+    if (lds > 64 * 1024 &&
+        hipFuncSetAttribute(end ? reinterpret_cast<const void *>(&toeplitz_f32_kernel<true>)
+                                : reinterpret_cast<const void *>(&toeplitz_f32_kernel<false>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)) != hipSuccess)
+        return CTBB_ERR_SHAPE;
     // grid.y may exceed 65535 for very tall inputs: split into launches
     const size_t max_y = 65535;
     for (size_t y0 = 0; y0 < gy; y0 += max_y) {
@@ -792,9 +813,9 @@ int launch_filter(const FilterArgs &a, hipStream_t stream) {
         if (a.out_bf16) s.out = reinterpret_cast<uint16_t *>(a.out) + y0 * BM * a.n;
         else s.out = reinterpret_cast<float *>(a.out) + y0 * BM * a.n;
         s.rows = a.rows - y0 * BM < ny * BM ? a.rows - y0 * BM : ny * BM;
-        dim3 grid(a.n / BN, static_cast<unsigned>(ny));
-        if (a.mode != CTBB_FILTER_F32 && a.mode != CTBB_FILTER_FFT32) return CTBB_ERR_ARG;
-        hipLaunchKernelGGL(toeplitz_f32_kernel, grid, dim3(256), lds, stream, s);
+        dim3 grid((a.n + BN - 1) / BN, static_cast<unsigned>(ny));
+        if (end) hipLaunchKernelGGL(toeplitz_f32_kernel<true>, grid, dim3(256), lds, stream, s);
+        else hipLaunchKernelGGL(toeplitz_f32_kernel<false>, grid, dim3(256), lds, stream, s);
         if (hipGetLastError() != hipSuccess) return CTBB_ERR_HIP;
     }
     return CTBB_OK;

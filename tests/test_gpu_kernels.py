@@ -39,6 +39,31 @@ def test_fft_filter_spectrum_sizes(ctx, n, rows):
     assert np.abs(got - want).max() <= 2e-6 * np.abs(want).max()
 
 
+@pytest.mark.parametrize("mode", [cb.FILTER_F32, cb.FILTER_BF16X3, cb.FILTER_F16X3])
+@pytest.mark.parametrize("n,rows", [(4, 3), (60, 65), (64, 33000), (66, 2), (68, 64), (128, 127), (188, 130), (192, 128),
+                                    (256, 129), (1472, 131), (1472, 1409), (1472, 2700), (1840, 63), (5460, 5), (5888, 2), (7040, 3), (10112, 2)])
+def test_toeplitz_edges(ctx, n, rows, mode):
+    """Toeplitz products at the edges of the tiles, with a guard past the last
+    row.  Samples and taps are small whole numbers, so every product and sum is
+    exact in each form and the result has to be equal."""
+    rng = np.random.default_rng(10 * n + mode)
+    x = rng.integers(-8, 9, (rows, n))
+    taps = rng.integers(-8, 9, 2 * n)
+    want = np.stack([np.convolve(r, taps)[n:2 * n] for r in x])
+    out = torch.full((rows * n + 64,), 7.0, dtype=torch.float32, device="cuda")
+    x_d, taps_d = dev(x.astype(np.float32)), dev(taps.astype(np.float32))
+    ctx.set_options(filter_mode=mode, proj_dtype=cb.PROJ_F32)
+    if mode == cb.FILTER_F32 and n > 7040:
+        with pytest.raises(cb.CTBBError):
+            ctx.filter_rows_dev(taps_d, n, rows, x_d, out)
+        return
+    ctx.filter_rows_dev(taps_d, n, rows, x_d, out)
+    got = host(out)
+    ctx.set_options(filter_mode=cb.FILTER_F32)
+    np.testing.assert_array_equal(got[:rows * n].reshape(rows, n), want)
+    assert (got[rows * n:] == 7.0).all()
+
+
 def _mini(tmp_path, channels, nrows, ffs="none", turn=192, centre=None, **scanner):
     """Planned small scan on a scanner of `channels` channels and `turn`
     projections per turn."""
