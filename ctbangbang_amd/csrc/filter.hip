@@ -309,25 +309,46 @@ __global__ __launch_bounds__(256) void conv_valu_kernel(FilterArgs a) {
 
 // ---------------------------------------------------------------------------
 // FP32 FFT form of the same convolution (CTBB_FILTER_FFT32).
-// Embedding: with L = 4096 >= 2n, h[m] = taps[m] for m < 2n and 0 above, the
-// circular convolution y = x (*) h of the zero-padded row gives
-// y[n + l] = sum_k x[k] taps[n + l - k] for l in [0, n) without wrap-around
+// Embedding: with L >= 2n and h[m] = taps[(m + n) mod L] (0 where that is >= 2n),
+// the circular convolution y = x (*) h of the zero-padded row gives
+// y[l] = sum_k x[k] taps[n + l - k] for l in [0, n) without wrap-around
 // (n + l - k lies in [1, 2n - 1]).  Two rows a, b travel as one complex
 // signal a + i b: h is real, so y = (a (*) h) + i (b (*) h).
-// H = DFT_L(h) / L and the twiddles e^(-2 pi i t / L) come from
-// filter_spectrum_kernel, evaluated in FP64 and rounded once.  L = 3072 where 2n <= 3072 (the
-// shipped scanners: 1472 and 1344 oversampled channels), else 4096.
-// Transforms (Stockham, the passes in between through LDS with one pad
-// entry per 16 to spread the banks; the inverse is conj(DFT(conj(Y)))):
+// H = DFT_L(h) / L and the twiddles come from filter_spectrum_kernel, evaluated
+// in FP64 and rounded once.  L = 3072 where 2n <= 3072 (the shipped scanners:
+// 1472 and 1344 oversampled channels), else 4096.
+// Transforms (Stockham, the passes in between through LDS; the inverse is
+// conj(DFT(conj(Y)))):
 //   L = 4096: radix 16, 16, 16, each pass 256 threads x 16 points;
 //   L = 3072: forward radix 12, 16, 16 (256 threads x 12 points, then
 //   192 x 16), the inverse in the reverse order 16, 16, 12, so each
-//   transform starts from the layout the previous one ended in: 25% fewer
-//   VALU instructions than L = 4096 for the same rows.
+//   transform starts from the layout the previous one ended in.
+// Bound by VALU issue (and, over long runs, by the clock that the power leaves:
+// 1.8 GHz), so the passes are built from few instructions:
+//   - the upper half of the samples is zero and, with the taps turned by n, only
+//     the lower half of the results is wanted: the first and the last pass leave
+//     those out;
+//   - constant twiddles are split into a factor and a vector with an entry of 1;
+//     the factor becomes the multiplicand of additions that follow anyway;
+//   - in each exchange the padding makes the address linear in the point's
+//     number (a constant offset of the LDS instruction) and spreads the banks;
+//   - rows are read and written through buffer descriptors of their length
+//     (zeros past the end, no stores there).
+// A pass's twiddles are w^r of one w per thread; w, w^2, w^4 and w^8 come from a
+// table in the threads' order and the others are formed by products.  All
+// fifteen from a table load 40% more data: 665 us where this takes 534.
+// Butterflies of six FMAs (a - t b as 2a - (a + t b)) are as fast but add 25% to
+// the rounding error.
+// 119168 rows of 1472: 634 -> 534 us (1454 -> 1036 VALU instructions per wave),
+// 60001 of 1344: 293 -> 245 us, 45001 of 1840: 265 -> 235 us; the traffic alone
+// would take 290, 130 and 135 us.
 constexpr int FFT_L = 4096;
-constexpr int FFT_LDS = FFT_L + FFT_L / 16;
 constexpr int FFT_L3 = 3072;
-constexpr int FFT_LDS3 = FFT_L3 + FFT_L3 / 8;
+// Twiddles of a pass of stride Ns and radix R: 4 x Ns entries w^(2^m), w = e^(-2
+// pi i t / (Ns R)), t < Ns.  Their places in the table:
+constexpr int TW_16 = 0, TW_256 = 64, TW_END = TW_256 + 4 * 256;                       // L = 4096
+constexpr int TW3_12 = 0, TW3_16 = 48, TW3_192 = 112, TW3_256 = 880, TW3_END = 1904;   // L = 3072
+constexpr float FFT_S3 = 0.86602540378443865f;   // sin(pi / 3)
 
 __device__ __forceinline__ float2 cmul(float2 a, float2 b) {
     return make_float2(fmaf(a.x, b.x, -a.y * b.y), fmaf(a.x, b.y, a.y * b.x));
@@ -345,73 +366,15 @@ __device__ __forceinline__ void dft4(float2 &a0, float2 &a1, float2 &a2, float2 
     a3 = make_float2(d02.x - d13.y, d02.y + d13.x);
 }
 
-// 16-point DFT in natural order, as 4 x 4: inner DFTs over r2 (r = r1 + 4 r2),
-// twiddles W16^(r1 k2), outer DFTs over r1; X[k2 + 4 k1] ends in slot k1 + 4 k2.
-__device__ __forceinline__ void fft16(float2 (&v)[16]) {
-    constexpr float C1 = 0.92387953251128674f, S1 = 0.38268343236508978f, H2 = 0.70710678118654757f;
-#pragma unroll
-    for (int r1 = 0; r1 < 4; r1++) dft4(v[r1], v[r1 + 4], v[r1 + 8], v[r1 + 12]);
-    // W16^m = (cos(pi m / 8), -sin(pi m / 8))
-    v[5] = cmul(v[5], make_float2(C1, -S1));     // r1 1, k2 1: m 1
-    v[9] = cmul(v[9], make_float2(H2, -H2));     // r1 1, k2 2: m 2
-    v[13] = cmul(v[13], make_float2(S1, -C1));   // r1 1, k2 3: m 3
-    v[6] = cmul(v[6], make_float2(H2, -H2));     // r1 2, k2 1: m 2
-    v[10] = make_float2(v[10].y, -v[10].x);      // r1 2, k2 2: m 4 (-i)
-    v[14] = cmul(v[14], make_float2(-H2, -H2));  // r1 2, k2 3: m 6
-    v[7] = cmul(v[7], make_float2(S1, -C1));     // r1 3, k2 1: m 3
-    v[11] = cmul(v[11], make_float2(-H2, -H2));  // r1 3, k2 2: m 6
-    v[15] = cmul(v[15], make_float2(-C1, S1));   // r1 3, k2 3: m 9
-#pragma unroll
-    for (int k2 = 0; k2 < 4; k2++) dft4(v[4 * k2], v[4 * k2 + 1], v[4 * k2 + 2], v[4 * k2 + 3]);
-    // slot k1 + 4 k2 holds X[k2 + 4 k1]: transpose to natural order
-    float2 t;
-    t = v[1]; v[1] = v[4]; v[4] = t;
-    t = v[2]; v[2] = v[8]; v[8] = t;
-    t = v[3]; v[3] = v[12]; v[12] = t;
-    t = v[6]; v[6] = v[9]; v[9] = t;
-    t = v[7]; v[7] = v[13]; v[13] = t;
-    t = v[11]; v[11] = v[14]; v[14] = t;
-}
-
 // in-place 3-point DFT, forward sign: X1 = a0 + w a1 + w^2 a2, w = e^(-2 pi i / 3)
 __device__ __forceinline__ void dft3(float2 &a0, float2 &a1, float2 &a2) {
-    constexpr float S3 = 0.86602540378443865f;   // sin(pi / 3)
     const float2 t = cadd(a1, a2);
-    const float2 d = make_float2(S3 * (a1.x - a2.x), S3 * (a1.y - a2.y));
+    const float2 d = make_float2(FFT_S3 * (a1.x - a2.x), FFT_S3 * (a1.y - a2.y));
     const float2 c = make_float2(fmaf(-0.5f, t.x, a0.x), fmaf(-0.5f, t.y, a0.y));
     a0 = cadd(a0, t);
     a1 = make_float2(c.x + d.y, c.y - d.x);     // c - i d
     a2 = make_float2(c.x - d.y, c.y + d.x);     // c + i d
 }
-
-// 12-point DFT of v[0 .. 11] in natural order, as 3 x 4: inner 3-point DFTs
-// over r2 (r = r1 + 4 r2), twiddles W12^(r1 k2), outer 4-point DFTs over r1;
-// X[k2 + 3 k1] ends in slot k1 + 4 k2.
-__device__ __forceinline__ void fft12(float2 (&v)[16]) {
-    constexpr float S3 = 0.86602540378443865f;
-#pragma unroll
-    for (int r1 = 0; r1 < 4; r1++) dft3(v[r1], v[r1 + 4], v[r1 + 8]);
-    // W12^m = (cos(pi m / 6), -sin(pi m / 6))
-    v[5] = cmul(v[5], make_float2(S3, -0.5f));     // r1 1, k2 1: m 1
-    v[9] = cmul(v[9], make_float2(0.5f, -S3));     // r1 1, k2 2: m 2
-    v[6] = cmul(v[6], make_float2(0.5f, -S3));     // r1 2, k2 1: m 2
-    v[10] = cmul(v[10], make_float2(-0.5f, -S3));  // r1 2, k2 2: m 4
-    v[7] = make_float2(v[7].y, -v[7].x);           // r1 3, k2 1: m 3 (-i)
-    v[11] = make_float2(-v[11].x, -v[11].y);       // r1 3, k2 2: m 6 (-1)
-#pragma unroll
-    for (int k2 = 0; k2 < 3; k2++) dft4(v[4 * k2], v[4 * k2 + 1], v[4 * k2 + 2], v[4 * k2 + 3]);
-    // natural order: X[k] sits in slot k / 3 + 4 (k % 3)
-    float2 o[12];
-#pragma unroll
-    for (int k = 0; k < 12; k++) o[k] = v[k / 3 + 4 * (k % 3)];
-#pragma unroll
-    for (int k = 0; k < 12; k++) v[k] = o[k];
-}
-
-__device__ __forceinline__ int fpad(int i) { return i + (i >> 4); }
-// (the 3072-point passes: one pad entry per 8, measured 2% faster than one
-// per 16 for their stride-12 and stride-16 stores)
-__device__ __forceinline__ int fpad3(int i) { return i + (i >> 3); }
 
 // v[r] *= w^r for r = 1 .. 15, from b[m] = w^(2^m), m = 0..3: the other
 // powers are products of at most three of them (each product rounds once,
@@ -442,205 +405,283 @@ __device__ __forceinline__ void twiddle16(float2 (&v)[16], const float2 (&b)[4])
     v[15] = cmul(v[15], cmul(b[3], w7));
 }
 
-// Forward 4096-point DFT.  On entry v[r] = x[j + 256 r]; on exit
-// v[r] = X[j + 256 r].  tw: e^(-2 pi i t / 4096), t in [0, 4096).  Each
-// pass's twiddles are w^r of one w per thread; its four power-of-two powers
-// are requested one pass ahead (before the LDS exchange) and the other
-// eleven are formed by products.
-__device__ __forceinline__ void fft4096(float2 (&v)[16], float2 *sh, int j, const float2 *__restrict__ tw) {
-    float2 b[4];
-#pragma unroll
-    for (int m = 0; m < 4; m++) b[m] = tw[(16 << m) * (j & 15)];
-    fft16(v);                                           // pass Ns = 1: no twiddles
-    __syncthreads();                                    // earlier readers of sh are done
-#pragma unroll
-    for (int r = 0; r < 16; r++) sh[fpad(16 * j + r)] = v[r];
-    __syncthreads();
-#pragma unroll
-    for (int r = 0; r < 16; r++) v[r] = sh[fpad(j + 256 * r)];
-    twiddle16(v, b);
-#pragma unroll
-    for (int m = 0; m < 4; m++) b[m] = tw[j << m];
-    fft16(v);                                           // pass Ns = 16
-    __syncthreads();
-    const int base = (j >> 4) * 256 + (j & 15);
-#pragma unroll
-    for (int r = 0; r < 16; r++) sh[fpad(base + 16 * r)] = v[r];
-    __syncthreads();
-#pragma unroll
-    for (int r = 0; r < 16; r++) v[r] = sh[fpad(j + 256 * r)];
-    twiddle16(v, b);
-    fft16(v);                                           // pass Ns = 256
+// a (c - i s) for constants c and s, of which those of size 0 and 1 cost nothing
+__device__ __forceinline__ float2 turn(float2 a, float c, float s) {
+    auto mul2 = [](float x, float c, float y, float s) {
+        if (s == 0.0f) return c == 1.0f ? x : c == -1.0f ? -x : c * x;
+        if (c == 0.0f) return s == 1.0f ? y : s == -1.0f ? -y : s * y;
+        if (c == 1.0f) return s == 1.0f ? x + y : s == -1.0f ? x - y : fmaf(s, y, x);
+        if (c == -1.0f) return s == 1.0f ? y - x : s == -1.0f ? -x - y : fmaf(s, y, -x);
+        if (s == 1.0f) return fmaf(c, x, y);
+        return fmaf(c, x, -y);       // s == -1
+    };
+    return make_float2(mul2(a.x, c, a.y, s), mul2(a.y, c, a.x, -s));
 }
 
-// Forward 3072-point DFT, radix 12, 16, 16.  On entry (every thread)
-// v[r] = x[j + 256 r], r < 12; on exit (threads j < 192) v[r] = X[j + 192 r],
-// r < 16.  tw: e^(-2 pi i t / 3072).  Stockham: the pass of radix R and
-// stride Ns takes butterfly j from x[j + r N / R], turns it by
-// w^r, w = e^(-2 pi i (j mod Ns) / (Ns R)), and leaves output r at
-// (j / Ns) Ns R + j mod Ns + r Ns.
-__device__ __forceinline__ void fft3072(float2 (&v)[16], float2 *sh, int j, const float2 *__restrict__ tw) {
-    const bool act = j < 192;               // butterflies of the radix-16 passes
-    float2 b[4];
-#pragma unroll
-    for (int m = 0; m < 4; m++) b[m] = tw[act ? (16 * (j % 12)) << m : 0];
-    fft12(v);                                           // R 12, Ns 1
-    __syncthreads();                                    // earlier readers of sh are done
-#pragma unroll
-    for (int r = 0; r < 12; r++) sh[fpad3(12 * j + r)] = v[r];
-    __syncthreads();
-    if (act) {
-#pragma unroll
-        for (int r = 0; r < 16; r++) v[r] = sh[fpad3(j + 192 * r)];
-        twiddle16(v, b);
-#pragma unroll
-        for (int m = 0; m < 4; m++) b[m] = tw[j << m];
-        fft16(v);                                       // R 16, Ns 12
-    }
-    __syncthreads();
-    if (act) {
-        const int base = (j / 12) * 192 + j % 12;
-#pragma unroll
-        for (int r = 0; r < 16; r++) sh[fpad3(base + 12 * r)] = v[r];
-    }
-    __syncthreads();
-    if (act) {
-#pragma unroll
-        for (int r = 0; r < 16; r++) v[r] = sh[fpad3(j + 192 * r)];
-        twiddle16(v, b);
-        fft16(v);                                       // R 16, Ns 192
-    }
+// 4-point DFT of a0, f1 u1, f2 u2 and f1 u3 into a0, x1, x2, x3
+__device__ __forceinline__ void dft4s(float2 &a0, float2 u1, float2 u2, float2 u3, float f2, float f1, float2 &x1,
+                                      float2 &x2, float2 &x3) {
+    const float2 s02 = make_float2(fmaf(f2, u2.x, a0.x), fmaf(f2, u2.y, a0.y));
+    const float2 d02 = make_float2(fmaf(-f2, u2.x, a0.x), fmaf(-f2, u2.y, a0.y));
+    const float2 s13 = make_float2(u1.x + u3.x, u1.y + u3.y), d13 = make_float2(u1.x - u3.x, u1.y - u3.y);
+    a0 = make_float2(fmaf(f1, s13.x, s02.x), fmaf(f1, s13.y, s02.y));
+    x2 = make_float2(fmaf(-f1, s13.x, s02.x), fmaf(-f1, s13.y, s02.y));
+    x1 = make_float2(fmaf(f1, d13.y, d02.x), fmaf(-f1, d13.x, d02.y));
+    x3 = make_float2(fmaf(-f1, d13.y, d02.x), fmaf(f1, d13.x, d02.y));
 }
 
-// The same DFT with the radices in reverse order (16, 16, 12): on entry
-// (threads j < 192) v[r] = x[j + 192 r], r < 16; on exit (every thread)
-// v[r] = X[j + 256 r], r < 12.
-__device__ __forceinline__ void fft3072_rev(float2 (&v)[16], float2 *sh, int j, const float2 *__restrict__ tw) {
-    const bool act = j < 192;
-    float2 b[4];
+// the same with f3 = 1: a0, f1 u1, f2 u2, u3
+__device__ __forceinline__ void dft4t(float2 &a0, float2 u1, float2 u2, float2 u3, float f2, float f1, float2 &x1,
+                                      float2 &x2, float2 &x3) {
+    const float2 s02 = make_float2(fmaf(f2, u2.x, a0.x), fmaf(f2, u2.y, a0.y));
+    const float2 d02 = make_float2(fmaf(-f2, u2.x, a0.x), fmaf(-f2, u2.y, a0.y));
+    const float2 s13 = make_float2(fmaf(f1, u1.x, u3.x), fmaf(f1, u1.y, u3.y));
+    const float2 d13 = make_float2(fmaf(f1, u1.x, -u3.x), fmaf(f1, u1.y, -u3.y));
+    a0 = make_float2(s02.x + s13.x, s02.y + s13.y);
+    x2 = make_float2(s02.x - s13.x, s02.y - s13.y);
+    x1 = make_float2(d02.x + d13.y, d02.y - d13.x);
+    x3 = make_float2(d02.x - d13.y, d02.y + d13.x);
+}
+
+// 16-point DFT of w^r v[r] (kTw: w^(2^m) in b[m]; else w = 1) in natural order,
+// as 4 x 4: inner DFTs over r2 (r = r1 + 4 r2), twiddles W16^(r1 k2), outer DFTs
+// over r1; X[k2 + 4 k1] ends in slot k1 + 4 k2.  kHalfIn: v[8 .. 15] are taken as
+// zero; kHalfOut: X[0 .. 7] only.
+template <bool kTw, bool kHalfIn = false, bool kHalfOut = false>
+__device__ __forceinline__ void fft16(float2 (&v)[16], const float2 (&b)[4]) {
+    // cos(pi / 8), tan(pi / 8), sqrt(1 / 2)
+    constexpr float C1 = 0.92387953251128674f, T1 = 0.41421356237309503f, H2 = 0.70710678118654757f;
+    if (kTw) twiddle16(v, b);
 #pragma unroll
-    for (int m = 0; m < 4; m++) b[m] = tw[act ? (12 * (j & 15)) << m : 0];
-    if (act) fft16(v);                                  // R 16, Ns 1
-    __syncthreads();                                    // earlier readers of sh are done
-    if (act) {
-#pragma unroll
-        for (int r = 0; r < 16; r++) sh[fpad3(16 * j + r)] = v[r];
+    for (int r1 = 0; r1 < 4; r1++) {
+        if (kHalfIn) {
+            const float2 a = v[r1], c = v[r1 + 4];
+            v[r1] = cadd(a, c);
+            v[r1 + 8] = csub(a, c);
+            v[r1 + 4] = make_float2(a.x + c.y, a.y - c.x);
+            v[r1 + 12] = make_float2(a.x - c.y, a.y + c.x);
+        } else {
+            dft4(v[r1], v[r1 + 4], v[r1 + 8], v[r1 + 12]);
+        }
     }
-    __syncthreads();
-    if (act) {
+    // (W16^m = cos(pi m / 8) - i sin(pi m / 8), m = r1 k2)
+    dft4(v[0], v[1], v[2], v[3]);
+    dft4s(v[4], turn(v[5], 1.0f, T1), turn(v[6], 1.0f, 1.0f), turn(v[7], T1, 1.0f), H2, C1, v[5], v[6], v[7]);
+    dft4s(v[8], turn(v[9], 1.0f, 1.0f), turn(v[10], 0.0f, 1.0f), turn(v[11], -1.0f, 1.0f), 1.0f, H2, v[9], v[10], v[11]);
+    dft4s(v[12], turn(v[13], T1, 1.0f), turn(v[14], -1.0f, 1.0f), turn(v[15], -1.0f, -T1), H2, C1, v[13], v[14], v[15]);
+    float2 o[16];
 #pragma unroll
-        for (int r = 0; r < 16; r++) v[r] = sh[fpad3(j + 192 * r)];
-        twiddle16(v, b);
-        fft16(v);                                       // R 16, Ns 16
+    for (int k = 0; k < (kHalfOut ? 8 : 16); k++) o[k] = v[(k >> 2) + 4 * (k & 3)];
+#pragma unroll
+    for (int k = 0; k < (kHalfOut ? 8 : 16); k++) v[k] = o[k];
+}
+
+// 12-point DFTs as 3 x 4: inner 3-point DFTs over r2 (r = r1 + 4 r2), twiddles
+// W12^(r1 k2), outer 4-point DFTs over r1; X[k2 + 3 k1] ends in slot k1 + 4 k2.
+// The part after the 3-point DFTs:
+__device__ __forceinline__ void fft12_tail(float2 (&v)[16]) {
+    constexpr float T3 = 0.57735026918962573f, R3 = 1.7320508075688772f;   // 1 / sqrt(3), sqrt(3)
+    dft4(v[0], v[1], v[2], v[3]);
+    dft4t(v[4], turn(v[5], 1.0f, T3), turn(v[6], 1.0f, R3), turn(v[7], 0.0f, 1.0f), 0.5f, FFT_S3, v[5], v[6], v[7]);
+    dft4t(v[8], turn(v[9], 1.0f, R3), turn(v[10], -1.0f, R3), turn(v[11], -1.0f, 0.0f), 0.5f, 0.5f, v[9], v[10], v[11]);
+    float2 o[12];
+#pragma unroll
+    for (int k = 0; k < 12; k++) o[k] = v[k / 3 + 4 * (k % 3)];
+#pragma unroll
+    for (int k = 0; k < 12; k++) v[k] = o[k];
+}
+
+// v[6 .. 11] are taken as zero
+__device__ __forceinline__ void fft12_first(float2 (&v)[16]) {
+#pragma unroll
+    for (int r = 0; r < 2; r++) {
+        const float2 a0 = v[r], a1 = v[r + 4];
+        const float2 m = make_float2(fmaf(-0.5f, a1.x, a0.x), fmaf(-0.5f, a1.y, a0.y));
+        v[r] = make_float2(a0.x + a1.x, a0.y + a1.y);
+        v[r + 4] = make_float2(fmaf(FFT_S3, a1.y, m.x), fmaf(-FFT_S3, a1.x, m.y));
+        v[r + 8] = make_float2(fmaf(-FFT_S3, a1.y, m.x), fmaf(FFT_S3, a1.x, m.y));
     }
-#pragma unroll
-    for (int m = 0; m < 4; m++) b[m] = tw[j << m];
-    __syncthreads();
-    if (act) {
-        const int base = (j >> 4) * 256 + (j & 15);
-#pragma unroll
-        for (int r = 0; r < 16; r++) sh[fpad3(base + 16 * r)] = v[r];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int r = 0; r < 12; r++) v[r] = sh[fpad3(j + 256 * r)];
+    v[6] = v[10] = v[2];
+    v[7] = v[11] = v[3];
+    fft12_tail(v);
+}
+
+// of w^r v[r], w^(2^m) in b[m]
+__device__ __forceinline__ void fft12_last(float2 (&v)[16], const float2 (&b)[4]) {
     twiddle16<12>(v, b);
-    fft12(v);                                           // R 12, Ns 256
+#pragma unroll
+    for (int r1 = 0; r1 < 4; r1++) dft3(v[r1], v[r1 + 4], v[r1 + 8]);
+    fft12_tail(v);
 }
 
-// L = 3072 form of fft_filter_kernel (2n <= 3072); spec = [H (3072)]
-// followed by [twiddles (3072)].
+// Rows ra and ra + 1 as the parts of v[r] = x[j + 256 r], r < R; their R x 256
+// samples cover the row.
+template <int R>
+__device__ __forceinline__ void fft_load(float2 (&v)[16], const FilterArgs &a, size_t ra, bool has_b, int j) {
+    const __amdgpu_buffer_rsrc_t xa = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float *>(a.in + ra * a.n), static_cast<short>(0), a.n * static_cast<int>(sizeof(float)), 0x00020000);
+    const __amdgpu_buffer_rsrc_t xb =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(a.in + (ra + has_b) * a.n), static_cast<short>(0),
+                                          has_b ? a.n * static_cast<int>(sizeof(float)) : 0, 0x00020000);
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        v[r].x = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xa, 4 * j + 1024 * r, 0, 0));
+        v[r].y = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(xb, 4 * j + 1024 * r, 0, 0));
+    }
+}
+
+// the conjugates of v[r], r < R, as rows ra and ra + 1 of the result
+template <int R>
+__device__ __forceinline__ void fft_store(const float2 (&v)[16], const FilterArgs &a, size_t ra, bool has_b, int j) {
+    const int es = a.out_bf16 ? 2 : 4;
+    char *const out = reinterpret_cast<char *>(a.out);
+    const __amdgpu_buffer_rsrc_t ya =
+        __builtin_amdgcn_make_buffer_rsrc(out + ra * a.n * es, static_cast<short>(0), a.n * es, 0x00020000);
+    const __amdgpu_buffer_rsrc_t yb = __builtin_amdgcn_make_buffer_rsrc(
+        out + (ra + has_b) * a.n * es, static_cast<short>(0), has_b ? a.n * es : 0, 0x00020000);
+    if (a.out_bf16) {
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            __builtin_amdgcn_raw_buffer_store_b16(f32_to_bf16_rne(v[r].x), ya, 2 * j + 512 * r, 0, 0);
+            __builtin_amdgcn_raw_buffer_store_b16(f32_to_bf16_rne(-v[r].y), yb, 2 * j + 512 * r, 0, 0);
+        }
+    } else {
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v[r].x), ya, 4 * j + 1024 * r, 0, 0);
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(-v[r].y), yb, 4 * j + 1024 * r, 0, 0);
+        }
+    }
+}
+
+// v <- conj(v H): the inverse transform is conj(DFT(conj))
+template <int STEP>
+__device__ __forceinline__ void fft_apply(float2 (&v)[16], const float2 *__restrict__ H) {
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+        const float2 h = H[STEP * r];
+        v[r] = make_float2(fmaf(v[r].x, h.x, -v[r].y * h.y), fmaf(-v[r].x, h.y, -v[r].y * h.x));
+    }
+}
+
+// v[r] -> LDS -> v[r], all threads or those of the first three waves at either
+// end: point r goes to `to` + S_TO r and comes from `from` + S_FROM r.
+template <int S, int R>
+__device__ __forceinline__ void fft_put(const float2 (&v)[16], float2 *to) {
+#pragma unroll
+    for (int r = 0; r < R; r++) to[S * r] = v[r];
+}
+template <int S, int R>
+__device__ __forceinline__ void fft_get(float2 (&v)[16], const float2 *from) {
+#pragma unroll
+    for (int r = 0; r < R; r++) v[r] = from[S * r];
+}
+
+// A pass of radix R and stride Ns takes butterfly j from x[j + r L / R], turns
+// it by w^r, w = e^(-2 pi i (j mod Ns) / (Ns R)), and leaves output r at (j / Ns)
+// Ns R + j mod Ns + r Ns.  spec = [H (L)] followed by the twiddles; a pass's four
+// powers of w are requested one pass ahead.
+// One workgroup per pair of rows, 2n <= 3072.
 __global__ __launch_bounds__(256) void fft3072_filter_kernel(FilterArgs a) {
-    __shared__ float2 sh[FFT_LDS3];
+    __shared__ float2 sh[13 * 256];
     const int j = threadIdx.x;
-    const int n = a.n;
-    const float2 *__restrict__ H = a.spec;
+    const bool act = j < 192;               // butterflies of the radix-16 passes
     const float2 *__restrict__ tw = a.spec + FFT_L3;
     const size_t ra = 2 * static_cast<size_t>(blockIdx.x);
     const bool has_b = ra + 1 < a.rows;
-    const float *xa = a.in + ra * n;
-    const float *xb = xa + n;
-    float2 v[16];
+    float2 v[16], b[4];
+    fft_load<6>(v, a, ra, has_b, j);
 #pragma unroll
-    for (int r = 0; r < 12; r++) {
-        const int m = j + 256 * r;
-        v[r] = make_float2(m < n ? xa[m] : 0.0f, (m < n && has_b) ? xb[m] : 0.0f);
-    }
-    fft3072(v, sh, j, tw);
-    if (j < 192) {
+    for (int m = 0; m < 4; m++) b[m] = tw[TW3_12 + 12 * m + j % 12];
+    fft12_first(v);                                     // R 12, Ns 1
+    // point i at i + i / 12
+    fft_put<1, 12>(v, sh + 13 * j);
+    __syncthreads();
+    if (act) {
+        fft_get<208, 16>(v, sh + j + j / 12);
+        fft16<true>(v, b);                              // R 16, Ns 12
 #pragma unroll
-        for (int r = 0; r < 16; r++) {
-            const float2 y = cmul(v[r], H[j + 192 * r]);
-            v[r] = make_float2(y.x, -y.y);
-        }
+        for (int m = 0; m < 4; m++) b[m] = tw[TW3_192 + 192 * m + j];
     }
-    fft3072_rev(v, sh, j, tw);
-    // y = conj(v); keep y[n .. 2n)
+    __syncthreads();
+    // point i at i + 12 (i / 192)
+    if (act) fft_put<12, 16>(v, sh + j / 12 * 204 + j % 12);
+    __syncthreads();
+    if (act) {
+        fft_get<204, 16>(v, sh + j);
+        fft16<true>(v, b);                              // R 16, Ns 192
+        fft_apply<192>(v, a.spec + j);
 #pragma unroll
-    for (int r = 0; r < 12; r++) {
-        const int m = j + 256 * r;
-        if (m >= n && m < 2 * n) {
-            const size_t o = ra * n + (m - n);
-            if (a.out_bf16) {
-                uint16_t *ob = reinterpret_cast<uint16_t *>(a.out);
-                ob[o] = f32_to_bf16_rne(v[r].x);
-                if (has_b) ob[o + n] = f32_to_bf16_rne(-v[r].y);
-            } else {
-                float *of = reinterpret_cast<float *>(a.out);
-                of[o] = v[r].x;
-                if (has_b) of[o + n] = -v[r].y;
-            }
-        }
+        for (int m = 0; m < 4; m++) b[m] = tw[TW3_16 + 16 * m + (j & 15)];
+        fft16<false>(v, b);                             // R 16, Ns 1
     }
+    __syncthreads();
+    // point i at i + i / 16
+    if (act) fft_put<1, 16>(v, sh + 17 * j);
+    __syncthreads();
+    if (act) {
+        fft_get<204, 16>(v, sh + j + (j >> 4));
+        fft16<true>(v, b);                              // R 16, Ns 16
+    }
+#pragma unroll
+    for (int m = 0; m < 4; m++) b[m] = tw[TW3_256 + 256 * m + j];
+    __syncthreads();
+    // point i at i + 16 (i / 256)
+    if (act) fft_put<16, 16>(v, sh + (j >> 4) * 272 + (j & 15));
+    __syncthreads();
+    fft_get<272, 12>(v, sh + j);
+    fft12_last(v, b);                                   // R 12, Ns 256
+    fft_store<6>(v, a, ra, has_b, j);
 }
 
-// One workgroup per pair of rows; spec = [H (L)] followed by [twiddles (L)]
-// as float2.
-__global__ __launch_bounds__(256) void fft_filter_kernel(FilterArgs a) {
-    __shared__ float2 sh[FFT_LDS];
+// The same for 2n <= 4096.
+__global__ __launch_bounds__(256) void fft4096_filter_kernel(FilterArgs a) {
+    __shared__ float2 sh[17 * 256];
     const int j = threadIdx.x;
-    const int n = a.n;
-    const float2 *__restrict__ H = a.spec;
     const float2 *__restrict__ tw = a.spec + FFT_L;
     const size_t ra = 2 * static_cast<size_t>(blockIdx.x);
     const bool has_b = ra + 1 < a.rows;
-    const float *xa = a.in + ra * n;
-    const float *xb = xa + n;
-    float2 v[16];
+    float2 v[16], b[4];
+    fft_load<8>(v, a, ra, has_b, j);
+    auto twiddles = [&](int NS, const float2 *T) {
 #pragma unroll
-    for (int r = 0; r < 16; r++) {
-        const int m = j + 256 * r;
-        v[r] = make_float2(m < n ? xa[m] : 0.0f, (m < n && has_b) ? xb[m] : 0.0f);
-    }
-    fft4096(v, sh, j, tw);
-#pragma unroll
-    for (int r = 0; r < 16; r++) {
-        const float2 y = cmul(v[r], H[j + 256 * r]);
-        v[r] = make_float2(y.x, -y.y);
-    }
-    fft4096(v, sh, j, tw);
-    // y = conj(v); keep y[n .. 2n)
-#pragma unroll
-    for (int r = 0; r < 16; r++) {
-        const int m = j + 256 * r;
-        if (m >= n && m < 2 * n) {
-            const size_t o = ra * n + (m - n);
-            if (a.out_bf16) {
-                uint16_t *ob = reinterpret_cast<uint16_t *>(a.out);
-                ob[o] = f32_to_bf16_rne(v[r].x);
-                if (has_b) ob[o + n] = f32_to_bf16_rne(-v[r].y);
-            } else {
-                float *of = reinterpret_cast<float *>(a.out);
-                of[o] = v[r].x;
-                if (has_b) of[o + n] = -v[r].y;
-            }
-        }
-    }
+        for (int m = 0; m < 4; m++) b[m] = T[NS * m];
+    };
+    // points i at i + i / 16, then at i + 16 (i / 256)
+    float2 *const to1 = sh + 17 * j, *const to2 = sh + (j >> 4) * 272 + (j & 15);
+    const float2 *const from1 = sh + j + (j >> 4), *const from2 = sh + j;
+    twiddles(16, tw + TW_16 + (j & 15));
+    fft16<false, true>(v, b);                           // Ns 1
+    fft_put<1, 16>(v, to1);
+    __syncthreads();
+    fft_get<272, 16>(v, from1);
+    fft16<true>(v, b);                                  // Ns 16
+    twiddles(256, tw + TW_256 + j);
+    __syncthreads();
+    fft_put<16, 16>(v, to2);
+    __syncthreads();
+    fft_get<272, 16>(v, from2);
+    fft16<true>(v, b);                                  // Ns 256
+    fft_apply<256>(v, a.spec + j);
+    twiddles(16, tw + TW_16 + (j & 15));
+    fft16<false>(v, b);                                 // Ns 1
+    __syncthreads();
+    fft_put<1, 16>(v, to1);
+    __syncthreads();
+    fft_get<272, 16>(v, from1);
+    fft16<true>(v, b);                                  // Ns 16
+    twiddles(256, tw + TW_256 + j);
+    __syncthreads();
+    fft_put<16, 16>(v, to2);
+    __syncthreads();
+    fft_get<272, 16>(v, from2);
+    fft16<true, false, true>(v, b);                     // Ns 256
+    fft_store<8>(v, a, ra, has_b, j);
 }
 
-// Spectrum of the taps and twiddles of the FFT form: spec[k] = DFT_L(taps)[k]
-// / L (taps zero-padded from `count` to L) and spec[L + t] = e^(-2 pi i t / L),
-// evaluated in FP64 and rounded once.  The taps are real, so one wave takes
+// Spectrum of the taps and twiddles of the FFT form: spec[k] = DFT_L(h)[k] / L
+// (h: the taps zero-padded from `count` = 2n to L and turned by n), then
+// the twiddles of the passes, evaluated in FP64 and rounded once.  The taps are real, so one wave takes
 // bin k <= L / 2 and also writes bin L - k as its conjugate.  Each lane sums
 // its taps m = lane, lane + 64, ... by Horner's rule in w^64 (w = e^(-2 pi i
 // k / L), at most 64 steps: error far below FP32), times w^lane; 3072 x 2944
@@ -656,8 +697,13 @@ __global__ __launch_bounds__(64 * SPEC_WAVES) void filter_spectrum_kernel(const 
     const int k = blockIdx.x * SPEC_WAVES + (threadIdx.x >> 6);
     const int t = blockIdx.x * (64 * SPEC_WAVES) + threadIdx.x;
     double sn, cs;
-    if (t < L) {
-        sincospi(-2.0 * t / L, &sn, &cs);
+    const bool l3 = L == FFT_L3;
+    if (t < (l3 ? TW3_END : TW_END)) {
+        const int from = l3 ? (t < TW3_16 ? TW3_12 : t < TW3_192 ? TW3_16 : t < TW3_256 ? TW3_192 : TW3_256)
+                            : (t < TW_256 ? TW_16 : TW_256);
+        const int ns = l3 ? (t < TW3_16 ? 12 : t < TW3_192 ? 16 : t < TW3_256 ? 192 : 256) : (t < TW_256 ? 16 : 256);
+        const int rad = l3 && t >= TW3_256 ? 12 : 16, q = t - from;
+        sincospi(-2.0 * ((q % ns) << (q / ns)) / (rad * ns), &sn, &cs);
         spec[L + t] = make_float2(static_cast<float>(cs), static_cast<float>(sn));
     }
     if (k > L / 2) return;
@@ -681,7 +727,7 @@ __global__ __launch_bounds__(64 * SPEC_WAVES) void filter_spectrum_kernel(const 
         for (int e = 0; e < 8; e++) step(x[e]);
     }
     for (; q >= 0; q--) step(taps[64 * q + lane]);
-    sincospi(-2.0 * ((k * lane) % L) / L, &sn, &cs);
+    sincospi(-2.0 * (k * (lane - count / 2) % L) / L, &sn, &cs);
     double hr = fma(re, cs, -im * sn), hi = fma(re, sn, im * cs);
     for (int s = 32; s > 0; s >>= 1) {
         hr += __shfl_xor(hr, s, 64);
@@ -737,7 +783,7 @@ int launch_split(const FilterArgs &a, hipStream_t stream) {
 int launch_filter_spectrum(const float *d_taps, int count, int L, float2 *d_spec, hipStream_t stream) {
     if (!d_taps || !d_spec || count <= 0 || count > L || (L != FFT_L && L != FFT_L3)) return CTBB_ERR_ARG;
     const unsigned grid = static_cast<unsigned>((L / 2 + 1 + SPEC_WAVES - 1) / SPEC_WAVES);
-    // (grid * 256 threads >= L: the twiddles are covered)
+    // (grid * 256 threads >= L > TW_END, TW3_END: the twiddles are covered)
     hipLaunchKernelGGL(filter_spectrum_kernel, dim3(grid), dim3(64 * SPEC_WAVES), 0, stream, d_taps, count, L, d_spec);
     return hipGetLastError() == hipSuccess ? CTBB_OK : CTBB_ERR_HIP;
 }
@@ -775,7 +821,7 @@ int launch_filter(const FilterArgs &a, hipStream_t stream) {
             if (fft3)
                 hipLaunchKernelGGL(fft3072_filter_kernel, dim3(static_cast<unsigned>(np)), dim3(256), 0, stream, s);
             else
-                hipLaunchKernelGGL(fft_filter_kernel, dim3(static_cast<unsigned>(np)), dim3(256), 0, stream, s);
+                hipLaunchKernelGGL(fft4096_filter_kernel, dim3(static_cast<unsigned>(np)), dim3(256), 0, stream, s);
             if (hipGetLastError() != hipSuccess) return CTBB_ERR_HIP;
         }
         return CTBB_OK;

@@ -93,7 +93,7 @@ struct FilterArgs {
     const float *in;           // [rows][n]
     void *out;                 // [rows][n] float32 or bfloat16
     const float *taps;         // [2n]
-    const float2 *spec;        // FFT32: [H (fft_len)][twiddles (fft_len)]
+    const float2 *spec;        // FFT32: [H (fft_len)][twiddles], 2 fft_len reserved
     int fft_len;               // length of spec's transform: 3072 (2n <= 3072) or 4096
     size_t rows;
     int n;

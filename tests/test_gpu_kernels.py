@@ -39,6 +39,27 @@ def test_fft_filter_spectrum_sizes(ctx, n, rows):
     assert np.abs(got - want).max() <= 2e-6 * np.abs(want).max()
 
 
+@pytest.mark.parametrize("n,rows", [(1, 3), (256, 2), (257, 1), (1279, 3), (1281, 2), (1472, 5), (1536, 1), (1537, 3),
+                                    (1792, 2), (2047, 1), (2048, 3)])
+def test_fft_filter_row_ends(ctx, n, rows):
+    """Row ends and the last, single row of the FFT form: nothing is written past
+    the result, and bfloat16 results are the rounded FP32 ones (the arithmetic
+    before the store is the same)."""
+    rng = np.random.default_rng(n)
+    x_d = dev(rng.standard_normal(rows * n).astype(np.float32))
+    taps_d = dev((rng.standard_normal(2 * n) / np.sqrt(n)).astype(np.float32))
+    out = {}
+    for dtype, tt in ((cb.PROJ_F32, torch.float32), (cb.PROJ_BF16, torch.bfloat16)):
+        ctx.set_options(filter_mode=cb.FILTER_FFT32, proj_dtype=dtype)
+        o = torch.full((rows * n + 64,), 7.0, dtype=tt, device="cuda")
+        ctx.filter_rows_dev(taps_d, n, rows, x_d, o)
+        torch.cuda.synchronize()
+        assert (o[rows * n:] == 7.0).all()
+        out[dtype] = o[:rows * n]
+    ctx.set_options(filter_mode=cb.FILTER_F32, proj_dtype=cb.PROJ_F32)
+    assert torch.equal(out[cb.PROJ_F32].to(torch.bfloat16), out[cb.PROJ_BF16])
+
+
 @pytest.mark.parametrize("mode", [cb.FILTER_F32, cb.FILTER_BF16X3, cb.FILTER_F16X3])
 @pytest.mark.parametrize("n,rows", [(4, 3), (60, 65), (64, 33000), (66, 2), (68, 64), (128, 127), (188, 130), (192, 128),
                                     (256, 129), (1472, 131), (1472, 1409), (1472, 2700), (1840, 63), (5460, 5), (5888, 2), (7040, 3), (10112, 2)])
