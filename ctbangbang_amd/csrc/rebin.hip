@@ -41,9 +41,9 @@ namespace {
 // views whose loads are in flight together.  1934 views of 64 rows x 1472
 // channels, four focal spots: 550 us (822 us with four loads per output and
 // the index arithmetic per view and tap); 16 to 128 views, batches of 4 or 8
-// and any occupancy from 4 waves per SIMD up stay within 545-575 us: the
-// kernel is bound by the cache lines a gather touches (a wave's 64 channels
-// lie on about 14 readings' rows), 90-110 cycles per CU and wave of output.
+// and any occupancy from 4 waves per SIMD up stay within 545-575 us: bound by
+// the cache lines a gather touches (a wave's 64 channels lie on the rows of 14
+// readings), 90-110 cycles per CU and wave of output.
 constexpr int kViews = 16;
 constexpr int kBatch = 4;
 
@@ -85,41 +85,56 @@ __device__ __forceinline__ void for_each_block(const RebinArgs &a, F f) {
     }
 }
 
-// kHot: frames whose flag a.hot is set come from a.raw_af (the adaptive
-// filter's output where it changed the frame), the others from the pull.
-template <bool kHot>
-__device__ __forceinline__ void rebin_block(const RebinArgs &a, unsigned bx, unsigned br, unsigned bz, bool &bad) {
+// What an output channel of a row interpolates between.
+struct Lane {
+    int c, set, j;              // channel (clamped into the row), set and raw row
+    bool store;                 // not past the row
+    int ch0, ch1, fs0, fs1;     // raw channel and focal spot of the two taps
+    float fc, ao0, ao1;         // weight of the upper tap, azimuthal offsets
+};
+
+__device__ __forceinline__ Lane lane_taps(const RebinArgs &a, unsigned bx, unsigned br) {
+    Lane L;
     const int cl = static_cast<int>(bx) * 256 + static_cast<int>(threadIdx.x);
-    const int c = min(cl, a.nos - 1);                   // (lanes past the row repeat its last channel, unstored)
-    const bool store = cl < a.nos;
+    L.c = min(cl, a.nos - 1);                           // (lanes past the row repeat its last channel, unstored)
+    L.store = cl < a.nos;
     const int r = static_cast<int>(br);
     // set of the row (kinds 1 and 3 interleave rows: set 0, the -dr focal
     // spot(s), -> row 2j, set 1 -> 2j + 1, swapped with ReverseRowInterleave)
     const bool inter = (a.kind & 1) != 0;
-    const int set = inter ? (r & 1) ^ (a.reverse_rows ? 1 : 0) : 0;
-    const int j = inter ? r >> 1 : r;
+    L.set = inter ? (r & 1) ^ (a.reverse_rows ? 1 : 0) : 0;
+    L.j = inter ? r >> 1 : r;
     // the two channel taps: raw channel, focal spot and azimuthal offset of
     // each (kinds 0 and 1: neighbouring raw channels of one spot; 2 and 3:
     // neighbouring oversampled channels, alternately of the set's two spots)
-    const float by = a.bidx[set * a.nos + c];
-    int t0, t1, ch0, ch1, fs0, fs1;
-    float fc, ao0, ao1;
+    const float by = a.bidx[L.set * a.nos + L.c];
+    int t0, t1;
     if (a.kind <= 1) {
-        taps(by, a.nch, t0, t1, fc);
-        ch0 = t0;
-        ch1 = t1;
-        fs0 = fs1 = a.kind == 1 ? set : 0;
-        ao0 = ao1 = a.aoff[set * a.nos + c];
+        taps(by, a.nch, t0, t1, L.fc);
+        L.ch0 = t0;
+        L.ch1 = t1;
+        L.fs0 = L.fs1 = a.kind == 1 ? L.set : 0;
+        L.ao0 = L.ao1 = a.aoff[L.set * a.nos + L.c];
     } else {
-        taps(by, a.nos, t0, t1, fc);
-        ch0 = t0 >> 1;
-        ch1 = t1 >> 1;
-        fs0 = 2 * set + (t0 & 1);
-        fs1 = 2 * set + (t1 & 1);
-        ao0 = a.aoff[set * a.nos + t0];
-        ao1 = a.aoff[set * a.nos + t1];
+        taps(by, a.nos, t0, t1, L.fc);
+        L.ch0 = t0 >> 1;
+        L.ch1 = t1 >> 1;
+        L.fs0 = 2 * L.set + (t0 & 1);
+        L.fs1 = 2 * L.set + (t1 & 1);
+        L.ao0 = a.aoff[L.set * a.nos + t0];
+        L.ao1 = a.aoff[L.set * a.nos + t1];
     }
-    const int v0 = static_cast<int>(bz) * kViews;
+    return L;
+}
+
+// Views v0 .. v0 + kViews - 1 (to the end of the output) of the lane.
+// kHot: frames whose flag a.hot is set come from a.raw_af (the adaptive
+// filter's output where it changed the frame), the others from the pull.
+template <bool kHot>
+__device__ __forceinline__ void rebin_views(const RebinArgs &a, const Lane &L, unsigned br, int v0, bool &bad) {
+    const int c = L.c, j = L.j, ch0 = L.ch0, ch1 = L.ch1, fs0 = L.fs0, fs1 = L.fs1, r = static_cast<int>(br);
+    const bool store = L.store;
+    const float fc = L.fc, ao0 = L.ao0, ao1 = L.ao1;
     const int n_v = min(kViews, a.n_proj_out - v0);
     // reading of the lower azimuthal tap at view v0
     const float fl0 = floorf(-ao0), fl1 = floorf(-ao1);
@@ -223,17 +238,189 @@ __device__ __forceinline__ void rebin_block(const RebinArgs &a, unsigned bx, uns
     }
 }
 
-// One workgroup per (x, y, z) block of the grid.  Few registers: waves of it
-// fit in the 64 per lane a running backprojection leaves.
 template <bool kHot>
-__global__ __launch_bounds__(256) void rebin_kernel(RebinArgs a) {
+__device__ __forceinline__ void rebin_block(const RebinArgs &a, unsigned bx, unsigned br, unsigned bz, bool &bad) {
+    rebin_views<kHot>(a, lane_taps(a, bx, br), br, static_cast<int>(bz) * kViews, bad);
+}
+
+// One workgroup per (x, y, z) block of the grid, for frames from two sources.
+__global__ __launch_bounds__(256) void rebin_hot_kernel(RebinArgs a) {
     bool bad = false;
-    rebin_block<kHot>(a, blockIdx.x, blockIdx.y, blockIdx.z, bad);
+    rebin_block<true>(a, blockIdx.x, blockIdx.y, blockIdx.z, bad);
+    report_nonfinite(a.nonfinite, bad);
+}
+
+// The rebin with the chip to itself: a wave keeps the readings that its 64
+// channels are at in LDS and loads each of them once, row by row, where a gather
+// from memory touches the rows of all of them for every view.  Ring of 32
+// readings x 32 channels per focal spot, and four more channels of each reading
+// (64 output channels take 33 or 34 raw ones); in rows of 32 the channel alone
+// decides a sample's bank, so lanes on different readings do not collide.  The
+// readings come in chunks of 8: 8 views need three of them, and the next chunk is
+// on its way into registers meanwhile.  Each wave has its own ring and runs
+// without barriers.
+// 1934 views of 64 rows x 1472 channels from four focal spots: 320 us, the copy
+// rate for its 1.48 GB (551 us from memory); 1862 views of 1344 channels from two
+// spots: 250 us (414).
+constexpr int kRing = 32, kChunk = 8;
+constexpr int kRingMain = kRing * 32, kRingMore = kRing * 4;       // floats per spot
+
+template <int kSpots>
+__global__ __launch_bounds__(256) void rebin_ring_kernel(RebinArgs a, int views) {
+    // [wave][spot][reading][32 channels], [wave][spot][reading][4 channels]
+    __shared__ __attribute__((aligned(4 * kRingMain))) float lds[4 * kSpots * (kRingMain + kRingMore)];
+    bool bad = false;
+    const unsigned br = blockIdx.y;
+    const Lane L = lane_taps(a, blockIdx.x, br);
+    const int v0 = static_cast<int>(blockIdx.z) * views, n_v = min(views, a.n_proj_out - v0);
+    const float fl0 = floorf(-L.ao0), fl1 = floorf(-L.ao1);
+    const int p0 = v0 + a.add + static_cast<int>(fl0), p1 = v0 + a.add + static_cast<int>(fl1);
+    const int p_lo = wave_min(min(p0, p1)), span = -wave_min(-max(p0, p1)) - p_lo;
+    const int c_lo = wave_min(min(L.ch0, L.ch1)), c_n = -wave_min(-max(L.ch0, L.ch1)) - c_lo + 1;
+    const size_t frame = static_cast<size_t>(a.n_rows_raw) * a.nch, step = static_cast<size_t>(a.n_ffs) * frame;
+    const size_t ostep = static_cast<size_t>(a.n_rows) * a.nos;
+    // readings p_lo .. p_lo + np - 1, one more than the views use if their
+    // number is odd (they are loaded in pairs)
+    int np = span + n_v + 1;
+    np += np & 1;
+    // all inside the pull and (with the output rows) within 32-bit byte
+    // offsets, and three chunks hold what 8 views use
+    if (p_lo < 0 || p_lo + np > a.n_proj || span >= 2 * kChunk || c_n > 36 ||
+        static_cast<unsigned long long>(np) * step >= (1ull << 29) ||
+        static_cast<unsigned long long>(views) * ostep >= (1ull << 29)) {
+        for (int vv = 0; vv < n_v; vv += kViews) rebin_views<false>(a, L, br, v0 + vv, bad);
+        report_nonfinite(a.nonfinite, bad);
+        return;
+    }
+    const unsigned step_b = static_cast<unsigned>(step) * 4u, ostep_b = static_cast<unsigned>(ostep) * 4u;
+    const unsigned fb = static_cast<unsigned>(frame) * 4u;
+    const __amdgpu_buffer_rsrc_t src = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float *>(a.raw + static_cast<size_t>(p_lo) * step), static_cast<short>(0),
+        static_cast<int>(static_cast<unsigned>(np) * step_b), 0x00020000);
+    const __amdgpu_buffer_rsrc_t dst = __builtin_amdgcn_make_buffer_rsrc(
+        a.out + (static_cast<size_t>(v0) * a.n_rows + br) * a.nos, static_cast<short>(0),
+        static_cast<int>(static_cast<unsigned>(n_v - 1) * ostep_b + a.nos * 4u), 0x00020000);
+    // A chunk is loaded in pairs of readings of 32 channels, and 4 channels more
+    // of all its readings (channels clamped into the row; readings past the last
+    // one repeat it and are not used).
+    const int l = static_cast<int>(threadIdx.x & 63);
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+    const int ls = kSpots > 1 ? l >> 5 : 0;                         // spot of the lane's further channel
+    const int fs = a.kind <= 1 ? L.set : 2 * L.set;                 // first of the spots (kind 0: set 0)
+    const unsigned row_b = static_cast<unsigned>(fs) * fb + static_cast<unsigned>(L.j * a.nch) * 4u;
+    const int o_main = static_cast<int>(row_b + static_cast<unsigned>(l >> 5) * step_b) + 4 * min(c_lo + (l & 31), a.nch - 1);
+    const int o_more = static_cast<int>(row_b + static_cast<unsigned>(ls) * fb) + 4 * min(c_lo + 32 + (l & 3), a.nch - 1);
+    constexpr int kMain = kSpots * kChunk / 2;
+    auto load = [&](int chunk, float (&m)[kMain + 1]) {
+        auto get = [&](int o, unsigned so) {
+            return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(src, o, static_cast<int>(so), 0));
+        };
+#pragma unroll
+        for (int i = 0; i < kMain; i++)
+            m[i] = get(o_main, static_cast<unsigned>(min(chunk * kChunk + 2 * (i % (kChunk / 2)), np - 2)) * step_b +
+                                   i / (kChunk / 2) * fb);
+        m[kMain] = get(o_more + static_cast<int>(static_cast<unsigned>(min(chunk * kChunk + ((l & 31) >> 2), np - 1)) * step_b), 0);
+    };
+    float *const ring = lds + wave * kSpots * kRingMain + l;
+    float *const rest = lds + (4 * kSpots * kRingMain + (wave * kSpots + ls) * kRingMore + (l & 31));
+    auto put = [&](int chunk, const float (&m)[kMain + 1]) {
+        const int h = chunk & (kRing / kChunk - 1);
+#pragma unroll
+        for (int i = 0; i < kMain; i++)
+            ring[i / (kChunk / 2) * kRingMain + h * 32 * kChunk + 64 * (i % (kChunk / 2))] = m[i];
+        rest[h * 4 * kChunk] = m[kMain];
+        // (a wave's LDS accesses keep their order)
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    };
+    // LDS byte address of a tap's reading: up by a row per view, round in the ring
+    const unsigned lds_b = (unsigned)(uintptr_t)(__attribute__((address_space(3))) void *)lds;
+    struct Tap {
+        unsigned at, row, mask;
+    };
+    auto tap = [&](int ch, int f, int p) {
+        const int cc = ch - c_lo, s = kSpots > 1 ? f - fs : 0;
+        Tap t;
+        t.row = cc < 32 ? 128u : 16u;
+        t.mask = t.row * kRing - 1;
+        t.at = lds_b + 4u * static_cast<unsigned>(cc < 32 ? (wave * kSpots + s) * kRingMain + cc
+                                                          : 4 * kSpots * kRingMain + (wave * kSpots + s) * kRingMore + cc - 32) +
+               static_cast<unsigned>(p - p_lo) * t.row;
+        return t;
+    };
+    auto read = [](const Tap &t) { return *(const __attribute__((address_space(3))) float *)t.at; };
+    auto next = [](Tap &t) {
+        const unsigned n = t.at + t.row;
+        t.at = (n & t.mask) | (t.at & ~t.mask);
+    };
+    float m[kMain + 1];
+    {
+        float m1[kMain + 1], m2[kMain + 1];
+        load(0, m);
+        load(1, m1);
+        load(2, m2);
+        __builtin_amdgcn_sched_barrier(0);
+        put(0, m);
+        put(1, m1);
+        put(2, m2);
+    }
+    Tap t0 = tap(L.ch0, L.fs0, p0), t1 = tap(L.ch1, L.fs1, p1);
+    const int oc = L.store ? L.c * 4 : static_cast<int>(0x80000000u);
+    unsigned oo = 0;
+    float chk = 0.0f;           // NaN once an output is not finite
+    float proj = static_cast<float>(v0 + a.add);
+    float u0 = read(t0), u1 = read(t1);
+    auto view = [&](float w0, float w1) {
+        // weight of the upper reading: the FP32 index proj - aoff less the
+        // lower reading's number proj + floor(-aoff) (both steps exact but
+        // for the index's own rounding)
+        const float fa0 = (proj - L.ao0) - (proj + fl0), fa1 = kSpots == 1 ? fa0 : (proj - L.ao1) - (proj + fl1);
+        proj += 1.0f;
+        const float x0 = fmaf(fa0, w0 - u0, u0), x1 = fmaf(fa1, w1 - u1, u1);
+        const float y = fmaf(L.fc, x1 - x0, x0);
+        u0 = w0;
+        u1 = w1;
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(y), dst, oc, static_cast<int>(oo), 0);
+        chk = fmaf(y, 0.0f, chk);
+        oo += ostep_b;
+    };
+#pragma unroll 1
+    for (int b = 0; b * kChunk < n_v; b++) {
+        const bool more = (b + 1) * kChunk < n_v;
+        if (more) load(b + 3, m);
+        __builtin_amdgcn_sched_barrier(0);
+        if ((b + 1) * kChunk <= n_v) {
+#pragma unroll
+            for (int g = 0; g < kChunk; g += kBatch) {
+                float w0[kBatch], w1[kBatch];
+#pragma unroll
+                for (int e = 0; e < kBatch; e++) {
+                    next(t0);
+                    w0[e] = read(t0);
+                    next(t1);
+                    w1[e] = read(t1);
+                }
+                __builtin_amdgcn_sched_barrier(0);      // all of the reads in flight
+#pragma unroll
+                for (int e = 0; e < kBatch; e++) view(w0[e], w1[e]);
+            }
+        } else {
+#pragma unroll 1
+            for (int vv = b * kChunk; vv < n_v; vv++) {
+                next(t0);
+                next(t1);
+                view(read(t0), read(t1));
+            }
+        }
+        if (more) put(b + 3, m);
+    }
+    bad |= chk != 0.0f;         // (true for NaN)
     report_nonfinite(a.nonfinite, bad);
 }
 
 // A one-dimensional grid of RebinArgs::max_groups workgroups looping over the
-// blocks.
+// blocks, from memory: in such a loop the ring takes 80 registers, and with its
+// LDS one workgroup per CU fits beside a backprojection.
 template <bool kHot>
 __global__ __launch_bounds__(256) void rebin_loop_kernel(RebinArgs a) {
     bool bad = false;
@@ -252,16 +439,22 @@ int launch_rebin(const RebinArgs &a, hipStream_t stream) {
     if (a.n_rows != rows_needed) return CTBB_ERR_SHAPE;
     const dim3 grid((a.nos + 255) / 256, a.n_rows, (a.n_proj_out + kViews - 1) / kViews);
     if (grid.z > 65535u || grid.y > 65535u || a.max_groups < 0) return CTBB_ERR_SHAPE;
-    const unsigned long long blocks = static_cast<unsigned long long>(grid.x) * grid.y * grid.z;
-    const bool hot = a.hot != nullptr;
-    if (a.max_groups > 0 && static_cast<unsigned long long>(a.max_groups) < blocks) {
+    const unsigned long long row_blocks = static_cast<unsigned long long>(grid.x) * grid.y;
+    if (a.max_groups > 0 && static_cast<unsigned long long>(a.max_groups) < row_blocks * grid.z) {
         const dim3 g1(static_cast<unsigned>(a.max_groups));
-        if (hot) hipLaunchKernelGGL(rebin_loop_kernel<true>, g1, dim3(256), 0, stream, a);
+        if (a.hot) hipLaunchKernelGGL(rebin_loop_kernel<true>, g1, dim3(256), 0, stream, a);
         else hipLaunchKernelGGL(rebin_loop_kernel<false>, g1, dim3(256), 0, stream, a);
-    } else if (hot) {
-        hipLaunchKernelGGL(rebin_kernel<true>, grid, dim3(256), 0, stream, a);
+    } else if (a.hot) {
+        hipLaunchKernelGGL(rebin_hot_kernel, grid, dim3(256), 0, stream, a);
     } else {
-        hipLaunchKernelGGL(rebin_kernel<false>, grid, dim3(256), 0, stream, a);
+        // 64 views per wave, or 32 where those are fewer than 2048 workgroups, 8
+        // per CU (64 rows of 1344 channels, 300 views: 30 us with 32, 33 with 64;
+        // 600 views: 92 and 88)
+        auto blocks_z = [&](int views) { return static_cast<unsigned>((a.n_proj_out + views - 1) / views); };
+        const int views = row_blocks * blocks_z(64) < 2048 ? 32 : 64;
+        const dim3 g(grid.x, grid.y, blocks_z(views));
+        if (a.kind <= 1) hipLaunchKernelGGL(rebin_ring_kernel<1>, g, dim3(256), 0, stream, a, views);
+        else hipLaunchKernelGGL(rebin_ring_kernel<2>, g, dim3(256), 0, stream, a, views);
     }
     return hipGetLastError() == hipSuccess ? CTBB_OK : CTBB_ERR_HIP;
 }

@@ -151,6 +151,27 @@ def test_rebin_edges(ctx, tmp_path, ffs, channels, nrows, centre, reverse):
     cb.free_metadata(mr)
 
 
+@pytest.mark.parametrize("ffs,channels,nrows,turn", [("none", 66, 1, 440), ("none", 66, 1, 800), ("z", 97, 2, 460),
+                                                     ("phi", 66, 2, 460), ("both", 130, 4, 440), ("both", 130, 4, 480)])
+def test_rebin_readings_per_wave(ctx, tmp_path, ffs, channels, nrows, turn):
+    """Rebinning where the 64 channels of a wave lie just within, on both sides
+    of and beyond the 16 readings up to which it keeps them in LDS.  Tolerance as
+    in test_rebin_edges."""
+    import oracle
+    mr = _mini(tmp_path, channels, nrows, ffs, turn=turn)
+    s = cb.block_sizes(mr)
+    rng = np.random.default_rng(turn)
+    raw = rng.random(s.raw_pull).astype(np.float32)
+    out = torch.empty(s.rebin, dtype=torch.float32, device="cuda")
+    raw_d = dev(raw)
+    ctx.rebin_dev(mr, raw_d, out)
+    ctx.synchronize()
+    want = oracle.rebin(mr, raw, double=True)
+    got = host(out).reshape(want.shape)
+    assert np.abs(got - want).max() <= 2e-5 + np.spacing(np.float32(mr.ri.n_proj_pull // mr.ri.n_ffs))
+    cb.free_metadata(mr)
+
+
 @pytest.mark.parametrize("turn", [126, 2040, 2052, 5626, 5636])
 def test_adaptive_threshold_windows(ctx, tmp_path, turn):
     """Per-view threshold bit for bit around the window sizes that change the
