@@ -570,7 +570,8 @@ int backproject_dev(ctbb_ctx *ctx, const recon_metadata *mr, const void *d_rebin
 // ev_prep_done; the caller has made the zero-padded pull, if any, there
 // too) and hand over to ctx->stream for the filter.
 // filter_after: the ramp filter waits for this event (the backprojection
-// running beside the preparation: the FFT kernel beside it would slow both).
+// running beside the preparation: a filter whose registers do not fit beside it
+// would slow both).
 int prep_block(ctbb_ctx *c, recon_metadata *mr, const float *win, void *d_out, hipStream_t head = nullptr,
                hipEvent_t filter_after = nullptr) {
     const ct_geom &cg = mr->cg;
@@ -659,8 +660,8 @@ int ensure_pipeline(ctbb_ctx *c, size_t rebin_bytes) {
 // resident workgroups.  Such a block launches one workgroup per tile, and
 // the next block's filter does not wait for it: the filter's workgroups take
 // the slots of its retiring workgroups between rounds.  A block of fewer
-// rounds keeps the resident grid, and the filter runs after it (beside a
-// resident grid it would only get the tail).  Measured per volume: C4
+// rounds keeps the resident grid, and a filter whose registers do not fit beside
+// it runs after it (it would only get the tail).  Measured per volume: C4
 // (1024^2, 8 rounds) 482 against 494 ms; C1 (512^2, 2 rounds) and the
 // 768^2 c3 scans (4.5 rounds) were faster with the resident grid (c3, one
 // call per scan: 1.19 against 1.30 s with the threshold at 4).
@@ -687,9 +688,16 @@ int pipeline_block(ctbb_ctx *c, recon_metadata *mr, int item, int b, const float
     if (item >= ctbb_ctx::kPipeDepth && hipStreamWaitEvent(c->stream, c->ev_bp[k], 0) != hipSuccess)
         return CTBB_ERR_HIP;
     // the previous item's backprojection (launched just before) is the one
-    // this preparation runs beside
+    // this preparation runs beside; the 3072-point FFT fits beside it, the other
+    // filters wait for it.  So does that FFT without the adaptive filter, where it
+    // would come early in the backprojection, not in its last part (volumes, ms,
+    // filter after / beside: 320^2 53.7 / 51.9, 512^2 44.5 / 43.3, 768^2 90.7 /
+    // 90.3; without the adaptive filter 53.3 / 51.6, 47.4 / 47.4, 91.3 / 92.8)
     const bool many_rounds = bp_many_rounds(c, mr);
-    hipEvent_t running = item > 0 && !many_rounds ? c->ev_bp[(item - 1) % ctbb_ctx::kPipeDepth] : nullptr;
+    const bool fits = c->opt.adaptive_filter && c->opt.filter_mode == CTBB_FILTER_FFT32 &&
+                      filter_fits_beside(mr->cg.n_channels_oversampled);
+    hipEvent_t running =
+        item > 0 && !many_rounds && !fits ? c->ev_bp[(item - 1) % ctbb_ctx::kPipeDepth] : nullptr;
     int st = prep_block(c, mr, win, out.p, head, running);
     if (st) return st;
     if (hipEventRecord(c->ev_filt[k], c->stream) != hipSuccess ||
@@ -1103,7 +1111,11 @@ int ctbb_reconstruct_dev(ctbb_ctx *c, struct recon_metadata *mr, const float *d_
     }
     // the next call's head starts once every preparation of this call is done
     // (so it runs beside this call's last backprojection, not beside a
-    // preparation) and the head's workspaces have been read
+    // preparation) and the head's workspaces have been read, and not before the
+    // last backprojection starts (the rebin's grid would take its places)
+    if (n_blocks > 1 &&
+        hipStreamWaitEvent(c->stream, c->ev_bp[(n_blocks - 2) % ctbb_ctx::kPipeDepth], 0) != hipSuccess)
+        return CTBB_ERR_HIP;
     if (hipEventRecord(c->ev_prep_done, c->stream) != hipSuccess) return CTBB_ERR_HIP;
     st = join_pipeline(c);
     if (st) return st;
@@ -1567,8 +1579,7 @@ int batch_persistent(ctbb_ctx *c, int n_scans, recon_metadata *const *mrs, const
                 // the rebinning of every block, straight into its slot
                 // (low-register kernels that run beside the backprojection
                 // before; the first kernel of each block capped as in
-                // prep_block), then the filter of every slot in place (the
-                // FFT kernel needs the registers the backprojection holds)
+                // prep_block), then the filter of every slot in place
                 for (int j = rg.first; j < rg.second && !st; j++) {
                     recon_metadata *m = mrs[jobs[j].s];
                     ctbb::plan_block(m, jobs[j].b);
@@ -1876,6 +1887,10 @@ int batch_pipeline(ctbb_ctx *c, int n_scans, struct recon_metadata *const *mrs, 
         st = launch_finalize_blob(c, m, d_image, d_finals[s], c->fin_tab.as<char>() + fin_off[s], fin_mt[s],
                                   fin_nf[s], c->stream_bp);
         if (st) return st;
+        // (the preparation that waits for the scan's last backprojection starts
+        // together with the next one, not before it)
+        if (hipEventRecord(c->ev_bp[(item - 1) % ctbb_ctx::kPipeDepth], c->stream_bp) != hipSuccess)
+            return CTBB_ERR_HIP;
     }
     return join_pipeline(c);
 }

@@ -101,6 +101,9 @@ struct FilterArgs {
     int out_bf16;              // 1: write bfloat16
 };
 int launch_filter(const FilterArgs &a, hipStream_t stream);
+// Whether the FFT kernel for rows of n channels fits into the registers and LDS
+// that a backprojection leaves (64 registers per lane, 56 KB).
+inline bool filter_fits_beside(size_t n) { return 2 * n <= 3072; }
 // FilterArgs::spec of `count` taps (device memory) for transforms of length
 // L (3072 or 4096, >= count): 2 L entries at d_spec.
 int launch_filter_spectrum(const float *d_taps, int count, int L, float2 *d_spec, hipStream_t stream);
