@@ -33,12 +33,12 @@ _libs = {}
 
 
 def build(quiet=True):
-    """Compile liboracle64/32 (and _ref when the reference tree exists)."""
+    """Compile liboracle64/32 (and _ref when the reference's sources are there)."""
     cmd = ["make", "-C", HERE, "all"]
     subprocess.run(cmd, check=True, capture_output=quiet)
-    if os.path.isdir(os.environ.get("CTBB_REFERENCE", "/root/reference")):
-        subprocess.run(["make", "-C", HERE, "ref", "REF=" + os.environ.get("CTBB_REFERENCE", "/root/reference")],
-                       check=True, capture_output=quiet)
+    ref = os.environ.get("CTBB_REFERENCE", "/root/reference")
+    if os.path.isdir(os.path.join(ref, "src")):
+        subprocess.run(["make", "-C", HERE, "ref", "REF=" + ref], check=True, capture_output=quiet)
 
 
 def _load(name):
