@@ -130,7 +130,7 @@ typedef enum {
     CTBB_FILTER_F32 = 0,        /* FP32 Toeplitz product, FP32 accumulation */
     CTBB_FILTER_BF16X3 = 1,     /* BF16 hi+lo split operands on MFMA, FP32 accumulation */
     CTBB_FILTER_F16X3 = 2,      /* FP16 hi+lo split operands on MFMA, FP32 accumulation */
-    CTBB_FILTER_FFT32 = 3       /* FP32 4096-point FFT convolution (rows up to 2048 channels; wider: F32) */
+    CTBB_FILTER_FFT32 = 3       /* FP32 FFT convolution (rows up to 2048 channels; wider: F32) */
 } ctbb_filter_mode;
 
 typedef enum {
@@ -240,7 +240,8 @@ int ctbb_rebin_dev(ctbb_ctx *ctx, const struct recon_metadata *mr,
  * rows[r][l] <- sum_k taps[n + l - k] * rows[r][k].  d_out == d_in (in place)
  * is allowed only for the CTBB_FILTER_FFT32 filter (rows of at most 2048
  * channels) with CTBB_PROJ_F32 output; any other overlap of d_in and d_out
- * returns CTBB_ERR_ARG. */
+ * returns CTBB_ERR_ARG.  d_taps, like d_in, is read on the context's stream:
+ * keep it until the work is done. */
 int ctbb_filter_rows_dev(ctbb_ctx *ctx, const float *d_taps, int n, size_t n_rows_total,
                          const float *d_in, void *d_out);
 
