@@ -13,6 +13,7 @@
 #include <map>
 #include <mutex>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "ctbb_hip.h"
@@ -115,8 +116,9 @@ struct ctbb_ctx {
     // rows, zero-padded pull), so it touches nothing the previous call or
     // other entry points use
     DevBuf head_af, head_work, head_rebin, head_pad;
-    // finalize tap lists last uploaded to fin_tab (unchanged lists are not
-    // uploaded again: the upload waits for the compute stream)
+    // the bytes in fin_tab, empty while they are unknown (finalize tap lists
+    // already there are not uploaded again: the upload waits for the compute
+    // stream).  Only upload_finalize_taps writes the two.
     std::vector<char> fin_blob;
     // cached host-side keys
     std::string taps_key, maps_key;
@@ -256,6 +258,7 @@ int ensure_taps(ctbb_ctx *ctx, const recon_metadata *mr) {
     std::vector<float> t(2 * mr->cg.n_channels_oversampled);
     int st = ctbb_load_filter(mr, t.data());
     if (st) return st;
+    ctx->taps_key.clear();      // (not valid again before the new taps and spectrum are there)
     st = upload(ctx, ctx->taps, t.data(), t.size() * sizeof(float));
     if (st) return st;
     st = make_spec(ctx, ctx->taps.as<float>(), t.size());
@@ -279,6 +282,7 @@ int ensure_maps(ctbb_ctx *ctx, const recon_metadata *mr) {
     std::vector<float> both(bidx.size() + aoff.size());
     std::memcpy(both.data(), bidx.data(), bidx.size() * sizeof(float));
     std::memcpy(both.data() + bidx.size(), aoff.data(), aoff.size() * sizeof(float));
+    ctx->maps_key.clear();
     st = upload(ctx, ctx->maps, both.data(), both.size() * sizeof(float));
     if (st) return st;
     ctx->maps_key = key;
@@ -475,6 +479,14 @@ int finalize_blob(const recon_metadata *mr, std::vector<char> &blob, int *mt, in
     return CTBB_OK;
 }
 
+// Tap lists of a call (one scan's, or a batch's one after the other) into fin_tab.
+int upload_finalize_taps(ctbb_ctx *ctx, std::vector<char> blob) {
+    ctx->fin_blob.clear();
+    const int st = upload(ctx, ctx->fin_tab, blob.data(), blob.size());
+    if (!st) ctx->fin_blob = std::move(blob);
+    return st;
+}
+
 // Launch the finalize kernel with tap lists already on the device at d_blob.
 int launch_finalize_blob(ctbb_ctx *ctx, const recon_metadata *mr, const float *d_image, float *d_final,
                          const char *d_blob, int mt, int nf, hipStream_t on) {
@@ -499,9 +511,8 @@ int do_finalize(ctbb_ctx *ctx, const recon_metadata *mr, const float *d_image, f
     int st = finalize_blob(mr, blob, &mt, &nf);
     if (st) return st;
     if (blob != ctx->fin_blob || !ctx->fin_tab.p) {
-        st = upload(ctx, ctx->fin_tab, blob.data(), blob.size());
+        st = upload_finalize_taps(ctx, std::move(blob));
         if (st) return st;
-        ctx->fin_blob = blob;
     }
     return launch_finalize_blob(ctx, mr, d_image, d_final, ctx->fin_tab.as<char>(), mt, nf, ctx->stream);
 }
@@ -1516,7 +1527,7 @@ int batch_persistent(ctbb_ctx *c, int n_scans, recon_metadata *const *mrs, const
         fin.resize(fin_off[s] + blob.size());
         std::memcpy(fin.data() + fin_off[s], blob.data(), blob.size());
     }
-    if ((st = upload(c, c->fin_tab, fin.data(), fin.size()))) return st;
+    if ((st = upload_finalize_taps(c, std::move(fin)))) return st;
     // the device work list of every group: plans, jobs, view tables, queues
     for (size_t g = 0; g < groups.size(); g++) {
         st = launch_plan_batch(reinterpret_cast<const ScanPlanIn *>(dplan + lay[g].scans),
@@ -1840,7 +1851,7 @@ int batch_pipeline(ctbb_ctx *c, int n_scans, struct recon_metadata *const *mrs, 
     }
     st = build_view_tables(c, jobs, total);
     if (st) return st;
-    st = upload(c, c->fin_tab, fin.data(), fin.size());
+    st = upload_finalize_taps(c, std::move(fin));
     if (st) return st;
     st = c->image_stack.ensure(max_image * sizeof(float));
     if (st) return st;

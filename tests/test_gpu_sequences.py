@@ -1,0 +1,59 @@
+"""Calls that follow each other on one context: what one of them leaves in the
+context's workspaces must not reach the results of the next."""
+import numpy as np
+import pytest
+
+import ctbangbang_amd as cb
+from ctbangbang_amd import scans
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+
+def host(t):
+    torch.cuda.synchronize()
+    return t.cpu().numpy()
+
+
+def _scan(ctx, tmp_path, mini_dir, name, n_slices, thickness):
+    tok = scans.mini_tokens("none", nrows=8, nx=32, rotations=24, n_slices=n_slices)
+    tok.update(SliceThickness=thickness, EndPos=tok["StartPos"] + (n_slices - 1) * thickness)
+    prm = str(tmp_path / name)
+    cb.write_prm(prm, tok)
+    mr = cb.metadata_from_prm(prm, install_dir=mini_dir)
+    frame = mr.cg.n_rows_raw * mr.cg.n_channels
+    raw = torch.empty(tok["Readings"] * frame, dtype=torch.float32, device="cuda")
+    ctx.synth_scan_dev(mr, scans.phantom_for(tok, 5), 0, tok["Readings"], raw)
+    out = torch.empty(cb.block_sizes(mr).final_stack, dtype=torch.float32, device="cuda")
+    return mr, raw, tok["Readings"], out
+
+
+@pytest.mark.parametrize("mode", [cb.BATCH_PERSISTENT, cb.BATCH_PIPELINE])
+def test_volume_after_batch(ctx, tmp_path, mini_dir, mode):
+    """A volume, a batch of scans of other thicknesses and slice numbers (other
+    tap lists), the same volume again: equal images, and the same for the
+    finalize stage alone."""
+    ctx.set_options(mu_water=0.02, adaptive_filter=1, filter_mode=cb.FILTER_FFT32, proj_dtype=cb.PROJ_F32)
+    a = _scan(ctx, tmp_path, mini_dir, "a.prm", 12, 2.4)
+    b = [_scan(ctx, tmp_path, mini_dir, "b.prm", 5, 6.0), _scan(ctx, tmp_path, mini_dir, "c.prm", 30, 1.3)]
+    stack = torch.rand(cb.block_sizes(a[0]).image_stack, device="cuda") * 0.04
+    torch.cuda.synchronize()
+    want = []
+    for again in (False, True):
+        for call in (lambda: ctx.reconstruct_dev(*a), lambda: ctx.finalize_dev(a[0], stack, a[3])):
+            if again:
+                ctx.set_options(batch_mode=mode)
+                ctx.reconstruct_batch_dev(*([s[i] for s in b] for i in range(4)))
+                ctx.set_options(batch_mode=cb.BATCH_PERSISTENT)
+            call()
+            ctx.synchronize()
+            got = host(a[3]).copy()
+            if again:
+                assert np.array_equal(got, want.pop(0))
+            else:
+                want.append(got)
+    assert np.abs(got).max() > 0
+    for s in [a] + b:
+        cb.free_metadata(s[0])
+    ctx.set_options(mu_water=0.0)
