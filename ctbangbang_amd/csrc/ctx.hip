@@ -402,11 +402,13 @@ int do_backproject(ctbb_ctx *ctx, const recon_metadata *mr, const void *d_rebin,
     a.vtab = d_vtab;
     a.out = d_out;
     // partial images (one set: backprojections of a context follow each other,
-    // on its compute stream or on stream_bp, which wait for one another)
+    // on its compute stream or on stream_bp, which wait for one another); without
+    // memory for them each workgroup takes the parts of its tile in turn
     if (a.parts > 1 && alloc) {
-        st = ctx->bp_partial.ensure(32 * static_cast<size_t>(a.nx) * a.ny * a.parts * sizeof(float));
-        if (st) return st;
-        a.partial = ctx->bp_partial.as<float>();
+        if (ctx->bp_partial.ensure(32 * static_cast<size_t>(a.nx) * a.ny * a.parts * sizeof(float)) == CTBB_OK)
+            a.partial = ctx->bp_partial.as<float>();
+        else
+            (void)hipGetLastError();            // (the launches that follow check it)
     }
     if (!timed) return launch_backproject(a, on, beside);
     EventPair e = ctx->begin("backproject", on);

@@ -57,3 +57,52 @@ def test_volume_after_batch(ctx, tmp_path, mini_dir, mode):
     for s in [a] + b:
         cb.free_metadata(s[0])
     ctx.set_options(mu_water=0.0)
+
+
+def test_backproject_without_memory_for_parts(tmp_path):
+    """A block whose angles are summed in parts, with less free device memory
+    than its partial images take: the same image, and the calls that follow
+    work."""
+    tok = scans.base_tokens()
+    tok.update(Scanner="definitionas.scanner", Nrows=16, CollSlicewidth=1.2, Zffs=0, Phiffs=0, PitchValue=19.2,
+               Readings=12 * 1152, Nx=816, Ny=816, ReconFOV=300.0, SliceThickness=2.0, StartPos=80.0, NSlices=10,
+               EndPos=98.0)
+    prm = str(tmp_path / "p.prm")
+    cb.write_prm(prm, tok)
+    mr = cb.metadata_from_prm(prm)
+    cb.plan_block(mr, 0)
+    s = cb.block_sizes(mr)
+    reb = torch.rand(s.rebin, device="cuda")
+    img = [torch.full((s.image_block,), float("nan"), device="cuda") for _ in range(2)]
+    stack = torch.rand(s.image_stack, device="cuda")
+    final = torch.empty(s.final_stack, device="cuda")
+    torch.cuda.synchronize()
+    c = cb.Context(0)
+    free = torch.cuda.mem_get_info()[0]
+    c.backproject_dev(mr, reb, img[0])
+    c.synchronize()
+    assert free - torch.cuda.mem_get_info()[0] >= 2 * 4 * s.image_block         # the partial images of two parts or more
+    c.close()
+    c = cb.Context(0)
+    keep, room = [], 2 * 4 * s.image_block + (64 << 20)
+    try:
+        chunk = 32 << 30
+        while chunk >= 1 << 24 and len(keep) < 64:
+            n = min(chunk, torch.cuda.mem_get_info()[0] - room)
+            try:
+                if n >= 1 << 24:
+                    keep.append(torch.empty(n, dtype=torch.uint8, device="cuda"))
+                    continue
+            except torch.OutOfMemoryError:
+                pass
+            chunk //= 2
+        assert torch.cuda.mem_get_info()[0] < 3 * 4 * s.image_block
+        c.backproject_dev(mr, reb, img[1])
+        c.finalize_dev(mr, stack, final)
+        c.synchronize()
+    finally:
+        keep.clear()
+        torch.cuda.empty_cache()
+        c.close()
+    assert np.array_equal(host(img[0]), host(img[1]))
+    cb.free_metadata(mr)
