@@ -318,6 +318,9 @@ class Context:
         _check(lib().ctbb_rebin_filter_dev(self._h, C.byref(mr), _ptr(d_raw), _ptr(d_rebin)), "rebin_filter_dev")
 
     def filter_rows_dev(self, d_taps, n, rows, d_in, d_out):
+        """Ramp filter of `rows` rows of n channels.  FILTER_FFT32 (n <= 2048) has
+        read d_taps when it returns; otherwise keep d_taps, and always d_in
+        and d_out, until synchronize()."""
         _check(lib().ctbb_filter_rows_dev(self._h, _ptr(d_taps), int(n), int(rows), _ptr(d_in), _ptr(d_out)),
                "filter_rows_dev")
 

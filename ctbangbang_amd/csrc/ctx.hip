@@ -898,20 +898,28 @@ int ctbb_filter_rows_dev(ctbb_ctx *c, const float *d_taps, int n, size_t n_rows_
     if (!c || !d_taps || !d_in || !d_out || n <= 0) return CTBB_ERR_ARG;
     if (hipSetDevice(c->device) != hipSuccess) return CTBB_ERR_HIP;
     c->reset_events();
-    if (c->opt.filter_mode == CTBB_FILTER_FFT32) {
-        // The spectrum of these taps, computed on the device every call (the
-        // cached one belongs to a prm's filter).  The default stream is
-        // waited for on the device, so taps and rows written there are seen.
-        if (!c->ev_default && hipEventCreateWithFlags(&c->ev_default, hipEventDisableTiming) != hipSuccess)
-            return CTBB_ERR_HIP;
-        if (hipEventRecord(c->ev_default, nullptr) != hipSuccess ||
-            hipStreamWaitEvent(c->stream, c->ev_default, 0) != hipSuccess)
-            return CTBB_ERR_HIP;
-        c->taps_key.clear();
-        const int st = make_spec(c, d_taps, 2 * static_cast<size_t>(n));
-        if (st) return st;
-    }
-    return do_filter(c, d_taps, n, n_rows_total, d_in, d_out, c->opt.proj_dtype == CTBB_PROJ_BF16);
+    const int out_bf16 = c->opt.proj_dtype == CTBB_PROJ_BF16;
+    if (c->opt.filter_mode != CTBB_FILTER_FFT32) return do_filter(c, d_taps, n, n_rows_total, d_in, d_out, out_bf16);
+    // The spectrum of these taps, computed on the device every call (the
+    // cached one belongs to a prm's filter).  The default stream is waited for
+    // on the device, so taps and rows written there are seen; the taps have
+    // been read when the call returns (the host waits for the spectrum, with
+    // the filter queued behind it), so a caller may drop or change them then.
+    if (!c->ev_default && hipEventCreateWithFlags(&c->ev_default, hipEventDisableTiming) != hipSuccess)
+        return CTBB_ERR_HIP;
+    if (hipEventRecord(c->ev_default, nullptr) != hipSuccess ||
+        hipStreamWaitEvent(c->stream, c->ev_default, 0) != hipSuccess)
+        return CTBB_ERR_HIP;
+    c->taps_key.clear();
+    int st = make_spec(c, d_taps, 2 * static_cast<size_t>(n));
+    if (st) return st;
+    st = do_filter(c, d_taps, n, n_rows_total, d_in, d_out, out_bf16);
+    // (the timing event before the filter stands behind the spectrum)
+    const std::vector<EventPair> &timed = c->events["filter"];
+    const bool whole = timed.empty() || c->timing_failed;
+    if ((whole ? hipStreamSynchronize(c->stream) : hipEventSynchronize(timed.back().a)) != hipSuccess)
+        return CTBB_ERR_HIP;
+    return st;
 }
 
 int ctbb_rebin_filter_dev(ctbb_ctx *c, const struct recon_metadata *mr, const float *d_raw, void *d_rebin) {

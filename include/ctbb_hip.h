@@ -240,8 +240,12 @@ int ctbb_rebin_dev(ctbb_ctx *ctx, const struct recon_metadata *mr,
  * rows[r][l] <- sum_k taps[n + l - k] * rows[r][k].  d_out == d_in (in place)
  * is allowed only for the CTBB_FILTER_FFT32 filter (rows of at most 2048
  * channels) with CTBB_PROJ_F32 output; any other overlap of d_in and d_out
- * returns CTBB_ERR_ARG.  d_taps, like d_in, is read on the context's stream:
- * keep it until the work is done. */
+ * returns CTBB_ERR_ARG.  With the CTBB_FILTER_FFT32 filter (rows of at most
+ * 2048 channels) d_taps has been read when the call returns, and work queued on
+ * the default stream before the call is waited for (on the device).  Otherwise
+ * d_taps, like d_in with every filter, is read on the context's stream, which
+ * waits for no other: finish writing it before the call and keep it until the
+ * work is done. */
 int ctbb_filter_rows_dev(ctbb_ctx *ctx, const float *d_taps, int n, size_t n_rows_total,
                          const float *d_in, void *d_out);
 

@@ -106,3 +106,32 @@ def test_backproject_without_memory_for_parts(tmp_path):
         c.close()
     assert np.array_equal(host(img[0]), host(img[1]))
     cb.free_metadata(mr)
+
+
+def test_filter_rows_taps_dropped(ctx):
+    """Taps overwritten as soon as filter_rows_dev has returned, with work on
+    the context's stream ahead of it: the result is the one of the taps that
+    were passed."""
+    n, rows = 1472, 64
+    rng = np.random.default_rng(4)
+    taps = torch.from_numpy((rng.standard_normal(2 * n) / np.sqrt(n)).astype(np.float32)).cuda()
+    x = torch.from_numpy(rng.standard_normal(rows * n).astype(np.float32)).cuda()
+    ahead = torch.zeros(20000 * n, device="cuda")
+    ahead_out = torch.empty_like(ahead)
+    ahead_taps = torch.ones(2 * n, device="cuda")
+    out = [torch.empty(rows * n, device="cuda") for _ in range(2)]
+    torch.cuda.synchronize()
+    ctx.set_options(filter_mode=cb.FILTER_FFT32, proj_dtype=cb.PROJ_F32)
+    ctx.filter_rows_dev(taps, n, rows, x, out[0])
+    ctx.synchronize()
+    ctx.set_options(filter_mode=cb.FILTER_F32)
+    for _ in range(10):
+        ctx.filter_rows_dev(ahead_taps, n, 20000, ahead, ahead_out)
+    ctx.set_options(filter_mode=cb.FILTER_FFT32)
+    ctx.filter_rows_dev(taps, n, rows, x, out[1])
+    taps.zero_()
+    torch.cuda.synchronize()
+    ctx.synchronize()
+    ctx.set_options(filter_mode=cb.FILTER_F32)
+    assert float(out[0].abs().max()) > 0
+    assert torch.equal(out[0], out[1])
