@@ -36,6 +36,8 @@ struct BpArgs {
 };
 // Parts for a block of n_tiles tiles and `half` angles on n_cu compute units.
 int backproject_parts(int n_tiles, int half, int n_cu);
+// Weight W(|q|), |q| < 1, as the kernels evaluate it (on the host).
+float backproject_weight(float abs_q);
 // beside: the caller schedules other kernels to run beside this launch
 // (then the grid is only the resident workgroups, which stride over the
 // tiles; otherwise one workgroup per tile).
