@@ -876,6 +876,12 @@ int with_variant(int id, Op op) {
 // 144^2 3.5 / 1.2, 208^2 4.4 / 3.0, 288^2 9.0 / 6.0, 400^2 5.5 / 3.8, 448^2
 // 5.7 / 4.3, 640^2 9.3 / 7.7 (512^2 keeps one); 16 rows x 3456 views, 256^2
 // 3.24 / 2.00.
+// Two per CU also where a wide window leaves room for one workgroup or the
+// one-group form for three: rounds of their own number choose no better (64 rows,
+// ms, one part / by rounds of two / of the own number: one per CU, 256^2 at 250
+// mm 4.51 / 4.52 / 4.51, 288^2 at 300 mm 7.17 / 4.64 / 4.63, 400^2 at 400 mm 10.6 /
+// 8.53 / 8.60; three, 256^2 at 120 mm 3.64 / 2.10 / 2.29, 400^2 at 190 mm 7.00 /
+// 5.33 / 5.30).
 int backproject_parts(int n_tiles, int half, int n_cu) {
     const long slots = 2l * std::max(n_cu, 1);
     int best = 1;

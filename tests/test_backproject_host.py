@@ -1,5 +1,6 @@
-"""Host-side functions of the backprojection: the weight that its kernels
-evaluate (the same source, built for the host)."""
+"""Host-side functions of the backprojection: the number of parts that a block's
+angles are summed in, and the weight that its kernels evaluate (the same source,
+built for the host)."""
 import ctypes as C
 
 import numpy as np
@@ -31,3 +32,23 @@ def test_stierstorfer_weight(lo, hi):
     assert np.abs(got / want - 1).max() <= 1e-6
     if hi <= 0.6:
         assert (got == 1).all()
+
+
+@pytest.mark.parametrize("n_tiles,half,want", [
+    (1024, 576, 1), (512, 576, 1), (4096, 576, 1),              # whole rounds of two workgroups per CU
+    (256, 63, 1), (1, 32, 1),                                    # fewer than 32 angles for each part
+    (256, 576, 2), (625, 576, 4), (225, 576, 9),
+    (32, 512, 16), (1, 4096, 16), (32, 511, 15)])                # the upper limit
+def test_backproject_parts_rule(n_tiles, half, want):
+    """Parts for 256 compute units: one where the tiles fill whole rounds, never
+    more than 16 or than leave 32 angles each."""
+    parts = _function("_ZN4ctbb17backproject_partsEiii", C.c_int, C.c_int, C.c_int, C.c_int)
+    assert parts(n_tiles, half, 256) == want
+
+
+@pytest.mark.parametrize("tiles", [1, 6, 40, 272])
+def test_backproject_parts_of_small_images(tiles):
+    """The images of 16^2 to 272 x 256 with 96 angles that the GPU tests take for
+    blocks in parts are."""
+    parts = _function("_ZN4ctbb17backproject_partsEiii", C.c_int, C.c_int, C.c_int, C.c_int)
+    assert parts(tiles, 96, 256) > 1

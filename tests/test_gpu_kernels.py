@@ -262,3 +262,43 @@ def test_finalize_edges(ctx, tmp_path, nx, ny, thickness, offset):
             assert np.array_equal(got, oracle.finalize(mr, img, mu, double=False))
         cb.free_metadata(mr)
     ctx.set_options(mu_water=0.0)
+
+
+def test_backproject_sixteen_parts(ctx, tmp_path):
+    """The most parts a block's angles are summed in, against the form that never
+    splits a tile bit for bit and against the oracle (tolerance of
+    test_backproject_parts)."""
+    import ctypes as C
+
+    import oracle
+    from ctbangbang_amd import scans
+    d = str(tmp_path)
+    scans.mini_install(d, dict(scans.MINI_SCANNER, NProjTurn=1152))
+    nx, ny = 64, 128
+    tok = scans.mini_tokens("none", nrows=8)
+    tok.update(Nx=nx, Ny=ny, AcqFOV=240.0, Readings=tok["Readings"] * 6)
+    prm = str(tmp_path / "p.prm")
+    cb.write_prm(prm, tok)
+    mr = cb.metadata_from_prm(prm, install_dir=d)
+    cb.plan_block(mr, 0)
+    s = cb.block_sizes(mr)
+    rule = cb.lib()._ZN4ctbb17backproject_partsEiii
+    rule.restype, rule.argtypes = C.c_int, [C.c_int] * 3
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    assert rule(nx * ny // 256, int(mr.cg.n_proj_turn) // 2, cus) == 16
+    reb = np.random.default_rng(nx).random(s.rebin).astype(np.float32)
+    reb_d = dev(reb)
+    img = [torch.full((s.image_block,), np.nan, dtype=torch.float32, device="cuda") for _ in range(2)]
+    torch.cuda.synchronize()
+    ctx.set_options(proj_dtype=cb.PROJ_F32, bp_tile=0)
+    ctx.backproject_dev(mr, reb_d, img[0])
+    ctx.backproject_dev_noalloc(mr, reb_d, img[1])
+    ctx.synchronize()
+    got = host(img[0]).reshape(32, nx, ny)
+    assert np.array_equal(got, host(img[1]).reshape(got.shape))
+    rng = np.random.default_rng(1)
+    cx, cy = rng.integers(0, nx, 64), rng.integers(0, ny, 64)
+    want = oracle.backproject(mr, reb, oracle.BP_GPU, cols=(cx, cy))[:, cx, cy]
+    err = np.abs(got[:, cx, cy] - want)
+    assert np.count_nonzero(err > 2e-4 * np.abs(want).max()) <= 1e-3 * err.size
+    cb.free_metadata(mr)
