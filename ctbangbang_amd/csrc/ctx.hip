@@ -583,8 +583,7 @@ int backproject_dev(ctbb_ctx *ctx, const recon_metadata *mr, const void *d_rebin
 // ev_prep_done; the caller has made the zero-padded pull, if any, there
 // too) and hand over to ctx->stream for the filter.
 // filter_after: the ramp filter waits for this event (the backprojection
-// running beside the preparation: a filter whose registers do not fit beside it
-// would slow both).
+// running beside the preparation, where the filter beside it would slow both).
 int prep_block(ctbb_ctx *c, recon_metadata *mr, const float *win, void *d_out, hipStream_t head = nullptr,
                hipEvent_t filter_after = nullptr) {
     const ct_geom &cg = mr->cg;
@@ -673,8 +672,8 @@ int ensure_pipeline(ctbb_ctx *c, size_t rebin_bytes) {
 // resident workgroups.  Such a block launches one workgroup per tile, and
 // the next block's filter does not wait for it: the filter's workgroups take
 // the slots of its retiring workgroups between rounds.  A block of fewer
-// rounds keeps the resident grid, and a filter whose registers do not fit beside
-// it runs after it (it would only get the tail).  Measured per volume: C4
+// rounds keeps the resident grid, and of the filters only the small FFT may start
+// before its end (pipeline_block).  Measured per volume: C4
 // (1024^2, 8 rounds) 482 against 494 ms; C1 (512^2, 2 rounds) and the
 // 768^2 c3 scans (4.5 rounds) were faster with the resident grid (c3, one
 // call per scan: 1.19 against 1.30 s with the threshold at 4).
@@ -701,16 +700,21 @@ int pipeline_block(ctbb_ctx *c, recon_metadata *mr, int item, int b, const float
     if (item >= ctbb_ctx::kPipeDepth && hipStreamWaitEvent(c->stream, c->ev_bp[k], 0) != hipSuccess)
         return CTBB_ERR_HIP;
     // the previous item's backprojection (launched just before) is the one
-    // this preparation runs beside; the 3072-point FFT fits beside it, the other
-    // filters wait for it.  So does that FFT without the adaptive filter, where it
-    // would come early in the backprojection, not in its last part (volumes, ms,
-    // filter after / beside: 320^2 53.7 / 51.9, 512^2 44.5 / 43.3, 768^2 90.7 /
-    // 90.3; without the adaptive filter 53.3 / 51.6, 47.4 / 47.4, 91.3 / 92.8)
+    // this preparation runs beside.  The 3072-point FFT does not wait for it, the
+    // other filters do.  Where a workgroup of that FFT fits beside the resident
+    // ones it takes their idle issue slots; where none does (512^2 at 340 mm: 25.6
+    // KB of LDS left of 26.9; bp_tile 32: 8 registers of 64) it takes the places
+    // of the last ones as they retire, before the launch has ended.  Without the
+    // adaptive filter it waits too: it would come early in the backprojection,
+    // not in its last part.  Volumes, ms, filter after / beside: 320^2 53.7 / 51.9,
+    // 512^2 44.5 / 43.3, at 340 mm 49.7 / 48.2, with bp_tile 32 70.8 / 66.7, 768^2
+    // 90.7 / 90.3; without the adaptive filter 53.3 / 51.6, 47.4 / 47.4 and (768^2)
+    // 91.3 / 92.8
     const bool many_rounds = bp_many_rounds(c, mr);
-    const bool fits = c->opt.adaptive_filter && c->opt.filter_mode == CTBB_FILTER_FFT32 &&
-                      filter_fits_beside(mr->cg.n_channels_oversampled);
+    const bool early = c->opt.adaptive_filter && c->opt.filter_mode == CTBB_FILTER_FFT32 &&
+                       filter_is_small(mr->cg.n_channels_oversampled);
     hipEvent_t running =
-        item > 0 && !many_rounds && !fits ? c->ev_bp[(item - 1) % ctbb_ctx::kPipeDepth] : nullptr;
+        item > 0 && !many_rounds && !early ? c->ev_bp[(item - 1) % ctbb_ctx::kPipeDepth] : nullptr;
     int st = prep_block(c, mr, win, out.p, head, running);
     if (st) return st;
     if (hipEventRecord(c->ev_filt[k], c->stream) != hipSuccess ||

@@ -34,7 +34,8 @@ struct BpArgs {
     float *partial;            // parts > 1: [parts][32][nx][ny], 16-byte aligned; each part in workgroups of its own
                                // (null: one workgroup takes a tile's parts one after the other, same sums)
 };
-// Parts for a block of n_tiles tiles and `half` angles on n_cu compute units.
+// Parts for a block of n_tiles tiles and `half` angles on n_cu compute units (the
+// same for every kernel variant).
 int backproject_parts(int n_tiles, int half, int n_cu);
 // Weight W(|q|), |q| < 1, as the kernels evaluate it (on the host).
 float backproject_weight(float abs_q);
@@ -103,9 +104,11 @@ struct FilterArgs {
     int out_bf16;              // 1: write bfloat16
 };
 int launch_filter(const FilterArgs &a, hipStream_t stream);
-// Whether the FFT kernel for rows of n channels fits into the registers and LDS
-// that a backprojection leaves (64 registers per lane, 56 KB).
-inline bool filter_fits_beside(size_t n) { return 2 * n <= 3072; }
+// Whether rows of n channels take the 3072-point FFT kernel, which has 64 registers
+// per lane and 26.6 KB of LDS (the 4096-point one 83 and 34 KB): what the usual
+// backprojections leave on a compute unit (512^2 at 250 mm, 64 rows: 64 registers
+// and 58.9 KB).
+inline bool filter_is_small(size_t n) { return 2 * n <= 3072; }
 // FilterArgs::spec of `count` taps (device memory) for transforms of length
 // L (3072 or 4096, >= count): 2 L entries at d_spec.
 int launch_filter_spectrum(const float *d_taps, int count, int L, float2 *d_spec, hipStream_t stream);
