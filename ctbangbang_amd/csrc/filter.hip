@@ -33,7 +33,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef short i16x4 __attribute__((ext_vector_type(4)));
 
 constexpr int BM = 64, BN = 64, BK = 32;
-constexpr int TAP_MARGIN = 64;     // >= BN - 4 columns, >= BK - 4 samples past the row
+constexpr int TAP_MARGIN = 64;     // >= BN - 4 columns past the row
 constexpr int A_STRIDE = BK + 4;   // 36 floats: 16-byte aligned rows
 
 __device__ __forceinline__ uint16_t f32_to_bf16_rne(float f) {
@@ -42,8 +42,9 @@ __device__ __forceinline__ uint16_t f32_to_bf16_rne(float f) {
     return static_cast<uint16_t>(u >> 16);
 }
 
-// FP32 Toeplitz product on v_mfma_f32_16x16x4_f32, n % 4 == 0 (samples past the
-// row are zeros, columns past it are not stored).  One chain of sums in the order
+// FP32 Toeplitz product on v_mfma_f32_16x16x4_f32, n % 4 == 0 (the sums end with
+// the row: a zero past it would bring in taps that a column does not have, NaN
+// for infinite ones; columns past it are not stored).  One chain of sums in the order
 // of the samples: a row's smooth part cancels from the far taps to the near ones,
 // where chains over parts of the row keep the parts' large sums and their
 // rounding (4x the largest error).  Matrix-core bound, 118 to
@@ -52,8 +53,7 @@ template <bool kEnd>
 __global__ __launch_bounds__(256) void toeplitz_f32_kernel(FilterArgs a) {
     extern __shared__ float smem[];
     const int n = a.n;
-    float *Tf = smem + 2 * BM * A_STRIDE;      // [2n] taps; kEnd: between margins of zeros
-    constexpr int kMargin = kEnd ? TAP_MARGIN : 0;
+    float *Tf = smem + 2 * BM * A_STRIDE;      // [2n] taps; kEnd: a margin of zeros behind them
 
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = tid >> 6;
@@ -61,8 +61,7 @@ __global__ __launch_bounds__(256) void toeplitz_f32_kernel(FilterArgs a) {
     const size_t m0 = static_cast<size_t>(blockIdx.y) * BM;
     const int n0 = blockIdx.x * BN;
 
-    for (int j = tid; j < 2 * n + 2 * kMargin; j += 256)
-        Tf[j] = !kEnd || (j >= kMargin && j < 2 * n + kMargin) ? a.taps[j - kMargin] : 0.0f;
+    for (int j = tid; j < 2 * n + (kEnd ? TAP_MARGIN : 0); j += 256) Tf[j] = !kEnd || j < 2 * n ? a.taps[j] : 0.0f;
 
     f32x4 acc[2][2];
 #pragma unroll
@@ -83,31 +82,41 @@ __global__ __launch_bounds__(256) void toeplitz_f32_kernel(FilterArgs a) {
     };
     load(0);
 
-    for (int k0 = 0; k0 < n; k0 += BK) {
-        // two chunks in LDS in turn: one barrier per chunk
+    // two chunks in LDS in turn: one barrier per chunk
+    auto chunk = [&](int k0) {
         float *As = smem + (k0 & BK) * (BM * A_STRIDE / BK);
         f32x4 *dst = reinterpret_cast<f32x4 *>(As + arow * A_STRIDE + aseg);
         dst[0] = x0;
         dst[1] = x1;
         __syncthreads();
+        return As;
+    };
+    auto step = [&](const float *As, int k0, int kk) {
+        float af[2], bfv[2];
+#pragma unroll
+        for (int rt = 0; rt < 2; rt++) af[rt] = As[(wr * 32 + rt * 16 + lr) * A_STRIDE + kk + lk];
+#pragma unroll
+        for (int ct = 0; ct < 2; ct++) {
+            const int col = n0 + wc * 32 + ct * 16 + lr;
+            bfv[ct] = Tf[n + col - (k0 + kk + lk)];
+        }
+#pragma unroll
+        for (int rt = 0; rt < 2; rt++)
+#pragma unroll
+            for (int ct = 0; ct < 2; ct++)
+                acc[rt][ct] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[rt], bfv[ct], acc[rt][ct], 0, 0, 0);
+    };
+    int k0 = 0;
+    for (; k0 + BK <= n; k0 += BK) {
+        const float *As = chunk(k0);
         // prefetch the next K chunk of this thread's row while the MFMAs run
         if (k0 + BK < n) load(k0 + BK);
 #pragma unroll
-        for (int kk = 0; kk < BK; kk += 4) {
-            float af[2], bfv[2];
-#pragma unroll
-            for (int rt = 0; rt < 2; rt++) af[rt] = As[(wr * 32 + rt * 16 + lr) * A_STRIDE + kk + lk];
-#pragma unroll
-            for (int ct = 0; ct < 2; ct++) {
-                const int col = n0 + wc * 32 + ct * 16 + lr;
-                bfv[ct] = Tf[kMargin + n + col - (k0 + kk + lk)];
-            }
-#pragma unroll
-            for (int rt = 0; rt < 2; rt++)
-#pragma unroll
-                for (int ct = 0; ct < 2; ct++)
-                    acc[rt][ct] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[rt], bfv[ct], acc[rt][ct], 0, 0, 0);
-        }
+        for (int kk = 0; kk < BK; kk += 4) step(As, k0, kk);
+    }
+    if (kEnd && k0 < n) {
+        const float *As = chunk(k0);
+        for (int kk = 0; k0 + kk < n; kk += 4) step(As, k0, kk);
     }
 
     // D layout of 16x16 MFMA tiles: lane l, register e -> row 4*(l/16)+e, column l%16
@@ -835,8 +844,8 @@ int launch_filter(const FilterArgs &a, hipStream_t stream) {
     // FFT32 with 2n > 4096 uses the FP32 Toeplitz product below
     // Split products on the double-K MFMAs.  Widths that are no multiple of 64
     // get FP32 products in every mode, on the matrix cores if the rows can be
-    // read 16 bytes at a time (30000 rows of 1840: 1.75 ms, 10.7 ms on the
-    // vector ALUs; 30000 of 36: 23 us, 30 us).
+    // read 16 bytes at a time (30000 rows of 1840: 1.67 ms, 10.7 ms on the
+    // vector ALUs; 30000 of 36: 18 us, 30 us).
     if (a.mode == CTBB_FILTER_BF16X3 && a.n % 64 == 0) return launch_split<CTBB_FILTER_BF16X3>(a, stream);
     if (a.mode == CTBB_FILTER_F16X3 && a.n % 64 == 0) return launch_split<CTBB_FILTER_F16X3>(a, stream);
     if (a.n % 64 == 0 && a.mode != CTBB_FILTER_F32 && a.mode != CTBB_FILTER_FFT32) return CTBB_ERR_ARG;
@@ -850,7 +859,7 @@ int launch_filter(const FilterArgs &a, hipStream_t stream) {
     // FP32 Toeplitz product (CTBB_FILTER_F32, and FFT32 rows wider than 2048)
     if ((BM * A_STRIDE + 2 * static_cast<size_t>(a.n)) * sizeof(float) > 64 * 1024) return CTBB_ERR_SHAPE;
     const bool end = a.n % 64 != 0;
-    const size_t lds = (2 * BM * A_STRIDE + 2 * static_cast<size_t>(a.n) + (end ? 2 * TAP_MARGIN : 0)) * sizeof(float);
+    const size_t lds = (2 * BM * A_STRIDE + 2 * static_cast<size_t>(a.n) + (end ? TAP_MARGIN : 0)) * sizeof(float);
     if (lds > 64 * 1024 &&
         hipFuncSetAttribute(end ? reinterpret_cast<const void *>(&toeplitz_f32_kernel<true>)
                                 : reinterpret_cast<const void *>(&toeplitz_f32_kernel<false>),

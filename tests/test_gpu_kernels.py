@@ -302,3 +302,27 @@ def test_backproject_sixteen_parts(ctx, tmp_path):
     err = np.abs(got[:, cx, cy] - want)
     assert np.count_nonzero(err > 2e-4 * np.abs(want).max()) <= 1e-3 * err.size
     cb.free_metadata(mr)
+
+
+@pytest.mark.parametrize("mode", [cb.FILTER_F32, cb.FILTER_BF16X3, cb.FILTER_F16X3])
+@pytest.mark.parametrize("n", [4, 36, 66, 100, 128, 1840])
+def test_toeplitz_first_tap_unused(ctx, n, mode):
+    """No sample of the result contains taps[0] (n + l - k is at least 1): its
+    value, infinite or NaN, does not reach the rows.  Whole numbers, exact."""
+    rng = np.random.default_rng(n)
+    rows = 3
+    x = rng.integers(-8, 9, (rows, n))
+    taps = rng.integers(-8, 9, 2 * n).astype(np.float32)
+    want = np.stack([np.convolve(r, taps)[n:2 * n] for r in x])
+    ctx.set_options(filter_mode=mode, proj_dtype=cb.PROJ_F32)
+    x_d = dev(x.astype(np.float32))
+    for first in (np.nan, np.inf):
+        taps[0] = first
+        taps_d = dev(taps)
+        out = torch.empty(rows * n, dtype=torch.float32, device="cuda")
+        torch.cuda.synchronize()
+        ctx.filter_rows_dev(taps_d, n, rows, x_d, out)
+        ctx.synchronize()
+        got = host(out).reshape(rows, n)
+        np.testing.assert_array_equal(got, want)
+    ctx.set_options(filter_mode=cb.FILTER_F32)
