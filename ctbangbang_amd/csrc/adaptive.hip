@@ -69,24 +69,28 @@ __global__ __launch_bounds__(256) void af_sup(const float *raw, float *sup, floa
 }
 
 // reference preprocessing.cuh:87-113.  64 views per workgroup, their window
-// of maxima (edge indices clamped) in LDS: the n_avg dependent fused
-// multiply-adds then wait for LDS instead of memory (8448 views, n_avg 231:
-// 5.3 against 23 us).
-constexpr int kSmoothViews = 64;
+// of maxima (edge indices clamped) in LDS, kSmoothPart values of a view's sum at a
+// time: the n_avg dependent fused multiply-adds then wait for LDS instead of
+// memory (8448 views, n_avg 231: 5.3 against 23 us).
+constexpr int kSmoothViews = 64, kSmoothPart = 1024;
 
 __global__ __launch_bounds__(kSmoothViews) void af_smooth(const float *sup, float *sm, int n_proj, int n_avg) {
-    extern __shared__ float w[];                // [kSmoothViews + n_avg]
+    __shared__ float w[kSmoothViews + kSmoothPart];
     const int p0 = blockIdx.x * kSmoothViews, off = n_avg / 2, max_idx = n_proj - 1;
-    for (int i = threadIdx.x; i < kSmoothViews + n_avg; i += kSmoothViews) {
-        int idx = p0 - off + i;
-        idx = idx < 0 ? 0 : (idx > max_idx ? max_idx : idx);
-        w[i] = sup[idx];
-    }
-    __syncthreads();
     const float inv = 1.0f / static_cast<float>(n_avg);
     float acc = 0.0f;
+    for (int i0 = 0; i0 < n_avg; i0 += kSmoothPart) {
+        const int n = min(n_avg - i0, kSmoothPart);
+        if (i0 > 0) __syncthreads();
+        for (int i = threadIdx.x; i < kSmoothViews + n; i += kSmoothViews) {
+            int idx = p0 - off + i0 + i;
+            idx = idx < 0 ? 0 : (idx > max_idx ? max_idx : idx);
+            w[i] = sup[idx];
+        }
+        __syncthreads();
 #pragma unroll 8
-    for (int i = 0; i < n_avg; i++) acc = fmaf(inv, w[threadIdx.x + i], acc);
+        for (int i = 0; i < n; i++) acc = fmaf(inv, w[threadIdx.x + i], acc);
+    }
     if (p0 + static_cast<int>(threadIdx.x) < n_proj) sm[p0 + threadIdx.x] = acc;
 }
 
@@ -396,10 +400,8 @@ int launch_adaptive(const AdaptiveArgs &a, hipStream_t stream) {
     else if (!fixed || a.hot_only)
         hipLaunchKernelGGL(af_sup<false>, dim3(gsup), dim3(256), 0, stream, a.raw, sup, a.out, frame, a.n_proj);
     if (!fixed) {
-        const size_t win = (kSmoothViews + static_cast<size_t>(n_avg)) * sizeof(float);
-        if (win > 65536) return CTBB_ERR_SHAPE;
         hipLaunchKernelGGL(af_smooth, dim3(static_cast<unsigned>((a.n_proj + kSmoothViews - 1) / kSmoothViews)),
-                           dim3(kSmoothViews), win, stream, sup, sm, a.n_proj, n_avg);
+                           dim3(kSmoothViews), 0, stream, sup, sm, a.n_proj, n_avg);
         if (n_range <= 64 * 16)
             hipLaunchKernelGGL(af_thresh<16>, dim3(a.n_proj), dim3(64), 0, stream, sm, thr, a.n_proj, n_range,
                                a.n_proj_ffs, a.strength);

@@ -326,3 +326,25 @@ def test_toeplitz_first_tap_unused(ctx, n, mode):
         got = host(out).reshape(rows, n)
         np.testing.assert_array_equal(got, want)
     ctx.set_options(filter_mode=cb.FILTER_F32)
+
+
+@pytest.mark.parametrize("n_ffs", [20460, 20480, 40960, 330000])
+def test_adaptive_long_smoothing_windows(ctx, tmp_path, n_ffs):
+    """Per-view threshold bit for bit with 18-degree windows around one and two
+    parts of a view's sum (1023, 1025 and 2049 maxima; odd numbers only) and of
+    many (16501), which no 64 KB of LDS hold."""
+    import oracle
+    mr = _mini(tmp_path, 4, 16, turn=2040)
+    n = int(mr.ri.n_proj_pull)
+    mr.cg.n_proj_ffs = n_ffs
+    rng = np.random.default_rng(n_ffs)
+    size = 1.0 + 0.8 * np.sin(np.arange(n) * (4 * np.pi / 2040))
+    raw = (rng.random((n, 64)) * size[:, None]).astype(np.float32)
+    want, _ = oracle.adaptive_filter(mr, raw)
+    raw_d = dev(raw.ravel())
+    out = torch.zeros_like(raw_d)
+    torch.cuda.synchronize()
+    ctx.adaptive_filter_dev(mr, raw_d, out)
+    ctx.synchronize()
+    assert np.array_equal(host(out).reshape(n, 64), want.reshape(n, 64))
+    cb.free_metadata(mr)
