@@ -46,6 +46,8 @@ namespace {
 // readings), 90-110 cycles per CU and wave of output.
 constexpr int kViews = 16;
 constexpr int kBatch = 4;
+// azimuthal offset that puts every view before the first reading (a whole number)
+constexpr float kFirstReading = 1073741824.0f;
 
 // Clamp a fractional index into [0, n-1] and split it into the two taps and
 // the weight of the upper tap (texture clamp addressing).
@@ -124,6 +126,10 @@ __device__ __forceinline__ Lane lane_taps(const RebinArgs &a, unsigned bx, unsig
         L.ao0 = a.aoff[L.set * a.nos + t0];
         L.ao1 = a.aoff[L.set * a.nos + t1];
     }
+    // A channel that no fan ray is parallel to (more than a radian off the central
+    // one) has no offset: NaN, which as an index clamps to the first reading.
+    if (L.ao0 != L.ao0) L.ao0 = kFirstReading;
+    if (L.ao1 != L.ao1) L.ao1 = kFirstReading;
     return L;
 }
 

@@ -348,3 +348,29 @@ def test_adaptive_long_smoothing_windows(ctx, tmp_path, n_ffs):
     ctx.synchronize()
     assert np.array_equal(host(out).reshape(n, 64), want.reshape(n, 64))
     cb.free_metadata(mr)
+
+
+@pytest.mark.parametrize("ffs", ["none", "z", "phi", "both"])
+def test_rebin_channels_beyond_the_fan(ctx, tmp_path, ffs):
+    """A fan so wide that the outermost parallel channels are parallel to no ray
+    (an arcsine beyond 1, NaN coordinates): they clamp to the first reading and
+    channel, whole numbers here, and are not taken for non-finite samples."""
+    mr = _mini(tmp_path, 300, 4, ffs, turn=1000)
+    s = cb.block_sizes(mr)
+    raw = np.random.default_rng(3).integers(1, 99, s.raw_pull).astype(np.float32)
+    out = torch.full((s.rebin,), np.nan, dtype=torch.float32, device="cuda")
+    raw_d = dev(raw)
+    torch.cuda.synchronize()
+    ctx.rebin_dev(mr, raw_d, out)
+    ctx.synchronize()
+    got = host(out).reshape(s.n_proj_out, mr.cg.n_rows, mr.cg.n_channels_oversampled)
+    assert np.isfinite(got).all()
+    sine = (np.arange(600) - 2.0 * mr.cg.central_channel) * (mr.cg.fan_angle_increment / 2)
+    beyond = np.flatnonzero(np.abs(sine) > 1.01)
+    assert beyond.size > 0
+    if ffs in ("none", "z"):
+        pull = raw.reshape(-1, mr.cg.n_rows_raw, mr.cg.n_channels)
+        for r in range(int(mr.cg.n_rows)):
+            spot, row = (r & 1, r >> 1) if ffs == "z" else (0, r)
+            assert (got[:, r, beyond] == pull[spot, row, 0]).all()
+    cb.free_metadata(mr)
