@@ -15,11 +15,13 @@
 //      held in registers (min and max taken on the way, order-free), then
 //      exact integer counts over it
 //   5. 5x5x5 triangle smoothing of samples above threshold: a wave takes 64
-//      channels x 8 rows of a view
+//      channels x 8 rows of a view, or of several views of few rows
 // A fixed-threshold mode (no counterpart in the reference) skips steps 1-4
 // and smooths the samples above one given line-integral threshold, e.g.
 // ln(I0 / N) for a noise threshold of N photons at I0 incident photons.
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
 
 #include "kernels.h"
 
@@ -225,7 +227,8 @@ __device__ __forceinline__ constexpr int af_tri(int i) { return 3 - (i < 3 ? 3 -
 // waves cover the loads and one row at a time needs the fewest registers (0.36
 // against 0.39 ms for two); where few waves smooth, each waits for memory at
 // every group.
-template <int kGroup>
+// kFew: rows outside the frame are passed over.
+template <int kGroup, bool kFew>
 __device__ __forceinline__ void af_smooth_rows(const float *raw, float (&acc)[kRows], int i, int j0, int p, int n_proj,
                                                int n_rows_raw, int nch, size_t ps) {
     __amdgpu_buffer_rsrc_t rs[5];
@@ -250,6 +253,10 @@ __device__ __forceinline__ void af_smooth_rows(const float *raw, float (&acc)[kR
         static_assert((kRows + 4) % kGroup == 0, "whole groups of rows");
 #pragma unroll
         for (int q0 = 0; q0 < kRows + 4; q0 += kGroup) {
+            if (kFew && (j0 - 2 + q0 + kGroup <= 0 || j0 - 2 + q0 >= n_rows_raw)) {
+                off = c_in ? off + kGroup * row_b : off;
+                continue;
+            }
             float v[kGroup][5];
 #pragma unroll
             for (int g = 0; g < kGroup; g++) {          // row j0 - 2 + q0 + g
@@ -294,7 +301,7 @@ __device__ __forceinline__ float af_norm(int i, int j, int p, int n_proj, int n_
 
 // Rows j0 .. j0 + kRows - 1 of channels i (one per lane) of view p; kCopied:
 // out already holds the raw samples, only waves that smooth some are written.
-template <bool kCopied, int kGroup>
+template <bool kCopied, int kGroup, bool kFew>
 __device__ __forceinline__ void af_apply_rows(const float *raw, float T, float *out, int i, int j0, int p, int n_proj,
                                               int n_rows_raw, int nch, size_t ps) {
     const size_t base = ps * p + static_cast<size_t>(j0) * nch + i;
@@ -307,7 +314,7 @@ __device__ __forceinline__ void af_apply_rows(const float *raw, float T, float *
     }
     if (__builtin_amdgcn_ballot_w64(hot)) {
         float acc[kRows];
-        af_smooth_rows<kGroup>(raw, acc, i, j0, p, n_proj, n_rows_raw, nch, ps);
+        af_smooth_rows<kGroup, kFew>(raw, acc, i, j0, p, n_proj, n_rows_raw, nch, ps);
 #pragma unroll
         for (int r = 0; r < kRows; r++)
             if (x[r] > T) x[r] = (1.0f / af_norm(i, j0 + r, p, n_proj, n_rows_raw, nch)) * acc[r];
@@ -350,10 +357,47 @@ __global__ __launch_bounds__(256) void af_apply(const float *raw, const float *s
 #pragma unroll 1
     for (int w = part * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); w < waves; w += 4 * bpv) {
         const int g = w / tiles;
-        af_apply_rows<kMode == kHotCopied, kMode == kAllViews ? 1 : 2>(
+        af_apply_rows<kMode == kHotCopied, kMode == kAllViews ? 1 : 2, false>(
             raw, T, out, (w - g * tiles) * 64 + (threadIdx.x & 63), g * kRows, p, n_proj, n_rows_raw, nch,
             static_cast<size_t>(nch) * n_rows_raw);
     }
+}
+
+// Every view of a detector of few rows: a wave takes the kRows / n_rows_raw views
+// that fill its rows, copies those without a sample above their threshold and
+// smooths the others one by one.  XCD x takes the x-th `band` of these groups of
+// views.  With 8 rows of one view per wave most of a wave were rows outside the
+// frame: 46592 views of 672 channels in one row, all smoothed / a thousandth of
+// the samples above the threshold, 348 / 102 against 1216 / 324 us (one thread per
+// four samples: 1178 / 134), 24192 views of two rows 265 / 112 against 660 / 217
+// (1967 / 217).
+__global__ __launch_bounds__(256) void af_apply_few(const float *raw, const float *thr, float *out, int n_proj,
+                                                    int n_rows_raw, int nch, int band) {
+    const int xcd = blockIdx.x & 7, tiles = (nch + 63) / 64, n_v = kRows / n_rows_raw;
+    const int w = static_cast<int>(blockIdx.x >> 3) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int group = w / tiles, i = (w - group * tiles) * 64 + (threadIdx.x & 63);
+    const int p0 = (xcd * band + group) * n_v;
+    if (group >= band || p0 >= n_proj) return;
+    const size_t ps = static_cast<size_t>(nch) * n_rows_raw;
+    // rows of the group's views, one after the other in memory
+    const int rows = min(n_v, n_proj - p0) * n_rows_raw;
+    const size_t base = ps * p0 + i;
+    float x[kRows];
+    unsigned hot = 0;               // views with a sample above their threshold
+#pragma unroll
+    for (int r = 0; r < kRows; r++) x[r] = r < rows && i < nch ? raw[base + static_cast<size_t>(r) * nch] : 0.0f;
+#pragma unroll
+    for (int r = 0; r < kRows; r++) {
+        const int v = r / n_rows_raw;
+        if (r < rows && __builtin_amdgcn_ballot_w64(i < nch && x[r] > thr[p0 + v])) hot |= 1u << v;
+    }
+#pragma unroll
+    for (int r = 0; r < kRows; r++)
+        if (r < rows && i < nch && !(hot >> (r / n_rows_raw) & 1u)) out[base + static_cast<size_t>(r) * nch] = x[r];
+#pragma unroll 1
+    for (int v = 0; hot >> v; v++)
+        if (hot >> v & 1u)
+            af_apply_rows<false, 1, true>(raw, thr[p0 + v], out, i, 0, p0 + v, n_proj, n_rows_raw, nch, ps);
 }
 
 // Fixed-threshold mode: every view's threshold is the same constant.
@@ -418,6 +462,8 @@ int launch_adaptive(const AdaptiveArgs &a, hipStream_t stream) {
     const int bpv = (af_view_waves(a.n_rows_raw, a.nch) + (few ? 15 : 3)) / (few ? 16 : 4);
     const unsigned long long grid = 8ull * static_cast<unsigned long long>((a.n_proj + 7) / 8) * bpv;
     if (grid > 0x7fffffffull) return CTBB_ERR_SHAPE;
+    // (bands of groups of views, af_apply_few)
+    const int few_views = kRows / std::min(a.n_rows_raw, kRows), few_band = ((a.n_proj + few_views - 1) / few_views + 7) / 8;
     unsigned char *hot = adaptive_hot_flags(a.work, a.n_proj);
     const dim3 g(static_cast<unsigned>(grid));
     if (a.hot_only)
@@ -426,6 +472,9 @@ int launch_adaptive(const AdaptiveArgs &a, hipStream_t stream) {
     else if (copied)
         hipLaunchKernelGGL(af_apply<kHotCopied>, g, dim3(256), 0, stream, a.raw, sup, thr, a.out, hot, a.n_proj,
                            a.n_rows_raw, a.nch, bpv);
+    else if (2 * a.n_rows_raw <= kRows)
+        hipLaunchKernelGGL(af_apply_few, dim3(8 * ((few_band * ((a.nch + 63) / 64) + 3) / 4)), dim3(256), 0, stream,
+                           a.raw, thr, a.out, a.n_proj, a.n_rows_raw, a.nch, few_band);
     else
         hipLaunchKernelGGL(af_apply<kAllViews>, g, dim3(256), 0, stream, a.raw, sup, thr, a.out, hot, a.n_proj,
                            a.n_rows_raw, a.nch, bpv);

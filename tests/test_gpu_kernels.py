@@ -374,3 +374,31 @@ def test_rebin_channels_beyond_the_fan(ctx, tmp_path, ffs):
             spot, row = (r & 1, r >> 1) if ffs == "z" else (0, r)
             assert (got[:, r, beyond] == pull[spot, row, 0]).all()
     cb.free_metadata(mr)
+
+
+@pytest.mark.parametrize("channels,nrows", [(4, 1), (68, 1), (128, 2), (130, 2), (60, 3), (68, 4), (64, 5)])
+@pytest.mark.parametrize("share", [0.002, 0.5])
+def test_adaptive_few_rows(ctx, tmp_path, channels, nrows, share):
+    """5x5x5 smoothing bit for bit where a wave takes several views of few rows,
+    numbers of views and channels that leave some of it over, with few and many
+    samples above the threshold, in the first and last views too."""
+    import oracle
+    mr = _mini(tmp_path, channels, nrows, turn=190)
+    n = int(mr.ri.n_proj_pull) // int(mr.ri.n_ffs)
+    n -= 1 - n % 2                              # an odd number of views
+    mr.ri.n_proj_pull = n
+    rng = np.random.default_rng(channels + nrows)
+    raw = rng.random((n, nrows, channels)).astype(np.float32)
+    raw[[0, n - 1], nrows - 1, channels - 1] = 2.0
+    T = np.float32(1.0 - share)
+    raw_d = dev(raw.ravel())
+    out = torch.full_like(raw_d, float("nan"))
+    torch.cuda.synchronize()
+    ctx.set_options(adaptive_threshold=float(T))
+    ctx.adaptive_filter_dev(mr, raw_d, out)
+    ctx.synchronize()
+    ctx.set_options(adaptive_threshold=0.0)
+    want = oracle.adaptive_apply(mr, raw.reshape(n, -1), np.full(n, T, dtype=np.float32))
+    assert 0 < np.count_nonzero(want != raw.reshape(n, -1)) <= 1.2 * share * raw.size
+    assert np.array_equal(host(out).reshape(n, -1), want)
+    cb.free_metadata(mr)
