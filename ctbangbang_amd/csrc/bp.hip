@@ -139,8 +139,8 @@ constexpr int ilog2(int v) { return v <= 1 ? 0 : 1 + ilog2(v >> 1); }
 
 // ZS z-groups of NZ slices share one workgroup (256 * ZS threads): thread t
 // takes column t % 256 and slices (t / 256) * NZ ... + NZ - 1 of the block.
-// NZ = 32, ZS = 1 keeps 96 accumulators per thread (150 VGPRs, 3 waves per
-// SIMD); NZ = 16, ZS = 2 halves them (120 VGPRs, 4 waves per SIMD) and
+// NZ = 32, ZS = 1 keeps 96 accumulators per thread (168 VGPRs, 3 waves per
+// SIMD); NZ = 16, ZS = 2 halves them (112 or 120 VGPRs, 4 waves per SIMD) and
 // shares one staged window between the two halves.
 // One 16x16-column tile (all 32 slices) of the block described by `a`, by
 // the whole workgroup; zblk selects the slice range when a launch splits
